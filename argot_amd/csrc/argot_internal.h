@@ -109,10 +109,13 @@ struct StepCounters {
 };
 
 // Run-time parameters of the chemistry (from struct run_param, plus the
-// helium number fraction).
+// helium number fraction), and what follows from them: the conversion of a
+// cooling rate to code units, 1/anow^3 and the bounds of the specific energy.
 struct ChemParams {
   double lunit, munit, tunit, uenetok, denstonh, helium_fact;
+  double convfact;
   float anow, znow;
+  float anow3i, uene_min, uene_max;
 };
 
 // Results of one chemistry launch: maxima over cells as float bits (the

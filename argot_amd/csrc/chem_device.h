@@ -13,6 +13,7 @@
 // difference from a host restatement of the same code.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <float.h>
 #include <stdint.h>
 
 #include "argot_internal.h"
@@ -47,11 +48,20 @@ __device__ __forceinline__ double mean_mass_inv(const State& c) {
 
 // ---------------------------------------------------------------- rates ---
 
-// exp(c0 + c1 L + c2 L^2 + ...) with the powers of L formed by repeated
+// The fits below are products of powers and exponentials of the temperature.
+// Every power is formed as exp(p ln T + const) from one logarithm per
+// temperature, and powers whose bases differ by a constant factor share an
+// exponential.  What bounds the chemistry is the length of this arithmetic:
+// a cell's sub-steps are a serial chain, and the cells next to a source need
+// thousands of them.  pow() in double keeps a double-double logarithm, about
+// 5 times the instructions of exp(); the fits' relative error grows from
+// 1e-16 to a few 1e-15, far below the float the coefficients are rounded to.
+
+// c0 + c1 L + c2 L^2 + ... with the powers of L formed by repeated
 // multiplication and the terms added left to right (the collisional
 // ionization fits of reaction_rate.cu; the signs live in the coefficients).
 template <int N>
-__device__ __forceinline__ double exp_poly(const double (&c)[N], double L) {
+__device__ __forceinline__ double poly_left(const double (&c)[N], double L) {
   double s = c[0];
   double p = L;
   s = s + c[1] * p;
@@ -60,59 +70,13 @@ __device__ __forceinline__ double exp_poly(const double (&c)[N], double L) {
     p = p * L;
     s = s + c[i] * p;
   }
-  return exp(s);
+  return s;
 }
 
-// a * lam^p / (1 + (lam/b)^q)^r: the Hui & Gnedin (1997) case-B fits.
-__device__ __forceinline__ double hui_gnedin(double a, double lam, double p, double b, double q,
-                                             double r) {
-  return a * pow(lam, p) / pow(1.0 + pow(lam / b, q), r);
-}
-
-// k01 (HI + e -> HII + 2e), reaction_rate.cu:33-62.
-__device__ inline double k01(double t) {
-  constexpr double c[9] = {-32.71396786375,      13.53655609057,     -5.739328757388,
-                           1.563154982022,       -0.2877056004391,   0.03482559773736999,
-                           -0.00263197617559,    0.0001119543953861, -2.039149852002e-6};
-  return exp_poly(c, log(t * kKtoEV));
-}
-
-// k02 (HII + e -> HI), case B, reaction_rate.cu:98-103.
-__device__ inline double k02(double t) {
-  return hui_gnedin(2.753e-14, 2.0 * 157807.0 / t, 1.5, 2.740, 0.407, 2.242);
-}
-
-// k03 (HeI + e -> HeII + 2e), reaction_rate.cu:108-136.
-__device__ inline double k03(double t) {
-  constexpr double c[9] = {-44.09864886561001, 23.91596563469,      -10.75323019821,
-                           3.058038757198,     -0.5685118909884001, 0.06795391233790001,
-                           -0.005009056101857001, 0.0002067236157507, -3.649161410833e-6};
-  const double tev = t * kKtoEV;
-  const double L = log(tev);
-  return tev > 0.8 ? exp_poly(c, L) : 0.0;
-}
-
-// k04 (HeII + e -> HeI), case B, reaction_rate.cu:152-164.
-__device__ inline double k04(double t) {
-  if (t > 500.3) return 1.26e-14 * pow(2.0 * 285335.0 / t, 0.75);
-  const double logt = log10(t);
-  return (1.12e-10 - 2.1e-11 * logt) / sqrt(t);
-}
-
-// k05 (HeII + e -> HeIII + 2e), reaction_rate.cu:167-192.
-__device__ inline double k05(double t) {
-  constexpr double c[9] = {-68.71040990212001, 43.93347632635,      -18.48066993568,
-                           4.701626486759002,  -0.7692466334492,    0.08113042097303,
-                           -0.005324020628287001, 0.0001975705312221, -3.165581065665e-6};
-  const double tev = t * kKtoEV;
-  const double L = log(tev);
-  return tev > 0.8 ? exp_poly(c, L) : 0.0;
-}
-
-// k06 (HeIII + e -> HeII), case B, reaction_rate.cu:200-203.
-__device__ inline double k06(double t) {
-  return hui_gnedin(1.3765e-14, 2.0 * 631515.0 / t, 1.5, 2.740, 0.407, 2.242);
-}
+// ln(lam T) for lam_HII = 2 * 157807 K / T and lam_HeIII = 2 * 631515 K / T
+// of the case-B fits a lam^p / (1 + (lam/b)^q)^r (Hui & Gnedin 1997).
+constexpr double kLnLamHII = 12.662275226919286;
+constexpr double kLnLamHeIII = 14.049024154019651;
 
 // The six rate coefficients at one temperature, each rounded to float as
 // the reference stores them (float K_01 ... K_06).
@@ -120,126 +84,227 @@ struct KSet {
   float k1, k2, k3, k4, k5, k6;
 };
 
+// k01, k03, k05 (collisional ionization), reaction_rate.cu:33-62,108-136,
+// 167-192; k02, k06 (case-B recombination, Hui & Gnedin 1997), :98-103,
+// 200-203; k04, :152-164.
 __device__ inline KSet rate_coefficients(float T) {
+  constexpr double c1[9] = {-32.71396786375,      13.53655609057,     -5.739328757388,
+                            1.563154982022,       -0.2877056004391,   0.03482559773736999,
+                            -0.00263197617559,    0.0001119543953861, -2.039149852002e-6};
+  constexpr double c3[9] = {-44.09864886561001, 23.91596563469,      -10.75323019821,
+                            3.058038757198,     -0.5685118909884001, 0.06795391233790001,
+                            -0.005009056101857001, 0.0002067236157507, -3.649161410833e-6};
+  constexpr double c5[9] = {-68.71040990212001, 43.93347632635,      -18.48066993568,
+                            4.701626486759002,  -0.7692466334492,    0.08113042097303,
+                            -0.005324020628287001, 0.0001975705312221, -3.165581065665e-6};
+  // ln(K_to_eV), ln(2.740)
+  constexpr double kLnKtoEV = -9.359277830950614, kLnB = 1.007957920399979;
   const double t = (double)T;
-  return {(float)k01(t), (float)k02(t), (float)k03(t), (float)k04(t), (float)k05(t),
-          (float)k06(t)};
+  const double tev = t * kKtoEV;
+  const double L = log(tev);
+  KSet K;
+  K.k1 = (float)exp(poly_left(c1, L));
+  K.k3 = 0.0f;
+  K.k5 = 0.0f;
+  if (tev > 0.8) {
+    K.k3 = (float)exp(poly_left(c3, L));
+    K.k5 = (float)exp(poly_left(c5, L));
+  }
+  const double l2 = (kLnLamHII + kLnKtoEV) - L;     // ln lam_HII
+  const double l6 = (kLnLamHeIII + kLnKtoEV) - L;   // ln lam_HeIII
+  const double x2 = exp(0.407 * (l2 - kLnB));
+  constexpr double kX6 = 1.7584044112379005;        // (631515/157807)^0.407
+  const double x6 = x2 * kX6;
+  K.k2 = (float)(2.753e-14 * exp(1.5 * l2 - 2.242 * log(1.0 + x2)));
+  K.k6 = (float)(1.3765e-14 * exp(1.5 * l6 - 2.242 * log(1.0 + x6)));
+  if (t > 500.3) {
+    constexpr double kLnLamHeII = 13.254566388120152;
+    K.k4 = (float)(1.26e-14 * exp(0.75 * ((kLnLamHeII + kLnKtoEV) - L)));
+  } else {
+    constexpr double kLog10e = 0.43429448190325182765;
+    K.k4 = (float)((1.12e-10 - 2.1e-11 * ((L - kLnKtoEV) * kLog10e)) / sqrt(t));
+  }
+  return K;
 }
 
 // ------------------------------------------------------------- cooling ---
 
-// Collisional ionization / excitation shape pre/(1 + sqrt(t 1e-5)) *
-// exp(-E/(t 1e-5)) shared by cooling_rate.cu:75-114.
-__device__ __forceinline__ double collisional(double pre, double sq5, double t5, double E) {
-  return pre / (1.0 + sq5) * exp(-E / t5);
+// What heat - cool of one cell depends on besides the temperature, formed
+// once per energy update.
+struct CoolTerms {
+  double heat;                          // photoheating [erg cm^-3 s^-1]
+  double hii, heii, heiii, hi, hei;     // ion densities times n_e
+  double ions;                          // (n_HII + n_HeII + n_HeIII) n_e
+  double ne;
+  double compt, tcmb;                   // Compton: compt * (T - tcmb) * n_e
+  double scale;                         // to code units: convfact / dens
+};
+
+__device__ __forceinline__ CoolTerms cool_terms(const State& c, float zred, double nH,
+                                                double helium_fact, double scale) {
+  CoolTerms k;
+  const double nHe = nH * helium_fact;
+  const double nHI = nH * (double)c.fHI, nHII = nH * (double)c.fHII;
+  const double nHeI = nHe * (double)c.fHeI, nHeII = nHe * (double)c.fHeII;
+  const double nHeIII = nHe * (double)c.fHeIII;
+  k.ne = nH * (double)c.felec;
+  k.heat = (double)c.HeatHI * nHI;
+  k.heat += (double)c.HeatHeI * nHeI + (double)c.HeatHeII * nHeII;
+  k.hi = nHI * k.ne;
+  k.hii = nHII * k.ne;
+  k.hei = nHeI * k.ne;
+  k.heii = nHeII * k.ne;
+  k.heiii = nHeIII * k.ne;
+  k.ions = k.hii + (k.heii + k.heiii);
+  const double z1 = 1.0 + (double)zred;
+  k.compt = 5.406e-36 * (z1 * z1 * z1 * z1);
+  k.tcmb = 2.73 * z1;
+  k.scale = scale;
+  return k;
 }
 
-// heat - cool for one cell [erg cm^-3 s^-1], calc_heatcool_rate_dev
-// (heatcool_rate.cu:10-74) with cooling_rate.cu's case-B functions.
-__device__ inline double heatcool_rate(const State& c, float zred, double nH, double T,
-                                       double helium_fact) {
-  const double nHI = nH * (double)c.fHI;
-  const double nHII = nH * (double)c.fHII;
-  const double nHe = nH * helium_fact;
-  const double nHeI = nHe * (double)c.fHeI;
-  const double nHeII = nHe * (double)c.fHeII;
-  const double nHeIII = nHe * (double)c.fHeIII;
-  const double ne = nH * (double)c.felec;
-
-  double heat = (double)c.HeatHI * nHI;
-  heat += (double)c.HeatHeI * nHeI + (double)c.HeatHeII * nHeII;
-
-  const double t5 = T * 1.e-5;
+// heat - cool of one cell in code units, calc_heatcool_rate_dev
+// (heatcool_rate.cu:10-74) with cooling_rate.cu's case-B functions:
+// recombination creh2 / crehe2 / crexihe2 / crehe3, collisional ionization
+// cioh1 / ciohe1 / ciohe2 and excitation cexh1 / cexhe1 / cexhe2,
+// bremsstrahlung with its Gaunt factor, Compton cooling off the CMB.
+// cexhe1 carries another factor n_e, which the reference gives it
+// ((cexhe1 n_e n_HeI + ...) n_e).  3 logarithms and 12 exponentials.
+__device__ __forceinline__ double heatcool_rate(const CoolTerms& k, double T) {
+  constexpr double kLnB = 0.8109302162163288;    // ln 2.25
+  constexpr double kX3 = 1.6844137772424854;      // (631515/157807)^0.376
+  constexpr double kLog10e = 0.43429448190325182765;
+  const double L = log(T);
+  const double it5 = 1.0e5 / T;                   // 1 / (T/1e5)
   const double sq = sqrt(T);
-  const double sq5 = sqrt(t5);
-  // recombination (case B), creh2 / crehe2 / crexihe2 / crehe3
-  const double creh2 = hui_gnedin(3.435e-30 * T, 2.0 * 157807.0 / T, 1.97, 2.25, 0.376, 3.72);
-  const double crehe2 = T < 980.0 ? 1.7e-26 * pow(T, 0.35) : 1.9e-25 * pow(T / 1.0e3, 0.15);
-  const double crexihe2 =
-      1.24e-13 / pow(T, 1.5) * exp(-4.7 / t5) * (1.0 + 0.3 * exp(-0.94 / t5));
-  const double crehe3 = hui_gnedin(3.435e-30 * T, 2.0 * (631515.0 / T), 1.97, 2.25, 0.376, 3.72);
-  // collisional ionization / excitation
-  const double cioh1 = collisional(1.27e-21 * sq, sq5, t5, 1.578091);
-  const double ciohe1 = collisional(9.38e-22 * sq, sq5, t5, 2.853354);
-  const double ciohe2 = collisional(4.95e-22 * sq, sq5, t5, 6.31515);
-  const double cexh1 = collisional(7.5e-19, sq5, t5, 1.18348);
-  const double cexhe1 = collisional(9.1e-27 * pow(T, -0.1687), sq5, t5, 0.13179);
-  const double cexhe2 = collisional(5.54e-17 * pow(T, -0.397), sq5, t5, 4.73638);
-  // bremsstrahlung with its Gaunt factor, and Compton cooling off the CMB
-  const double lg = 5.5 - log10(T);
-  const double gaunt = 1.1 + 0.34 * exp(-lg * lg / 3.0);
+  const double sq5 = sq * 0.0031622776601683794;  // sqrt(T/1e5)
+  const double l1 = kLnLamHII - L, l3 = kLnLamHeIII - L;
+  const double x1 = exp(0.376 * (l1 - kLnB));
+  const double x3 = x1 * kX3;
+  const double a = 3.435e-30 * T;
+  const double creh2 = a * exp(1.97 * l1 - 3.72 * log(1.0 + x1));
+  const double crehe3 = a * exp(1.97 * l3 - 3.72 * log(1.0 + x3));
+  // pow(T, 0.35) and pow(T/1e3, 0.15), either side of 980 K
+  const bool cold = T < 980.0;
+  const double crehe2 = (cold ? 1.7e-26 : 1.9e-25) *
+                        exp(cold ? 0.35 * L : 0.15 * (L - 6.907755278982137));
+  // exp(-4.7/t5) as the fifth power of exp(-0.94/t5)
+  const double y = exp(-0.94 * it5);
+  const double y2 = y * y;
+  const double rsq = 1.0 / (T * sq * (1.0 + sq5));  // one division for T^-1.5 and 1/(1+sqrt(T5))
+  const double t15 = rsq * (1.0 + sq5);
+  const double r5 = rsq * (T * sq);
+  const double crexihe2 = 1.24e-13 * t15 * (y2 * y2 * y) * (1.0 + 0.3 * y);
+  const double cioh1 = exp(-1.578091 * it5), ciohe1 = exp(-2.853354 * it5);
+  const double ciohe2 = exp(-6.31515 * it5), cexh1 = exp(-1.18348 * it5);
+  const double cexhe1 = exp(-0.1687 * L - 0.13179 * it5);
+  const double cexhe2 = exp(-0.397 * L - 4.73638 * it5);
+  const double lg = 5.5 - L * kLog10e;
+  const double gaunt = 1.1 + 0.34 * exp(-lg * lg * (1.0 / 3.0));
   const double brems = 1.42e-27 * gaunt * sq;
-  const double z1 = 1.0 + (double)zred;
-  const double z14 = z1 * z1 * z1 * z1;
-  const double compt = 5.406e-36 * z14 * (T - 2.73 * z1);
-
-  double cool = (creh2 * nHII + cioh1 * nHI + cexh1 * nHI) * ne + brems * ne * nHII + compt * ne;
-  cool += ((crehe2 + crexihe2) * nHeII + crehe3 * nHeIII) * ne +
-          (ciohe1 * nHeI + ciohe2 * nHeII) * ne + (cexhe1 * ne * nHeI + cexhe2 * nHeII) * ne +
-          brems * ne * (nHeII + nHeIII);
-  return heat - cool;
+  const double col = (k.hi * (1.27e-21 * sq * cioh1 + 7.5e-19 * cexh1) +
+                      k.hei * (9.38e-22 * sq * ciohe1 + 9.1e-27 * cexhe1 * k.ne) +
+                      k.heii * (4.95e-22 * sq * ciohe2 + 5.54e-17 * cexhe2)) * r5;
+  const double cool = creh2 * k.hii + crehe3 * k.heiii + (crehe2 + crexihe2) * k.heii + col +
+                      brems * k.ions + k.compt * (T - k.tcmb) * k.ne;
+  return (k.heat - cool) * k.scale;
 }
 
 // ------------------------------------------------------ heating/cooling ---
 
 // Implicit energy update over dtime (code units): bracket the root of
-// u_new - u_old - Lambda((u_old+u_new)/2) dt and bisect it to 1e-5
-// (advance_heatcool_dev, step_heatcool.cu:19-181).  Returns the
-// bisection count.
+// F(u) = u - u_old - dt Lambda((u_old + u)/2) and bisect it to 1e-5
+// (advance_heatcool_dev, step_heatcool.cu:19-181).  Returns the bisection
+// count.
+//
+// The result is the bisection's last midpoint, so the bisection itself is
+// replayed; but a midpoint's sign needs no evaluation where it is known from
+// the root's place.  Two secant steps from the bracket's own two evaluations
+// place the root to 1e-9 of u (F is close to linear over the bracket's 10%),
+// and a midpoint is evaluated only when it falls inside that margin: about 4
+// evaluations of Lambda per update instead of 16.  The midpoints and their
+// order are the bisection's, so the result is too, as long as F rises through
+// the bracket.  Where that is not plain (a slope of the secants below 0.3 or
+// changing by more than a factor 1.6, the recombination fits' break at 980 K
+// inside the bracket, a value that is no number) every midpoint is evaluated.
+// With the fits above, a 128^3 mesh over 100 kyr (8.0e6 sub-steps, the longest
+// cell's chain setting the time) took 12.4 ms instead of 100 ms, with the same
+// bits in every cell.
 __device__ inline int advance_heatcool(float dens_cell, float* uene, const State& c,
                                        const ChemParams& p, float dtime) {
-  const double eunit = (p.lunit * p.lunit) / (p.tunit * p.tunit);
-  const double convfact = p.tunit / eunit * (p.lunit * p.lunit * p.lunit) / p.munit;
-  const float wmol_min = (float)(4.0 / (5.0 * kXH + 3.0));
-  const float wmol_max = (float)(1.0 / (kXH + 0.25 * kYHe));
-  // pow(10, LOG_T_MIN + 0.5) = 10 and pow(10, LOG_T_MAX - 0.5) = 1e8 exactly
-  const float uene_min = (float)(10.0 / p.uenetok / (double)wmol_max);
-  const float uene_max = (float)(1.0e8 / p.uenetok / (double)wmol_min);
-  const float anow3i = (float)(1.0 / (double)(p.anow * p.anow * p.anow));
-  const double dens = (double)(dens_cell * anow3i);
+  const double dens = (double)(dens_cell * p.anow3i);
+  const double uene_min = (double)p.uene_min, uene_max = (double)p.uene_max;
 
-  double uene_old = (double)*uene;
-  double uene_up = uene_old, uene_lo = uene_old;
-  if (uene_old < (double)uene_min) {
-    uene_up = uene_lo = uene_old = (double)uene_min;
-  } else if (uene_old > (double)uene_max) {
-    uene_up = uene_lo = uene_old = (double)uene_max;
+  const double uene_in = (double)*uene;
+  double uene_old = uene_in;
+  if (uene_old < uene_min) {
+    uene_old = uene_min;
+  } else if (uene_old > uene_max) {
+    uene_old = uene_max;
   }
   const float wmol = (float)mean_mass_inv(c);
   const double nH = dens * p.denstonh;
-  auto rate = [&](double T) {
-    return heatcool_rate(c, p.znow, nH, T, p.helium_fact) / dens * convfact;
-  };
-  double T = (double)*uene * p.uenetok * (double)wmol;
-  double heatcool = rate(T);
+  const CoolTerms k = cool_terms(c, p.znow, nH, p.helium_fact, p.convfact / dens);
+  auto temp = [&](double u) { return u * p.uenetok * (double)wmol; };
   const double dt = (double)dtime;
-  if (heatcool > 0.0) {
-    uene_up = min_of(uene_up * kSqrtFact, (double)uene_max);
-    uene_lo = max_of(uene_lo / kSqrtFact, (double)uene_min);
-    heatcool = rate(uene_up * p.uenetok * (double)wmol);
-    while (uene_up - uene_old - heatcool * dt < 0.0) {
-      uene_up *= 1.1;
-      uene_lo *= 1.1;
-      if (uene_up > (double)uene_max) break;
-      heatcool = rate(uene_up * p.uenetok * (double)wmol);
-    }
-  } else {
-    uene_up = min_of(uene_up * kSqrtFact, (double)uene_max);
-    uene_lo = max_of(uene_lo / kSqrtFact, (double)uene_min);
-    heatcool = rate(uene_lo * p.uenetok * (double)wmol);
-    while (uene_lo - uene_old - heatcool * dt > 0.0) {
-      uene_up /= 1.1;
-      uene_lo /= 1.1;
-      if (uene_lo < (double)uene_min) break;
-      heatcool = rate(uene_lo * p.uenetok * (double)wmol);
+  const double h0 = heatcool_rate(k, temp(uene_in));
+  // Heating brackets upwards, cooling downwards; one loop for both, so that
+  // the lanes of a wavefront evaluate together.
+  const bool heating = h0 > 0.0;
+  double uene_up = min_of(uene_old * kSqrtFact, uene_max);
+  double uene_lo = max_of(uene_old / kSqrtFact, uene_min);
+  double h1, end;
+  for (;;) {
+    end = heating ? uene_up : uene_lo;
+    h1 = heatcool_rate(k, temp(end));
+    const double f = end - uene_old - h1 * dt;
+    if (!(heating ? f < 0.0 : f > 0.0)) break;
+    uene_up = heating ? uene_up * 1.1 : uene_up / 1.1;
+    uene_lo = heating ? uene_lo * 1.1 : uene_lo / 1.1;
+    if (heating ? uene_up > uene_max : uene_lo < uene_min) break;
+  }
+  auto residual = [&](double u) {
+    return u - uene_old - heatcool_rate(k, temp(0.5 * (uene_old + u))) * dt;
+  };
+  // F(u) <= 0 is known for u <= below, F(u) > 0 for u >= above
+  double below = -DBL_MAX, above = DBL_MAX;
+  {
+    const double m = (h1 - h0) / (end - uene_in);
+    double s = 1.0 - 0.5 * dt * m;
+    const double r0 = uene_old + dt * (h0 + m * (uene_old - uene_in)) / s;
+    const bool smooth = s > 0.3 && s < 1.0e6 && r0 > 0.5 * uene_lo && r0 < 2.0 * uene_up &&
+                        !(temp(0.5 * (uene_old + uene_lo)) < 980.0 &&
+                          temp(0.5 * (uene_old + uene_up)) >= 980.0);
+    if (smooth) {
+      double f = residual(r0), r = r0;
+      for (int it = 0; it < 4; it++) {
+        const double rn = r - f / s;
+        const double fn = residual(rn);
+        // (points closer than rounding lets F be told apart keep the slope)
+        const double sn = fabs(rn - r) > 1.0e-11 * r0 ? (fn - f) / (rn - r) : s;
+        if (!(sn > 0.6 * s && sn < 1.6 * s)) break;
+        s = sn;
+        r = rn;
+        f = fn;
+        const double step = f / s;
+        const double tol = fabs(step) + 1.0e-12 * r;
+        if (tol < 1.0e-9 * r) {
+          below = r - step - tol;
+          above = r - step + tol;
+          break;
+        }
+      }
     }
   }
   int iter = 0;
   double uene_new;
   do {
     uene_new = 0.5 * (uene_up + uene_lo);
-    heatcool = rate(0.5 * (uene_old + uene_new) * p.uenetok * (double)wmol);
-    if (uene_new - uene_old - heatcool * dt > 0.0)
+    bool positive = uene_new >= above;
+    if (!positive && !(uene_new <= below)) {
+      positive = residual(uene_new) > 0.0;
+    }
+    if (positive)
       uene_up = uene_new;
     else
       uene_lo = uene_new;

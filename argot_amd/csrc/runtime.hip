@@ -1261,6 +1261,15 @@ static ChemParams chem_params(const run_param* r) {
   p.helium_fact = g_helium_fact;
   p.anow = r->anow;
   p.znow = r->znow;
+  // step_heatcool.cu:19-60; hydrogen 0.755 and helium 0.245 by mass
+  // (chemistry.h:23-24), temperatures between 10 and 1e8 K
+  const double eunit = (p.lunit * p.lunit) / (p.tunit * p.tunit);
+  p.convfact = p.tunit / eunit * (p.lunit * p.lunit * p.lunit) / p.munit;
+  const float wmol_min = (float)(4.0 / (5.0 * 0.755 + 3.0));
+  const float wmol_max = (float)(1.0 / (0.755 + 0.25 * 0.245));
+  p.uene_min = (float)(10.0 / p.uenetok / (double)wmol_max);
+  p.uene_max = (float)(1.0e8 / p.uenetok / (double)wmol_min);
+  p.anow3i = (float)(1.0 / (double)(p.anow * p.anow * p.anow));
   return p;
 }
 
