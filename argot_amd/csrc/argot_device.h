@@ -484,41 +484,60 @@ __device__ inline void ray_rate_setup(const GridDev& g, const RateTables& rt, co
   rr->r[2] = 1.0 / (nHeII * vsh + kRateTiny);
 }
 
+__device__ __forceinline__ double lane_value(double v, int lane) { return __shfl(v, lane, 64); }
+
 // The reference's frequency loop in FP64, calc_photoion_rate.c:285-387,
-// bin by bin (used when FP32 would overflow, e.g. a target cell that holds
-// the ray's source, where the reference itself produces inf/NaN).
+// for the lanes of a wavefront that need it (where FP32 would overflow, e.g.
+// a target cell that holds the ray's source, where the reference itself
+// produces inf/NaN).  Such rays are single lanes, and one lane taking 256
+// bins of double-precision exponentials and quotients holds its wavefront
+// for longer than a small mesh's whole step; so the wavefront takes each of
+// them together, a lane every 64th bin, and adds the lanes' sums.  Every lane
+// of the wavefront calls this; spec(owner, k) is bin k of lane owner's ray.
 template <typename SpecFn>
-__device__ inline void rate_loop_f64(const RateTables& rt, const RayRate& rr, SpecFn spec,
-                                     double out[6]) {
-  double g0 = 0, h0 = 0, g1 = 0, g2 = 0, h1 = 0, h2 = 0;
-  for (int k = 0; k < rt.ngrid; k++) {
-    const float nu = rt.nu[k];
-    const double s0 = rt.cs[3 * k + 0], s1 = rt.cs[3 * k + 1], s2 = rt.cs[3 * k + 2];
-    double tau = rr.t[0] * s0;
-    double w0 = rr.d[0] * s0;
-    double dtot = w0;
-    tau += rr.t[1] * s1;
-    tau += rr.t[2] * s2;
-    double w1 = rr.d[1] * s1;
-    double w2 = rr.d[2] * s2;
-    dtot += w1 + w2;
-    const double absorbed = spec(k) * exp(-tau) * (1.0e0 - exp(-dtot));
-    w0 /= (dtot + kRateTiny);
-    g0 += w0 * absorbed * rr.r[0];
-    if ((double)nu > 1.0) h0 += w0 * absorbed * ((double)nu - 1.0) * rr.r[0];
-    w1 /= (dtot + kRateTiny);
-    w2 /= (dtot + kRateTiny);
-    g1 += w1 * absorbed * rr.r[1];
-    g2 += w2 * absorbed * rr.r[2];
-    if ((double)nu > 1.8125) h1 += w1 * absorbed * ((double)nu - 1.8125) * rr.r[1];
-    if ((double)nu > 4.0) h2 += w2 * absorbed * ((double)nu - 4.0) * rr.r[2];
+__device__ inline void rate_f64_wave(const RateTables& rt, const RayRate& rr, bool need,
+                                     SpecFn spec, double out[6]) {
+  const int lane = threadIdx.x & 63;
+  for (unsigned long long todo = __ballot(need); todo != 0; todo &= todo - 1) {
+    const int owner = __builtin_ctzll(todo);
+    double t[3], d[3], r[3];
+#pragma unroll
+    for (int s = 0; s < 3; s++) {
+      t[s] = lane_value(rr.t[s], owner);
+      d[s] = lane_value(rr.d[s], owner);
+      r[s] = lane_value(rr.r[s], owner);
+    }
+    double g[6] = {0, 0, 0, 0, 0, 0};   // Gamma HI, Heat HI, Gamma HeI, HeII, Heat HeI, HeII
+    for (int k = lane; k < rt.ngrid; k += 64) {
+      const double nu = (double)rt.nu[k];
+      const double s0 = rt.cs[3 * k + 0], s1 = rt.cs[3 * k + 1], s2 = rt.cs[3 * k + 2];
+      double tau = t[0] * s0;
+      double w0 = d[0] * s0;
+      double dtot = w0;
+      tau += t[1] * s1;
+      tau += t[2] * s2;
+      double w1 = d[1] * s1;
+      double w2 = d[2] * s2;
+      dtot += w1 + w2;
+      const double absorbed = spec(owner, k) * exp(-tau) * (1.0e0 - exp(-dtot));
+      w0 /= (dtot + kRateTiny);
+      g[0] += w0 * absorbed * r[0];
+      if (nu > 1.0) g[1] += w0 * absorbed * (nu - 1.0) * r[0];
+      w1 /= (dtot + kRateTiny);
+      w2 /= (dtot + kRateTiny);
+      g[2] += w1 * absorbed * r[1];
+      g[3] += w2 * absorbed * r[2];
+      if (nu > 1.8125) g[4] += w1 * absorbed * (nu - 1.8125) * r[1];
+      if (nu > 4.0) g[5] += w2 * absorbed * (nu - 4.0) * r[2];
+    }
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) g[i] += __shfl_xor(g[i], off, 64);
+      if (i == 1 || i > 3) g[i] *= kHnuL;
+      if (lane == owner) out[i] = g[i];
+    }
   }
-  out[0] = g0;
-  out[1] = h0 * kHnuL;
-  out[2] = g1;
-  out[3] = g2;
-  out[4] = h1 * kHnuL;
-  out[5] = h2 * kHnuL;
 }
 
 }  // namespace argot

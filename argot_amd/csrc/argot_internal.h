@@ -46,6 +46,11 @@ struct RateTables {
   const float* dsig;   // [3*ngrid] sigma_s(k) - sigma_s(last bin), species-major
   double cs_max[3];    // max over bins of sigma_s
   double cs_last[3];   // sigma_s at the last bin
+  // quadrature form (rate_rule.h): cross-sections at its nodes, and the
+  // first-bin cross-sections that scale a ray against a spectrum's limit
+  const float* qsig;   // [3*kRuleNodes] sigma_s, species-major
+  const float* qdsig;  // [3*kRuleNodes] sigma_s - sigma_s(last bin)
+  float edge[9];       // [range][species]
 };
 
 // Source tree in depth-first pre-order (children in octant order), as
@@ -63,6 +68,8 @@ struct TreeDev {
   const NodeLink* link;      // [nnode]
   const float* spec;         // [nnode*ngrid] spectrum / spec_scale, FP32
   const double* spec_scale;  // [nnode] max over bins of the spectrum
+  const float* weight;       // [nnode*kRuleWeights] quadrature weights of spec (rate_rule.h)
+  const float* limit;        // [nnode] thickest ray the quadrature serves (0: none)
   const float* src_pos;      // [4*nsrc]
 };
 

@@ -35,14 +35,30 @@ hipError_t launch_walk_segments(const GridDev& g, const float4* nf, void* seg, i
 // crossing (no packed-field buffer; identical optical depths).
 hipError_t launch_walk_segments_mesh(const GridDev& g, const void* mesh, double helium_fact,
                                      void* seg, int64_t nseg, int kahan, hipStream_t s);
+// The quadrature rule's matrices on the device (rate_rule.h).
+struct RuleDev {
+  int usable;
+  int start[4];
+  const double* project;   // [ngrid][kRuleW3]
+  const float* test;       // [ngrid][kRuleTests][2]
+};
+// Quadrature weights [nspec * kRuleWeights] and limits [nspec] of spectra
+// [nspec * ngrid].
+hipError_t launch_project_spectra(const RuleDev& rule, const float* spec, int nspec, int ngrid,
+                                  float* weight, float* limit, hipStream_t s);
+// The distinct spectra of a calc_photoion_rate_cuda call.
+struct CallSpectra {
+  const float* spec32;     // [nspec * ngrid] scaled by 1/scale
+  const double* spec64;    // [nspec * ngrid] as given
+  const double* scale;     // [nspec] the spectrum's maximum
+  const float* weight;     // quadrature weights of spec32, and
+  const float* limit;      // the thickest ray they serve
+};
 // calc_photoion_rate_cuda: ntarget targets, each with its consecutive rays
 // (rays[first .. first + count)), rates added to the mesh's prev_chem.
-// spec32/spec64/spec_scale: the distinct spectra ([nspec * ngrid] FP32
-// scaled by 1/spec_scale, FP64 as given, and the per-spectrum maximum).
 hipError_t launch_target_rates(const GridDev& g, const RateTables& rt, void* mesh,
                               const CallTarget* tg, int64_t ntarget, const CallRay* rays,
-                              const float* spec32, const double* spec64, const double* spec_scale,
-                              hipStream_t s);
+                              const CallSpectra& sp, hipStream_t s);
 hipError_t launch_reset_counters(StepCounters* ctr, hipStream_t s);
 // smooth_photoion_rate on one rank; tmp_in/tmp_out: 6*ncell floats each.
 // On return (stream order) tmp_out holds the smoothed rates as six planes.

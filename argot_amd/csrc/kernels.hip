@@ -15,6 +15,7 @@
 #include "argot_device.h"
 #include "argot_internal.h"
 #include "kernels.h"
+#include "rate_rule.h"
 
 namespace argot {
 
@@ -300,19 +301,114 @@ __device__ __forceinline__ void rate_bins_mixed(const RateTables& rt, int k0, in
   }
 }
 
-// FP32 frequency loop (photon-conserving form, calc_photoion_rate.c:327-386
+typedef float F4 __attribute__((ext_vector_type(4)));
+
+// Nodes [o, o + N) of the quadrature form for one bin range with NS active
+// species: the same f as the bin loops above (thin form, and in MIXED
+// wavefronts the direct form by lane and node), at the range's nodes, summed
+// with the spectrum's weight rows G_s, H_s.  w(i): the i-th four weights of
+// the range; cl: -log2(e) times the range's constant optical depth.
+template <int NS, int N, bool MIXED, typename WeightF>
+__device__ __forceinline__ void rate_nodes(const RateTables& rt, int o, float cl,
+                                           const float nl[3], const float dl[3], bool thin,
+                                           WeightF w, double G[3], double H[3]) {
+  constexpr float kHalfLog2eN = -0.5f * kLog2e;
+  float g[NS], h[NS];
+#pragma unroll
+  for (int s = 0; s < NS; s++) g[s] = h[s] = 0.0f;
+#pragma unroll 1
+  for (int j = 0; j < N; j += 4) {
+    F4 sg[NS], ds[NS], wg[NS], wh[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      sg[s] = ldc(reinterpret_cast<const F4*>(rt.qsig + s * kRuleNodes + o + j));
+      ds[s] = ldc(reinterpret_cast<const F4*>(rt.qdsig + s * kRuleNodes + o + j));
+      wg[s] = w((2 * s * N + j) / 4);
+      wh[s] = w(((2 * s + 1) * N + j) / 4);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      float yl = 0.0f;
+#pragma unroll
+      for (int s = 0; s < NS; s++) yl = __builtin_fmaf(dl[s], sg[s][i], yl);
+      float z = NS < 3 ? yl + cl : yl;
+#pragma unroll
+      for (int s = 0; s < NS; s++) z = __builtin_fmaf(nl[s], ds[s][i], z);
+      float f = __builtin_amdgcn_exp2f(z) * sinhc_l(yl);
+      if constexpr (MIXED) {
+        float zt = cl;
+#pragma unroll
+        for (int s = 0; s < NS; s++) zt = __builtin_fmaf(nl[s], ds[s][i], zt);
+        const float om = 1.0f - __builtin_amdgcn_exp2f(yl + yl);
+        const float fk =
+            __builtin_amdgcn_exp2f(zt) * om * (__builtin_amdgcn_rcpf(yl) * kHalfLog2eN);
+        f = (thin || yl >= kYlThin) ? f : fk;
+      }
+#pragma unroll
+      for (int s = 0; s < NS; s++) {
+        g[s] = __builtin_fmaf(wg[s][i], f, g[s]);
+        h[s] = __builtin_fmaf(wh[s][i], f, h[s]);
+      }
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+    G[s] += g[s];
+    H[s] += h[s];
+  }
+}
+
+template <bool MIXED, typename WeightF>
+__device__ __forceinline__ void rate_all_nodes(const RateTables& rt, float cl1, float cl2,
+                                               const float nl[3], const float dl[3], bool thin,
+                                               WeightF w, double G[3], double H[3]) {
+  rate_nodes<1, kRuleN1, MIXED>(rt, 0, cl1, nl, dl, thin, w, G, H);
+  rate_nodes<2, kRuleN2, MIXED>(rt, kRuleN1, cl2, nl, dl, thin,
+                                [&](int i) { return w(kRuleW1 / 4 + i); }, G, H);
+  rate_nodes<3, kRuleN3, MIXED>(rt, kRuleN1 + kRuleN2, 0.0f, nl, dl, thin,
+                                [&](int i) { return w((kRuleW1 + kRuleW2) / 4 + i); }, G, H);
+}
+
+// FP32 frequency integral (photon-conserving form, calc_photoion_rate.c:327-386
 // regrouped): with B_k = N_k exp(-tau_k) (1 - exp(-dtau_k)) / dtau_k,
 //   Gamma_s = r_s d_s sum_k sigma_s(k) B_k,  Heat_s = r_s d_s sum_k hsig_s(k) B_k.
 // The optical depth is shifted by its last-bin value tsh (folded back in
 // FP64): tau_k - tsh = sum_s N_s (sigma_s(k) - sigma_s(last)).  Bins below
 // the HeI and HeII edges skip the absent species.
-template <typename SpecF>
+// A ray within its spectrum's limit takes the sums as quadratures over the
+// rule's 44 nodes (rate_rule.cpp), any other ray bin by bin; which one
+// depends on the ray alone, not on its wavefront.
+template <typename SpecF, typename WeightF>
 __device__ inline void rate_loop_f32(const RateTables& rt, const RayRate& rr, double scale,
-                                     SpecF spec, double out[6]) {
+                                     float limit, SpecF spec, WeightF weight, double out[6]) {
   const double tsh = rr.t[0] * rt.cs_last[0] + rr.t[1] * rt.cs_last[1] + rr.t[2] * rt.cs_last[2];
   const float n[3] = {(float)rr.t[0], (float)rr.t[1], (float)rr.t[2]};
   const float c1 = (float)(-(rr.t[1] * rt.cs_last[1] + rr.t[2] * rt.cs_last[2]));
   const float c2 = (float)(-(rr.t[2] * rt.cs_last[2]));
+  // Scale of the ray against the rule's test columns, from its columns at the
+  // far side of the cell (and, where the half-cell shift made one
+  // negative, its negative part).
+  float lam = 0.0f, neg = 0.0f;
+  {
+    float tf[3], tn[3];
+#pragma unroll
+    for (int s = 0; s < 3; s++) {
+      tf[s] = fmaxf(n[s], n[s] + (float)rr.d[s]);
+      tn[s] = fmaxf(-n[s], 0.0f);
+    }
+#pragma unroll
+    for (int g = 0; g < 3; g++) {
+      float e = 0.0f, m = 0.0f;
+#pragma unroll
+      for (int s = 0; s <= g; s++) {
+        e = __builtin_fmaf(fabsf(tf[s]), rt.edge[3 * g + s], e);
+        m = __builtin_fmaf(tn[s], rt.edge[3 * g + s], m);
+      }
+      lam = fmaxf(lam, e);
+      neg = fmaxf(neg, m);
+    }
+  }
+  const bool nodes = lam <= limit && neg <= kRuleNegative && limit > 0.0f;
   // per-ray prefactors first (same operations as after the loop), so that
   // only they, not the ray's FP64 quantities, stay live through the bins
   // exp(-tsh) as 2^n 2^f, n = floor(-tsh log2 e) and f in [0, 1): the FP32
@@ -342,7 +438,18 @@ __device__ inline void rate_loop_f32(const RateTables& rt, const RayRate& rr, do
   const float nl[3] = {(float)(rr.t[0] * -kLog2eD), (float)(rr.t[1] * -kLog2eD),
                        (float)(rr.t[2] * -kLog2eD)};
   const bool thin = dmax <= kThinMax;
-  if (__all(thin)) {
+  if (nodes) {
+    const float cl1 = c1 * -kLog2e, cl2 = c2 * -kLog2e;
+    if (__all(thin))
+      rate_all_nodes<false>(rt, cl1, cl2, nl, dl, thin, weight, G, H);
+    else
+      rate_all_nodes<true>(rt, cl1, cl2, nl, dl, thin, weight, G, H);
+#pragma unroll
+    for (int s = 0; s < 3; s++) {
+      G[s] *= 1.0 / kRuleScale;
+      H[s] *= 1.0 / kRuleScale;
+    }
+  } else if (__all(thin)) {
     rate_bins_thin<1, false>(rt, 0, rt.k_he1, c1, n, nl, dl, spec, G, H);
     rate_bins_thin<2, false>(rt, rt.k_he1, rt.k_he2, c2, n, nl, dl, spec, G, H);
     rate_bins_thin<3, true>(rt, rt.k_he2, rt.ngrid, 0.0f, n, nl, dl, spec, G, H);
@@ -357,6 +464,74 @@ __device__ inline void rate_loop_f32(const RateTables& rt, const RayRate& rr, do
   out[3] = p2 * G[2];
   out[4] = p1 * H[1] * kHnuL;
   out[5] = p2 * H[2] * kHnuL;
+}
+
+// Quadrature weights and limits of nspec spectra (rows of ngrid floats,
+// scaled to their maximum): the rule's projection matrices times the
+// spectrum.  A block takes NB spectra, so that each matrix entry it reads
+// serves NB of them; 448 threads, one per weight (192) and per test column and
+// rate (210).
+constexpr int kProjectThreads = 448;
+static_assert(kRuleWeights + kRuleTests <= kProjectThreads, "one thread per output");
+template <int NB>
+__global__ __launch_bounds__(kProjectThreads) void project_spectra_kernel(
+    RuleDev rule, const float* __restrict__ spec, int nspec, int ngrid,
+    float* __restrict__ weight, float* __restrict__ limit) {
+  __shared__ float sp[kNgridMax][NB];
+  __shared__ unsigned fail[NB];
+  const int t = threadIdx.x;
+  const int u0 = blockIdx.x * NB;
+  for (int i = t; i < NB * ngrid; i += kProjectThreads) {
+    const int j = i / ngrid, k = i % ngrid;
+    sp[k][j] = u0 + j < nspec ? spec[(int64_t)(u0 + j) * ngrid + k] : 0.0f;
+  }
+  if (t < NB) fail[t] = 0u;
+  __syncthreads();
+  if (t < kRuleWeights) {
+    const int g = t < kRuleW1 ? 0 : t < kRuleW1 + kRuleW2 ? 1 : 2;
+    const int o = t - (g == 0 ? 0 : g == 1 ? kRuleW1 : kRuleW1 + kRuleW2);
+    double w[NB];
+#pragma unroll
+    for (int j = 0; j < NB; j++) w[j] = 0.0;
+#pragma unroll 8
+    for (int k = rule.start[g]; k < rule.start[g + 1]; k++) {
+      const double m = rule.project[(int64_t)k * kRuleW3 + o];
+#pragma unroll
+      for (int j = 0; j < NB; j++) w[j] += (double)sp[k][j] * m;
+    }
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+      if (u0 + j < nspec) weight[(int64_t)(u0 + j) * kRuleWeights + t] = (float)w[j];
+  } else if (t < kRuleWeights + kRuleTests) {
+    const int c = t - kRuleWeights;
+    float sum[NB], err[NB];
+#pragma unroll
+    for (int j = 0; j < NB; j++) sum[j] = err[j] = 0.0f;
+#pragma unroll 8
+    for (int k = 0; k < ngrid; k++) {
+      const float2 m = reinterpret_cast<const float2*>(rule.test)[(int64_t)k * kRuleTests + c];
+#pragma unroll
+      for (int j = 0; j < NB; j++) {
+        sum[j] = __builtin_fmaf(sp[k][j], m.x, sum[j]);
+        err[j] = __builtin_fmaf(sp[k][j], m.y, err[j]);
+      }
+    }
+    const int level = c / 6 / kRuleMixes;
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+      if (!(fabsf(err[j]) <= kRuleTol * sum[j]))
+        atomicOr(&fail[j], 1u << (level < kRuleLevels ? level : 0));
+  }
+  __syncthreads();
+  if (t < NB && u0 + t < nspec) {
+    constexpr float kLevel[kRuleLevels] = {0.2f, 0.4f, 0.7f, 1.0f, 1.7f, 3.0f};
+    const unsigned f = rule.usable ? fail[t] : 1u;
+    float lim = 0.0f;
+#pragma unroll
+    for (int l = kRuleLevels - 1; l >= 0; l--)
+      if ((f & ((2u << l) - 1u)) == 0u && lim == 0.0f) lim = kLevel[l];
+    limit[u0 + t] = lim;
+  }
 }
 
 // Lower bound of the shifted bin optical depth and upper bound of the
@@ -405,17 +580,14 @@ __device__ __forceinline__ T wave_sum(T v) {
 // cell.  A target's rays are consecutive in the caller's order and its lane
 // sums their rates in FP64 in that order, then adds the sum to the cell
 // once: no atomics, no per-ray buffer.  Each ray names one of the call's
-// distinct spectra (rays from one source or tree node share it).  The
-// wavefront visits the spectra its lanes' next rays use in increasing index
-// order (the host numbers them by first appearance, so the lists of
-// neighbouring targets run nearly in step): the lanes at that spectrum take
-// their ray with the bins read through scalar loads, the others wait.  Each
-// ray's arithmetic is the fused kernel's, so a ray list taken from the
+// distinct spectra (rays from one source or tree node share it), whose
+// quadrature weights (768 B) its lane reads in 16-B loads: every lane takes
+// its next ray at each pass, whichever spectra the wavefront's rays have.
+// Each ray's arithmetic is the fused kernel's, so a ray list taken from the
 // fused step gives its bits.
 __global__ __launch_bounds__(64) ARGOT_CALL_OCCUPANCY void target_rates_kernel(
     GridDev g, RateTables rt, unsigned char* __restrict__ mesh, const CallTarget* __restrict__ tg,
-    int64_t ntarget, const CallRay* __restrict__ rays, const float* __restrict__ spec32,
-    const double* __restrict__ spec64, const double* __restrict__ spec_scale) {
+    int64_t ntarget, const CallRay* __restrict__ rays, CallSpectra sp) {
   const int lane = threadIdx.x;
   const int64_t t = (int64_t)blockIdx.x * 64 + lane;
   const bool valid = t < ntarget;
@@ -434,24 +606,31 @@ __global__ __launch_bounds__(64) ARGOT_CALL_OCCUPANCY void target_rates_kernel(
   const int64_t rend = T.first + T.count;
   double acc[6] = {0, 0, 0, 0, 0, 0};
   const int ng = rt.ngrid;
-  for (;;) {
+  while (__any(r < rend)) {
     const bool more = r < rend;
-    const int sp = more ? rays[r].spec : INT_MAX;
-    const int u = wave_min(sp);
-    if (u == INT_MAX) break;
-    if (more && sp == u) {
+    bool wide = false;   // FP32 cannot serve this ray
+    int u = 0;
+    RayRate rr{};
+    double res[6] = {0, 0, 0, 0, 0, 0};
+    if (more) {
       const CallRay R = rays[r];
+      u = R.spec;
       const Vec3f src{R.src[0], R.src[1], R.src[2]};
-      RayRate rr;
       ray_rate_setup(g, rt, R.tau, src, tgt, dens, fHI, fHeI, fHeII, &rr);
-      double res[6];
-      if (fast_rate_ok(rt, rr)) {
-        const float* s32 = spec32 + (int64_t)u * ng;
-        rate_loop_f32(rt, rr, ldc(spec_scale + u), [&](int k) { return ldc(s32 + k); }, res);
-      } else {
-        const double* s64 = spec64 + (int64_t)u * ng;
-        rate_loop_f64(rt, rr, [&](int k) { return ldc(s64 + k); }, res);
+      wide = !fast_rate_ok(rt, rr);
+      if (!wide) {
+        const float* s32 = sp.spec32 + (int64_t)u * ng;
+        const F4* w = reinterpret_cast<const F4*>(sp.weight + (int64_t)u * kRuleWeights);
+        rate_loop_f32(rt, rr, sp.scale[u], sp.limit[u], [&](int k) { return s32[k]; },
+                      [&](int i) { return w[i]; }, res);
       }
+    }
+    rate_f64_wave(rt, rr, wide,
+                  [&](int owner, int k) {
+                    return sp.spec64[(int64_t)__shfl(u, owner, 64) * ng + k];
+                  },
+                  res);
+    if (more) {
 #pragma unroll
       for (int k = 0; k < 6; k++) acc[k] += res[k];
       r++;
@@ -685,19 +864,18 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY_FOR(SURR) void fused_step_kerne
           }
         }
       }
-      if (exact) {
-        if (fast_rate_ok(rt, rr)) {
-          const float* sp = tr.spec + (int64_t)u * rt.ngrid;
-          rate_loop_f32(rt, rr, ldc(tr.spec_scale + u), [&](int k) { return ldc(sp + k); }, res);
-        } else {
-          // the node spectrum as spec * spec_scale (within 6e-8 of the
-          // double sums; this loop serves the rays FP32 cannot)
-          const float* sp = tr.spec + (int64_t)u * rt.ngrid;
-          const double sc = ldc(tr.spec_scale + u);
-          rate_loop_f64(rt, rr, [&](int k) { return (double)ldc(sp + k) * sc; }, res);
-          my_fb++;
-        }
+      const float* sp = tr.spec + (int64_t)u * rt.ngrid;
+      const double sc = ldc(tr.spec_scale + u);
+      const bool wide = exact && !fast_rate_ok(rt, rr);   // FP32 cannot serve this ray
+      if (exact && !wide) {
+        const F4* wt = reinterpret_cast<const F4*>(tr.weight + (int64_t)u * kRuleWeights);
+        rate_loop_f32(rt, rr, sc, ldc(tr.limit + u), [&](int k) { return ldc(sp + k); },
+                      [&](int i) { return ldc(wt + i); }, res);
       }
+      // the node spectrum as spec * spec_scale (within 6e-8 of the double
+      // sums; this loop serves the rays FP32 cannot)
+      rate_f64_wave(rt, rr, wide, [&](int, int k) { return (double)sp[k] * sc; }, res);
+      if (wide) my_fb++;
       if (emit) {
 #pragma unroll
         for (int k = 0; k < 6; k++) acc_lds[k][lane] += res[k];
@@ -911,11 +1089,24 @@ hipError_t launch_walk_segments_mesh(const GridDev& g, const void* mesh, double 
 
 hipError_t launch_target_rates(const GridDev& g, const RateTables& rt, void* mesh,
                               const CallTarget* tg, int64_t ntarget, const CallRay* rays,
-                              const float* spec32, const double* spec64, const double* spec_scale,
-                              hipStream_t s) {
+                              const CallSpectra& sp, hipStream_t s) {
   if (ntarget <= 0) return hipSuccess;
   target_rates_kernel<<<nblocks(ntarget, 64), 64, 0, s>>>(
-      g, rt, static_cast<unsigned char*>(mesh), tg, ntarget, rays, spec32, spec64, spec_scale);
+      g, rt, static_cast<unsigned char*>(mesh), tg, ntarget, rays, sp);
+  return hipGetLastError();
+}
+
+// 16 spectra to a block where that still gives every CU a block; few spectra
+// spread out, 4 to a block, so that the launch is short.
+hipError_t launch_project_spectra(const RuleDev& rule, const float* spec, int nspec, int ngrid,
+                                  float* weight, float* limit, hipStream_t s) {
+  if (nspec <= 0) return hipSuccess;
+  if (nspec >= 16 * 256)
+    project_spectra_kernel<16><<<nblocks(nspec, 16), kProjectThreads, 0, s>>>(
+        rule, spec, nspec, ngrid, weight, limit);
+  else
+    project_spectra_kernel<4><<<nblocks(nspec, 4), kProjectThreads, 0, s>>>(
+        rule, spec, nspec, ngrid, weight, limit);
   return hipGetLastError();
 }
 

@@ -21,6 +21,7 @@
 #include "argot_hip.h"
 #include "argot_internal.h"
 #include "kernels.h"
+#include "rate_rule.h"
 #include "surrogate.h"
 #include "tree.h"
 
@@ -153,6 +154,13 @@ struct Ctx {
   DevBuf<float> nu, cs, sig, hsig, dsig;
   double cs_max[3] = {0, 0, 0}, cs_last[3] = {0, 0, 0};
   int ngrid = 0, k_he1 = 0, k_he2 = 0;
+  // quadrature rule of the tables (one buffer), and the weights and limits
+  // of the spectra in use (one buffer)
+  DevBuf<double> rule_buf;
+  DevBuf<float> weight;
+  RuleDev rule{};
+  const float *qsig = nullptr, *qdsig = nullptr;
+  float edge[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
   // tree
   DevBuf<NodeLink> link;
   DevBuf<float> cm, spec, src_pos;
@@ -188,6 +196,8 @@ struct Ctx {
     sig.release();
     hsig.release();
     dsig.release();
+    rule_buf.release();
+    weight.release();
     link.release();
     cm.release();
     spec.release();
@@ -294,51 +304,114 @@ RateTables rate_tables(const Ctx& g) {
     t.cs_max[s] = g.cs_max[s];
     t.cs_last[s] = g.cs_last[s];
   }
+  t.qsig = g.qsig;
+  t.qdsig = g.qdsig;
+  memcpy(t.edge, g.edge, sizeof t.edge);
   return t;
 }
 
 // Tables of run_param (freq.nu, csect) in the layouts the kernels read.
-void upload_tables(Ctx& g, const run_param* r) {
+struct HostTables {
+  std::vector<float> nu, cs, sig, hsig, dsig;
+  double cs_max[3], cs_last[3];
+  int k_he1, k_he2;   // first bins with HeI, with HeII (cross-section or heating weight)
+};
+
+HostTables host_tables(const run_param* r) {
   const int ng = ARGOT_NGRID_NU;
-  std::vector<float> nu(ng), cs(3 * ng), sig(3 * ng), hsig(3 * ng), dsig(3 * ng);
+  HostTables t{std::vector<float>(ng), std::vector<float>(3 * ng), std::vector<float>(3 * ng),
+               std::vector<float>(3 * ng), std::vector<float>(3 * ng), {0, 0, 0}, {0, 0, 0}, 0, 0};
   const double thr[3] = {1.0, 1.8125, 4.0};   // HI, HeI, HeII limits [nu_L]
   for (int k = 0; k < ng; k++) {
-    nu[k] = (float)r->freq.nu[k];
+    t.nu[k] = (float)r->freq.nu[k];
     const float c[3] = {r->csect[k].csect_HI, r->csect[k].csect_HeI, r->csect[k].csect_HeII};
     for (int s = 0; s < 3; s++) {
-      cs[3 * k + s] = c[s];
-      sig[s * ng + k] = c[s];
-      hsig[s * ng + k] =
-          (double)nu[k] > thr[s] ? (float)((double)c[s] * ((double)nu[k] - thr[s])) : 0.0f;
+      t.cs[3 * k + s] = c[s];
+      t.sig[s * ng + k] = c[s];
+      t.hsig[s * ng + k] =
+          (double)t.nu[k] > thr[s] ? (float)((double)c[s] * ((double)t.nu[k] - thr[s])) : 0.0f;
     }
   }
   for (int s = 0; s < 3; s++) {
     double mx = 0.0;
-    for (int k = 0; k < ng; k++) mx = std::max(mx, (double)sig[s * ng + k]);
-    g.cs_max[s] = mx;
-    g.cs_last[s] = sig[s * ng + ng - 1];
+    for (int k = 0; k < ng; k++) mx = std::max(mx, (double)t.sig[s * ng + k]);
+    t.cs_max[s] = mx;
+    t.cs_last[s] = t.sig[s * ng + ng - 1];
     for (int k = 0; k < ng; k++)
-      dsig[s * ng + k] = (float)((double)sig[s * ng + k] - g.cs_last[s]);
+      t.dsig[s * ng + k] = (float)((double)t.sig[s * ng + k] - t.cs_last[s]);
   }
   // Bin ranges with absent species (sigma and heating weight both zero).
   auto first_nonzero = [&](int s) {
     for (int k = 0; k < ng; k++)
-      if (sig[s * ng + k] != 0.0f || hsig[s * ng + k] != 0.0f) return k;
+      if (t.sig[s * ng + k] != 0.0f || t.hsig[s * ng + k] != 0.0f) return k;
     return ng;
   };
-  g.k_he2 = first_nonzero(2);
-  g.k_he1 = std::min(first_nonzero(1), g.k_he2);
+  t.k_he2 = first_nonzero(2);
+  t.k_he1 = std::min(first_nonzero(1), t.k_he2);
+  return t;
+}
+
+// The quadrature rule of the tables.  The last one is kept (its matrices take
+// about 0.6 ms to form, and every context of a program has the same tables);
+// it is taken again only for tables with the same values.
+std::mutex g_rule_mu;
+std::vector<float> g_rule_key;
+std::shared_ptr<const RateRule> g_rule;
+
+std::shared_ptr<const RateRule> rate_rule(const HostTables& t) {
+  std::vector<float> key(t.sig);
+  key.insert(key.end(), t.hsig.begin(), t.hsig.end());
+  std::lock_guard<std::mutex> lk(g_rule_mu);
+  if (!g_rule || key.size() != g_rule_key.size() ||
+      memcmp(key.data(), g_rule_key.data(), sizeof(float) * key.size()) != 0) {
+    auto made = std::make_shared<RateRule>();
+    build_rate_rule(t.sig.data(), t.hsig.data(), ARGOT_NGRID_NU, t.k_he1, t.k_he2, made.get());
+    g_rule = std::move(made);
+    g_rule_key = std::move(key);
+  }
+  return g_rule;
+}
+
+void upload_tables(Ctx& g, const run_param* r) {
+  const int ng = ARGOT_NGRID_NU;
+  const HostTables t = host_tables(r);
+  for (int s = 0; s < 3; s++) {
+    g.cs_max[s] = t.cs_max[s];
+    g.cs_last[s] = t.cs_last[s];
+  }
+  g.k_he1 = t.k_he1;
+  g.k_he2 = t.k_he2;
   g.ngrid = ng;
   HIP_OK(g.nu.reserve(ng));
   HIP_OK(g.cs.reserve(3 * ng));
   HIP_OK(g.sig.reserve(3 * ng));
   HIP_OK(g.hsig.reserve(3 * ng));
   HIP_OK(g.dsig.reserve(3 * ng));
-  HIP_OK(hipMemcpy(g.nu.p, nu.data(), ng * sizeof(float), hipMemcpyHostToDevice));
-  HIP_OK(hipMemcpy(g.cs.p, cs.data(), 3 * ng * sizeof(float), hipMemcpyHostToDevice));
-  HIP_OK(hipMemcpy(g.sig.p, sig.data(), 3 * ng * sizeof(float), hipMemcpyHostToDevice));
-  HIP_OK(hipMemcpy(g.hsig.p, hsig.data(), 3 * ng * sizeof(float), hipMemcpyHostToDevice));
-  HIP_OK(hipMemcpy(g.dsig.p, dsig.data(), 3 * ng * sizeof(float), hipMemcpyHostToDevice));
+  HIP_OK(hipMemcpy(g.nu.p, t.nu.data(), ng * sizeof(float), hipMemcpyHostToDevice));
+  HIP_OK(hipMemcpy(g.cs.p, t.cs.data(), 3 * ng * sizeof(float), hipMemcpyHostToDevice));
+  HIP_OK(hipMemcpy(g.sig.p, t.sig.data(), 3 * ng * sizeof(float), hipMemcpyHostToDevice));
+  HIP_OK(hipMemcpy(g.hsig.p, t.hsig.data(), 3 * ng * sizeof(float), hipMemcpyHostToDevice));
+  HIP_OK(hipMemcpy(g.dsig.p, t.dsig.data(), 3 * ng * sizeof(float), hipMemcpyHostToDevice));
+  const std::shared_ptr<const RateRule> kept = rate_rule(t);
+  const RateRule& rule = *kept;
+  g.rule = RuleDev{};
+  g.rule.usable = rule.usable ? 1 : 0;
+  for (int k = 0; k < 4; k++) g.rule.start[k] = rule.usable ? rule.start[k] : 0;
+  memcpy(g.edge, rule.edge, sizeof g.edge);
+  // project (double), then test, sig and dsig (float; sizes multiples of 4)
+  const size_t np = rule.project.size(), nt = rule.test.size(), ns = rule.sig.size();
+  std::vector<double> buf(np + (nt + 2 * ns) / 2);
+  std::copy(rule.project.begin(), rule.project.end(), buf.begin());
+  float* const f = reinterpret_cast<float*>(buf.data() + np);
+  std::copy(rule.test.begin(), rule.test.end(), f);
+  std::copy(rule.sig.begin(), rule.sig.end(), f + nt);
+  std::copy(rule.dsig.begin(), rule.dsig.end(), f + nt + ns);
+  HIP_OK(g.rule_buf.reserve(buf.size()));
+  HIP_OK(hipMemcpy(g.rule_buf.p, buf.data(), buf.size() * sizeof(double), hipMemcpyHostToDevice));
+  g.rule.project = g.rule_buf.p;
+  g.rule.test = reinterpret_cast<const float*>(g.rule_buf.p + np);
+  g.qsig = g.rule.test + nt;
+  g.qdsig = g.qsig + ns;
 }
 
 // The caller's context, ready and for a mesh of this_run's size, or null
@@ -974,13 +1047,19 @@ static void calc_photoion_rate_cuda_body(struct cuda_mem_space* cuda_mem, struct
   HIP_OK(hipMemcpyAsync(d, stage, off_tab, hipMemcpyHostToDevice, g.stream));
   HIP_OK(hipMemcpyAsync(d + off_tab, tab, tab_bytes, hipMemcpyHostToDevice, g.stream));
   const RateTables rt = rate_tables(g);
-  HIP_OK(hipEventRecord(g.ev_c0, g.stream));
-  HIP_OK(launch_target_rates(
-      gd, rt, g.mesh, reinterpret_cast<const CallTarget*>(d + sizeof(CallRay) * nray), ntarget,
-      reinterpret_cast<const CallRay*>(d), reinterpret_cast<const float*>(d + off_tab),
+  HIP_OK(g.weight.reserve((size_t)nspec * (kRuleWeights + 1)));
+  float* const limit = g.weight.p + (size_t)nspec * kRuleWeights;
+  const CallSpectra spectra{
+      reinterpret_cast<const float*>(d + off_tab),
       reinterpret_cast<const double*>(d + off_tab + sizeof(float) * ng * nspec),
       reinterpret_cast<const double*>(d + off_tab + (sizeof(float) + sizeof(double)) * ng * nspec),
-      g.stream));
+      g.weight.p, limit};
+  HIP_OK(hipEventRecord(g.ev_c0, g.stream));
+  HIP_OK(launch_project_spectra(g.rule, spectra.spec32, (int)nspec, ng, g.weight.p, limit,
+                                g.stream));
+  HIP_OK(launch_target_rates(
+      gd, rt, g.mesh, reinterpret_cast<const CallTarget*>(d + sizeof(CallRay) * nray), ntarget,
+      reinterpret_cast<const CallRay*>(d), spectra, g.stream));
   HIP_OK(hipEventRecord(g.ev_c1, g.stream));
   HIP_OK(hipStreamSynchronize(g.stream));
   float ms = 0.0f;
@@ -1148,6 +1227,11 @@ static void point_source_pass(Ctx& g, struct radiation_src* src, struct run_para
   HIP_OK(hipMemcpyAsync(g.src_pos.p, T.src_pos.data(), sizeof(float) * T.src_pos.size(),
                         hipMemcpyHostToDevice, g.stream));
   const double t_built = now_ms();
+  // Every spectrum's quadrature weights, on the stream before the fused kernel.
+  HIP_OK(g.weight.reserve((size_t)nn * (kRuleWeights + 1)));
+  float* const limit = g.weight.p + (size_t)nn * kRuleWeights;
+  HIP_OK(launch_project_spectra(g.rule, g.spec.p, nn, ARGOT_NGRID_NU, g.weight.p, limit,
+                                g.stream));
 
   FusedArgs a{};   // zero-initialised: the graph cache compares its bytes
   a.grid = make_grid(this_run);
@@ -1158,6 +1242,8 @@ static void point_source_pass(Ctx& g, struct radiation_src* src, struct run_para
   a.tree.spec = g.spec.p;
   a.tree.spec_scale = g.spec_scale.p;
   a.tree.src_pos = g.src_pos.p;
+  a.tree.weight = g.weight.p;
+  a.tree.limit = limit;
   a.rates = rate_tables(g);
   // With no trusted cell every ray would take the exact integral, so the
   // plain kernel runs.
@@ -1630,6 +1716,26 @@ int argot_hip_segment_start(const struct run_param* r, const float* src, int ix,
   start[1] = st.y;
   start[2] = st.z;
   return n;
+}
+
+// The quadrature rule of run_param's tables on the host: cross-sections
+// sigma_s and sigma_s - sigma_s(last) at its nodes [3 * 44 each], and the
+// weights [nspec * 192] and limits [nspec] of FP32 spectra [nspec * 256].
+// Returns the number of nodes, 0 where the tables have no rule.
+int argot_hip_rate_rule(const struct run_param* r, const float* spec, int nspec, float* sig,
+                        float* dsig, float* weight, float* limit) {
+  try {
+    const HostTables t = host_tables(r);
+    RateRule rule;
+    build_rate_rule(t.sig.data(), t.hsig.data(), ARGOT_NGRID_NU, t.k_he1, t.k_he2, &rule);
+    memcpy(sig, rule.sig.data(), sizeof(float) * rule.sig.size());
+    memcpy(dsig, rule.dsig.data(), sizeof(float) * rule.dsig.size());
+    project_spectra_host(rule, spec, nspec, ARGOT_NGRID_NU, weight, limit);
+    return rule.usable ? kRuleNodes : 0;
+  } catch (const std::bad_alloc&) {
+    set_err(ARGOT_ERR_NOMEM);
+  }
+  return 0;
 }
 
 // Product tree on the host: build from nsrc sources and list the rays of a

@@ -42,7 +42,7 @@ def algorithmic_bytes(nray, ncross, ncell):
 # Sources that define the fused kernel's code: a committed profile figure is
 # used only when it was measured on these exact sources.
 KERNEL_SOURCES = ("kernels.hip", "argot_device.h", "argot_internal.h", "kernels.h", "mlp.h",
-                  "surrogate.h", "Makefile")
+                  "rate_rule.h", "surrogate.h", "Makefile")
 
 
 def kernel_source_hash():
