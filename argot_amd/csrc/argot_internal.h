@@ -103,16 +103,21 @@ struct CallTarget {
   int32_t g[3];      // global cell indices (target centre)
 };
 
+// Work counters of one fused launch.  Each tile queue (one per XCD) has a
+// cache line of its own with its next tile and the counts of the blocks of
+// that XCD; the host adds them up.
 struct StepCounters {
-  unsigned long long nray;
-  unsigned long long ncross;
-  unsigned long long nfallback;
   unsigned long long nrecord;
-  unsigned long long nsurrogate;
-  unsigned long long nvisit;       // tree nodes visited, summed over wavefronts
-  unsigned long long nemit_iter;   // of those, visits where some lane emitted a ray
   unsigned long long noverflow;    // rays that would need NSEG_PER_RAY or more segments
-  int queue[kNumQueues];
+  struct alignas(128) Queue {
+    int next;
+    unsigned long long nray;
+    unsigned long long ncross;
+    unsigned long long nfallback;
+    unsigned long long nsurrogate;
+    unsigned long long nvisit;       // tree nodes visited, summed over wavefronts
+    unsigned long long nemit_iter;   // of those, visits where some lane emitted a ray
+  } queue[kNumQueues];
 };
 
 // Run-time parameters of the chemistry (from struct run_param, plus the

@@ -1320,18 +1320,27 @@ static void point_source_pass(Ctx& g, struct radiation_src* src, struct run_para
     HIP_OK(hipMemcpy(g_capture_host, g.rec.p, sizeof(RayRecord) * n, hipMemcpyDeviceToHost));
   }
   g.stats.ntarget = (uint64_t)g.ncell;
-  g.stats.nray = hc.nray;
-  g.stats.ncross = hc.ncross;
-  g.stats.nfallback = hc.nfallback;
-  g.stats.nsurrogate = hc.nsurrogate;
-  g.stats.nvisit = hc.nvisit;
-  g.stats.nemit_iter = hc.nemit_iter;
+  StepCounters::Queue sum{};
+  for (const StepCounters::Queue& q : hc.queue) {
+    sum.nray += q.nray;
+    sum.ncross += q.ncross;
+    sum.nfallback += q.nfallback;
+    sum.nsurrogate += q.nsurrogate;
+    sum.nvisit += q.nvisit;
+    sum.nemit_iter += q.nemit_iter;
+  }
+  g.stats.nray = sum.nray;
+  g.stats.ncross = sum.ncross;
+  g.stats.nfallback = sum.nfallback;
+  g.stats.nsurrogate = sum.nsurrogate;
+  g.stats.nvisit = sum.nvisit;
+  g.stats.nemit_iter = sum.nemit_iter;
   g.stats.noverflow = hc.noverflow;
   g.stats.ms_build = t_built - t_start;
   g.stats.ms_kernel = ms;
   g.stats.ms_total = now_ms() - t_start;
-  this_run->nray = hc.nray;
-  this_run->nseg = hc.nray;
+  this_run->nray = sum.nray;
+  this_run->nseg = sum.nray;
   // The reference asserts num_segment < NSEG_PER_RAY for every ray
   // (calc_ray_segment.c:212); here the step reports it.
   if (hc.noverflow) set_err(ARGOT_ERR_TOO_MANY_SEGMENTS);
