@@ -101,6 +101,7 @@ def lib():
     L.argot_hip_segment_start.argtypes = [rp, C.c_void_p, C.c_int, C.c_int, C.c_int,
                                           C.c_void_p]
     L.argot_hip_segment_start.restype = C.c_int
+    L.argot_hip_quotients.argtypes = 3 * [C.c_void_p] + [C.c_int64]
     L.argot_hip_rate_rule.argtypes = [rp, C.c_void_p, C.c_int] + 4 * [C.c_void_p]
     L.argot_hip_rate_rule.restype = C.c_int
     L.argot_hip_tree_build.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_void_p,

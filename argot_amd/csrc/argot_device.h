@@ -35,6 +35,35 @@ __device__ __forceinline__ float div_by(float a, double rb) {
   return (float)((double)a * rb);
 }
 
+// Exact quotients, reciprocals and roots in FP32.  On gfx950 an FP32
+// multiply-add issues in 2 cycles per wavefront, FP64, conversions and
+// comparisons in 4, a reciprocal estimate in 8; the library's IEEE sequences
+// take 30 to 60 cycles, an FP64 detour 12 and more.
+//
+// RN(a/b) from hi = RN(1/b): a*hi lies within 1.5 ulp of a/b, and adding
+// residual * hi brings the unrounded sum to within 2^-21 ulp of it.  It then
+// rounds as a/b does unless a/b lies that close to the middle of two floats;
+// every pair of 24-bit significands whose quotient does (8.7e7 of them) was
+// tried, and all came out right.  Holds where nothing underflows: |a| zero or
+// above 1e-30, |b| between 1e-31 and 1e30.
+ARGOT_HD inline float div_exact(float a, float b, float hi) {
+  const float q = a * hi;
+  return __builtin_fmaf(__builtin_fmaf(-q, b, a), hi, q);
+}
+// RN(1/b): the estimate and one Newton step (checked against IEEE division
+// for every significand and the exponents -107 to 52).
+__device__ __forceinline__ float rcp_exact(float b) {
+  const float y = __builtin_amdgcn_rcpf(b);
+  return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+}
+// RN(sqrt(s)) (checked against IEEE sqrt for every significand and the
+// exponents -75 to 52).
+__device__ __forceinline__ float sqrt_exact(float s) {
+  const float y = __builtin_amdgcn_rsqf(s);
+  const float g = s * y;
+  return __builtin_fmaf(__builtin_fmaf(-g, g, s), 0.5f * y, g);
+}
+
 // Target cell centre, setup_light_ray_tree.c:341-343 / calc_ray_segment.c:48:
 // (float)i + 0.5 is double, the sum is rounded to float once.
 ARGOT_HD inline float cell_centre(float lo, int i, float h) {
@@ -60,11 +89,25 @@ ARGOT_HD inline int segment_start(const GridDev& g, Vec3f src, Vec3f tgt, Vec3f*
   const float dxd = (g.xmax - g.xmin) / 1.0f;
   const float dyd = (g.ymax - g.ymin) / 1.0f;
   const float dzd = (g.zmax - g.zmin) / 1.0f;
+  const bool inside = !(src.x < g.xmin || src.x > g.xmax || src.y < g.ymin || src.y > g.ymax ||
+                        src.z < g.zmin || src.z > g.zmax);
+  // Source and target both in the box: the domain index (int)(a/d) of an
+  // offset 0 <= a <= d is 1 where a = d and 0 elsewhere (a smaller float's
+  // quotient is at most 1 - 2^-24), so no division is needed to see that the
+  // two lie in the same domain.
+  {
+    const float ax = tgt.x - g.xmin, ay = tgt.y - g.ymin, az = tgt.z - g.zmin;
+    const bool tgt_inside =
+        ax >= 0.0f && ax <= dxd && ay >= 0.0f && ay <= dyd && az >= 0.0f && az <= dzd;
+    if (inside && tgt_inside && (src.x - g.xmin >= dxd) == (ax >= dxd) &&
+        (src.y - g.ymin >= dyd) == (ay >= dyd) && (src.z - g.zmin >= dzd) == (az >= dzd)) {
+      *start = src;
+      return 1;
+    }
+  }
   const int ixt = (int)((tgt.x - g.xmin) / dxd);
   const int iyt = (int)((tgt.y - g.ymin) / dyd);
   const int izt = (int)((tgt.z - g.zmin) / dzd);
-  const bool inside = !(src.x < g.xmin || src.x > g.xmax || src.y < g.ymin || src.y > g.ymax ||
-                        src.z < g.zmin || src.z > g.zmax);
   if (inside) {
     const int ixs = (int)((src.x - g.xmin) / dxd);
     const int iys = (int)((src.y - g.ymin) / dyd);
@@ -131,6 +174,52 @@ ARGOT_HD inline int segment_start(const GridDev& g, Vec3f src, Vec3f tgt, Vec3f*
   start->y = sy;
   start->z = sz;
   return nseg;
+}
+
+// Direction of a ray as the walk forms it (calc_optical_depth.c:103-127), its
+// cosines' reciprocals, and its length.  The reference takes roots in double,
+// with TINY added, and two quotients in double; where x^2 + y^2 exceeds 1e-12
+// TINY is below half an ulp of the double it is added to, and a double root or
+// quotient of floats rounds to float as the float operation does (53 bits are
+// more than twice 24 plus 2), so FP32 gives the same bits.  plain: that was
+// so, and calc_photoion_rate's chord has the same cosines.
+struct RayDir {
+  float xo, yo, zo;   // direction cosines (with the TINY guards)
+  float hx, hy, hz;   // RN(1/xo) etc.
+  float dist;         // (float)sqrt(dx^2 + dy^2 + dz^2); plain only
+  bool plain;
+};
+
+__device__ inline RayDir ray_dir(float dx, float dy, float dz) {
+  RayDir d;
+  const float s2 = dx * dx + dy * dy;
+  const float s3 = s2 + dz * dz;
+  d.plain = s2 > 1.0e-12f && s3 < 1.0e12f;
+  if (d.plain) {
+    const float dl = sqrt_exact(s3), dxy = sqrt_exact(s2);
+    const float rl = rcp_exact(dl), rxy = rcp_exact(dxy);
+    const float sin_t = div_exact(dxy, dl, rl);
+    d.zo = div_exact(dz, dl, rl);
+    d.xo = div_exact(dx, dxy, rxy) * sin_t;
+    d.yo = div_exact(dy, dxy, rxy) * sin_t;
+    d.dist = dl;
+  } else {
+    const float dl = (float)__builtin_sqrt((double)s3 + kWalkTiny);
+    const float dxy = (float)__builtin_sqrt((double)s2);
+    const float sin_t = dxy / dl;
+    d.zo = dz / dl;
+    d.xo = (float)((double)dx / ((double)dxy + kWalkTiny)) * sin_t;
+    d.yo = (float)((double)dy / ((double)dxy + kWalkTiny)) * sin_t;
+    d.dist = 0.0f;
+  }
+  constexpr float kTinyF = (float)kWalkTiny;   // (a smaller magnitude, and only one, becomes it)
+  if (!(fabsf(d.xo) >= kTinyF)) d.xo = d.xo >= 0.0f ? kTinyF : -kTinyF;
+  if (!(fabsf(d.yo) >= kTinyF)) d.yo = d.yo >= 0.0f ? kTinyF : -kTinyF;
+  if (!(fabsf(d.zo) >= kTinyF)) d.zo = d.zo >= 0.0f ? kTinyF : -kTinyF;
+  d.hx = rcp_exact(d.xo);
+  d.hy = rcp_exact(d.yo);
+  d.hz = rcp_exact(d.zo);
+  return d;
 }
 
 // Per-ray state of the DDA walk, calc_optical_depth.c:76-143.  Along each
@@ -242,6 +331,103 @@ __device__ inline void dda_setup(const GridDev& g, Vec3f s, Vec3f e, Dda* d) {
   d->zc = s.z - g.zmin;
 }
 
+// The state of the walk in its float form (walk_float): as Dda, but all of it
+// FP32, the index too (a byte offset, a multiple of 16 below 2^28, is exact).
+struct DdaF {
+  float fx, fy, fz;
+  float sdx, sdy, sdz;
+  float stx, sty, stz;
+  float idx, idxe;
+  float xo, yo, zo;
+  float hx, hy, hz;
+  float xc, yc, zc;
+};
+
+// Cell of a coordinate, calc_optical_depth.c:84-101.
+__device__ __forceinline__ int cell_of(float a, float h, float rh, int n) {
+  return max(min((int)div_exact(a, h, rh), n - 1), 0);
+}
+
+template <bool POW2>
+__device__ inline DdaF dda_float(const GridDev& g, const RayDir& r, Vec3f s, Vec3f e) {
+  DdaF d;
+  d.xc = s.x - g.xmin;
+  d.yc = s.y - g.ymin;
+  d.zc = s.z - g.zmin;
+  const int ix = cell_of(d.xc, g.dx, g.rdx, g.nx), iy = cell_of(d.yc, g.dy, g.rdy, g.ny),
+            iz = cell_of(d.zc, g.dz, g.rdz, g.nz);
+  d.idx = (float)(int)(cell_index(g, ix, iy, iz) * 16u);
+  d.idxe = (float)(int)(cell_index(g, cell_of(e.x - g.xmin, g.dx, g.rdx, g.nx),
+                                   cell_of(e.y - g.ymin, g.dy, g.rdy, g.ny),
+                                   cell_of(e.z - g.zmin, g.dz, g.rdz, g.nz)) *
+                        16u);
+  d.xo = r.xo, d.yo = r.yo, d.zo = r.zo;
+  d.hx = r.hx, d.hy = r.hy, d.hz = r.hz;
+  const bool px = r.xo > 0.0f, py = r.yo > 0.0f, pz = r.zo > 0.0f;
+  d.sdx = px ? g.dx : -g.dx;
+  d.sdy = py ? g.dy : -g.dy;
+  d.sdz = pz ? g.dz : -g.dz;
+  if constexpr (POW2) {
+    d.fx = (px ? (float)ix + 1.0f : (float)ix) * g.dx;
+    d.fy = (py ? (float)iy + 1.0f : (float)iy) * g.dy;
+    d.fz = (pz ? (float)iz + 1.0f : (float)iz) * g.dz;
+  } else {
+    d.fx = px ? (float)ix + 1.0f : -(float)ix;
+    d.fy = py ? (float)iy + 1.0f : -(float)iy;
+    d.fz = pz ? (float)iz + 1.0f : -(float)iz;
+  }
+  const float sy = (float)(g.nz * 16), sx = (float)(g.ny * g.nz * 16);
+  d.stx = px ? sx : -sx;
+  d.sty = py ? sy : -sy;
+  d.stz = pz ? 16.0f : -16.0f;
+  return d;
+}
+
+// 1 where r equals the smallest distance m, else 0: r - m is +0 or positive,
+// and 1 - 2^126 (r - m) clamped to [0, 1] is 1 or, for any difference of at
+// least 2^-126, 0.  (A comparison and the selects it steers take 4 cycles each
+// on gfx950; the difference and this multiply-add take 2 each, and the result
+// multiplies straight into the updates.)
+__device__ __forceinline__ float is_smallest(float r, float m) {
+  float u;
+  asm("v_fma_f32 %0, %1, %2, 1.0 clamp" : "=v"(u) : "v"(r - m), "s"(-0x1p126f));
+  return u;
+}
+
+// One step of calc_optical_depth.c:163-179 in the float form.
+template <bool POW2>
+__device__ __forceinline__ float dda_step(DdaF* d) {
+  const float ddx = (POW2 ? d->fx : d->sdx * d->fx) - d->xc;
+  const float ddy = (POW2 ? d->fy : d->sdy * d->fy) - d->yc;
+  const float ddz = (POW2 ? d->fz : d->sdz * d->fz) - d->zc;
+  const float rx = div_exact(ddx, d->xo, d->hx);
+  const float ry = div_exact(ddy, d->yo, d->hy);
+  const float rz = div_exact(ddz, d->zo, d->hz);
+  const float rmin = fminf(rx, fminf(ry, rz));
+  const float ux = is_smallest(rx, rmin), uy = is_smallest(ry, rmin), uz = is_smallest(rz, rmin);
+  d->fx = POW2 ? __builtin_fmaf(ux, d->sdx, d->fx) : d->fx + ux;
+  d->fy = POW2 ? __builtin_fmaf(uy, d->sdy, d->fy) : d->fy + uy;
+  d->fz = POW2 ? __builtin_fmaf(uz, d->sdz, d->fz) : d->fz + uz;
+  d->idx = __builtin_fmaf(ux, d->stx, __builtin_fmaf(uy, d->sty, __builtin_fmaf(uz, d->stz, d->idx)));
+  d->xc = d->xc + rmin * d->xo;
+  d->yc = d->yc + rmin * d->yo;
+  d->zc = d->zc + rmin * d->zo;
+  return rmin;
+}
+
+// Is the current cell inside the mesh?  (A walk that has left never returns.)
+template <bool POW2>
+__device__ __forceinline__ bool dda_inside(const GridDev& g, const DdaF& d) {
+  const bool px = d.xo > 0.0f, py = d.yo > 0.0f, pz = d.zo > 0.0f;
+  if constexpr (POW2)
+    return ((d.fx < (px ? (float)g.nx + 0.5f : -0.5f) * g.dx) == px) &
+           ((d.fy < (py ? (float)g.ny + 0.5f : -0.5f) * g.dy) == py) &
+           ((d.fz < (pz ? (float)g.nz + 0.5f : -0.5f) * g.dz) == pz);
+  else
+    return (d.fx < (px ? (float)(g.nx + 1) : 1.0f)) & (d.fy < (py ? (float)(g.ny + 1) : 1.0f)) &
+           (d.fz < (pz ? (float)(g.nz + 1) : 1.0f));
+}
+
 // The walk continues while the current cell lies inside the mesh and is not
 // the end cell (the index is meaningful only when the cell is inside).
 template <bool POW2>
@@ -275,8 +461,9 @@ __device__ __forceinline__ float dda_step(Dda* d) {
 }
 
 // calc_optical_depth.c:194-203: length from the last face to the end point.
-__device__ __forceinline__ float dda_depth(const GridDev& g, const Dda& d, Vec3f e) {
-  const float x = d.xc + g.xmin, y = d.yc + g.ymin, z = d.zc + g.zmin;
+__device__ __forceinline__ float dda_depth(const GridDev& g, float xc, float yc, float zc,
+                                           Vec3f e) {
+  const float x = xc + g.xmin, y = yc + g.ymin, z = zc + g.zmin;
   const float ex = e.x - x, ey = e.y - y, ez = e.z - z;
   return (float)__builtin_sqrt((double)(ex * ex + ey * ey + ez * ez));
 }
@@ -300,6 +487,7 @@ __device__ __forceinline__ void kahan_add(float& s, float& c, float term) {
 // reads zeros or another cell's data, never memory outside the array, so
 // the walk need not redirect the loads of lanes that have left the mesh).
 constexpr int64_t kNarrowCells = (int64_t)1 << 28;
+constexpr int64_t kFloatCells = (int64_t)1 << 24;
 constexpr int kBufferWord3 = 0x00020000;   // raw 32-bit buffer, gfx9 layout
 
 // Per-cell FP32 densities (nHI, nHeI, nHeII) from the packed float4 array.
@@ -324,6 +512,98 @@ struct PackedFields {
     }
   }
 };
+
+// The walk in its float form: the same operations on the same values as the
+// walk below (every optical depth and position has its bits), arranged for
+// gfx950's issue rates, where FP32 products and sums take 2 cycles per
+// wavefront and comparisons, selects, conversions and FP64 take 4: exact
+// quotients by FP32 multiply-adds, the face choice as 0/1 factors, the cell
+// index in FP32, and no test at each crossing whether the cell is inside the
+// mesh.  About 86 cycles per crossing instead of 136: with the gathers (26
+// cycles of the vector memory path each) this is what bounds the fused
+// kernel.  With the set-up around it in the same arithmetic (ray_dir) the step
+// on 256^3 cells and 4096 sources took 88 ms instead of 99, on 128^3 and 1024
+// with Kahan sums 31.5 instead of 35.2, on 72 x 58 x 87 and 250 4.9 instead of 5.7.
+// A walk normally ends in its end cell; one that misses
+// it (rounding has carried it past, or a face difference below 2^-126 was no
+// clean 0 or 1) runs on over range-checked loads to the cap of nx + ny + nz
+// crossings, more than any walk inside the mesh has, or meets the end cell's
+// index outside the mesh; both are seen afterwards, false is returned and
+// the caller walks the segment again in the other form.
+template <bool KAHAN, bool HASH, bool POW2, typename Fields>
+__device__ inline bool walk_float(const GridDev& g, const Fields& fields, const RayDir& dir,
+                                  Vec3f s, Vec3f e, WalkOut* out) {
+  DdaF d = dda_float<POW2>(g, dir, s, e);
+  float t0 = 0.0f, t1 = 0.0f, t2 = 0.0f;
+  float c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
+  int nc = 0;
+  uint64_t h = 0xcbf29ce484222325ull;
+  auto active = [&]() { return d.idx != d.idxe; };
+  auto load = [&]() { return fields((uint32_t)d.idx); };
+  auto mark = [&]() {
+    if (HASH) h = (h ^ (uint64_t)((uint32_t)d.idx >> 4)) * 0x100000001b3ull;
+  };
+  auto add = [&](float r, const float4& n) {
+    if (KAHAN) {
+      kahan_add(t0, c0, r * n.x);
+      kahan_add(t1, c1, r * n.y);
+      kahan_add(t2, c2, r * n.z);
+    } else {
+      t0 = t0 + r * n.x;
+      t1 = t1 + r * n.y;
+      t2 = t2 + r * n.z;
+    }
+  };
+  // Two field slots alternate over passes of two crossings, as below.
+  bool actA = active();
+  float4 nA = load();
+  float rA = 0.0f, rB = 0.0f;
+  bool actB = false;
+  if (actA) {
+    mark();
+    rA = dda_step<POW2>(&d);
+    actB = active();
+  }
+  float4 nB = load();
+  int passes = (g.nx + g.ny + g.nz) / 2 + 1;   // wave-uniform
+  while (actA && passes > 0) {
+    passes--;
+    nc++;
+    add(rA, nA);
+    bool a2 = false;
+    if (actB) {
+      mark();
+      rB = dda_step<POW2>(&d);
+      a2 = active();
+    }
+    nA = load();
+    bool a3 = false;
+    if (actB) {
+      nc++;
+      add(rB, nB);
+      if (a2) {
+        mark();
+        rA = dda_step<POW2>(&d);
+        a3 = active();
+      }
+    }
+    nB = load();
+    actA = a2;
+    actB = a3;
+  }
+  if (d.idx != d.idxe || !dda_inside<POW2>(g, d)) return false;
+  const float depth = dda_depth(g, d.xc, d.yc, d.zc, e);
+  const float4 n = load();
+  mark();
+  nc++;
+  add(depth, n);
+  out->tau[0] = t0;
+  out->tau[1] = t1;
+  out->tau[2] = t2;
+  out->ncross = nc;
+  out->hash = h;
+  return true;
+}
 
 // The whole walk of one segment (calc_optical_depth.c:76-227).  fields(idx)
 // gives the per-cell FP32 densities (nHI, nHeI, nHeII) formed as the
@@ -397,7 +677,7 @@ __device__ inline void walk_segment_with(const GridDev& g, const Fields& fields,
     actA = a2;
     actB = a3;
   } while (actA);
-  const float depth = dda_depth(g, d, e);
+  const float depth = dda_depth(g, d.xc, d.yc, d.zc, e);
   const uint32_t ie = d.idxe;
   float4 n = fields(ie);
   if (HASH) h = (h ^ (uint64_t)(ie / S)) * 0x100000001b3ull;
@@ -418,12 +698,17 @@ __device__ inline void walk_segment_with(const GridDev& g, const Fields& fields,
   out->hash = h;
 }
 
-// The walk over the packed per-cell densities nf (float4 per cell).
-template <bool KAHAN, bool HASH, bool NARROW, bool POW2>
+// The walk over the packed per-cell densities nf (float4 per cell) from s to
+// e, along dir (ray_dir of e - s).
+template <bool KAHAN, bool HASH, bool NARROW, bool POW2, bool FLOAT>
 __device__ __forceinline__ void walk_segment(const GridDev& g, const float4* __restrict__ nf,
-                                             Vec3f s, Vec3f e, WalkOut* out) {
+                                             const RayDir& dir, Vec3f s, Vec3f e, WalkOut* out) {
   const uint32_t nbytes = NARROW ? (uint32_t)((int64_t)g.nx * g.nyz * 16) : 0u;
-  walk_segment_with<KAHAN, HASH, POW2>(g, PackedFields<NARROW>{nf, nbytes}, s, e, out);
+  const PackedFields<NARROW> fields{nf, nbytes};
+  if constexpr (FLOAT) {
+    if (walk_float<KAHAN, HASH, POW2>(g, fields, dir, s, e, out)) return;
+  }
+  walk_segment_with<KAHAN, HASH, POW2>(g, fields, s, e, out);
 }
 
 // delta_length, calc_photoion_rate.c:52-90.
@@ -451,19 +736,26 @@ __device__ inline float delta_length(const GridDev& g, float dx, float dy, float
 struct RayRate {
   double t[3];    // column densities at the cell entry [cm^-2]
   double d[3];    // in-cell optical-depth weights n_s*delta*lunit
-  double r[3];    // 1/(n_s V_sh + TINY)
+  double v[3];    // n_s V_sh + TINY
 };
 
-__device__ inline void ray_rate_setup(const GridDev& g, const RateTables& rt, const float tau[3],
+// dir: ray_dir of tgt - src.
+__device__ inline void ray_rate_setup(const GridDev& g, const RayDir& dir, const float tau[3],
                                       Vec3f src, Vec3f tgt, float dens, float fHI, float fHeI,
                                       float fHeII, RayRate* rr) {
   const double col = g.lunit * g.denstonh;
   rr->t[0] = (double)tau[0] * col;
   rr->t[1] = (double)tau[1] * col;
   rr->t[2] = (double)tau[2] * col;
-  const float dx = tgt.x - src.x, dy = tgt.y - src.y, dz = tgt.z - src.z;
-  const float delta = delta_length(g, dx, dy, dz);
-  const float dist = (float)__builtin_sqrt((double)(dx * dx + dy * dy + dz * dz));
+  float delta = fminf(fabsf(div_exact(g.dx, dir.xo, dir.hx)),
+                      fminf(fabsf(div_exact(g.dy, dir.yo, dir.hy)),
+                            fabsf(div_exact(g.dz, dir.zo, dir.hz))));
+  float dist = dir.dist;
+  if (!dir.plain) {
+    const float dx = tgt.x - src.x, dy = tgt.y - src.y, dz = tgt.z - src.z;
+    delta = delta_length(g, dx, dy, dz);
+    dist = (float)__builtin_sqrt((double)(dx * dx + dy * dy + dz * dz));
+  }
   const double nH = (double)dens * g.denstonh;
   const double nHI = nH * (double)fHI;
   rr->d[0] = nHI * (double)delta * g.lunit;
@@ -479,9 +771,16 @@ __device__ inline void ray_rate_setup(const GridDev& g, const RateTables& rt, co
   const double b = (double)dist - 0.5 * (double)delta;
   const double lu = g.lunit;
   const double vsh = 4.0 * kPi / 3.0 * (a * a * a - b * b * b) * (lu * lu * lu);
-  rr->r[0] = 1.0 / (nHI * vsh + kRateTiny);
-  rr->r[1] = 1.0 / (nHeI * vsh + kRateTiny);
-  rr->r[2] = 1.0 / (nHeII * vsh + kRateTiny);
+  rr->v[0] = nHI * vsh + kRateTiny;
+  rr->v[1] = nHeI * vsh + kRateTiny;
+  rr->v[2] = nHeII * vsh + kRateTiny;
+}
+
+// 1/v to about an ulp of double: the estimate and two Newton steps.
+__device__ __forceinline__ double rcp_f64(double v) {
+  double y = __builtin_amdgcn_rcp(v);
+  y = __builtin_fma(__builtin_fma(-v, y, 1.0), y, y);
+  return __builtin_fma(__builtin_fma(-v, y, 1.0), y, y);
 }
 
 __device__ __forceinline__ double lane_value(double v, int lane) { return __shfl(v, lane, 64); }
@@ -505,7 +804,7 @@ __device__ inline void rate_f64_wave(const RateTables& rt, const RayRate& rr, bo
     for (int s = 0; s < 3; s++) {
       t[s] = lane_value(rr.t[s], owner);
       d[s] = lane_value(rr.d[s], owner);
-      r[s] = lane_value(rr.r[s], owner);
+      r[s] = 1.0 / lane_value(rr.v[s], owner);
     }
     double g[6] = {0, 0, 0, 0, 0, 0};   // Gamma HI, Heat HI, Gamma HeI, HeII, Heat HeI, HeII
     for (int k = lane; k < rt.ngrid; k += 64) {

@@ -30,6 +30,7 @@ struct GridDev {
   float dx, dy, dz;
   double lunit, denstonh, helium_fact;
   float theta_sq;   // SQR(theta_crit) in FP32 (setup_light_ray_tree.c:577)
+  float rdx, rdy, rdz;   // RN(1/dx) etc.
 };
 
 // Frequency tables (device pointers).  sig/hsig are [3][ngrid] SoA:

@@ -111,13 +111,39 @@ __global__ void set_rates_kernel(unsigned char* __restrict__ mesh, const float* 
 // estimated crossing count (counting sort in LDS), so that the lanes of a
 // wavefront walk segments of similar length; each segment's result does not
 // depend on which lane walks it.
-// Fields: where the per-cell densities come from (PackedFields: the packed
-// float4 array; MeshFields: the mesh records).  POW2: the DDA's face-position
-// form for power-of-two cell sizes.
+// walk(g, s, e, kahan, out) walks one segment: WalkPacked or WalkMesh.
 constexpr int kWalkBlock = 256;
-template <bool POW2, typename Fields>
+
+// The walk over packed densities (see walk_segment).
+template <bool NARROW, bool POW2, bool FLOAT>
+struct WalkPacked {
+  const float4* nf;
+  __device__ __forceinline__ void operator()(const GridDev& g, Vec3f s, Vec3f e, bool kahan,
+                                             WalkOut* w) const {
+    const RayDir dir = ray_dir(e.x - s.x, e.y - s.y, e.z - s.z);
+    if (kahan)
+      walk_segment<true, false, NARROW, POW2, FLOAT>(g, nf, dir, s, e, w);
+    else
+      walk_segment<false, false, NARROW, POW2, FLOAT>(g, nf, dir, s, e, w);
+  }
+};
+
+// The walk over the mesh records.
+template <bool POW2>
+struct WalkMesh {
+  MeshFields f;
+  __device__ __forceinline__ void operator()(const GridDev& g, Vec3f s, Vec3f e, bool kahan,
+                                             WalkOut* w) const {
+    if (kahan)
+      walk_segment_with<true, false, POW2>(g, f, s, e, w);
+    else
+      walk_segment_with<false, false, POW2>(g, f, s, e, w);
+  }
+};
+
+template <typename Walk>
 __global__ __launch_bounds__(kWalkBlock) void walk_segments_kernel(
-    GridDev g, Fields fields, unsigned char* __restrict__ seg, int64_t nseg, int kahan) {
+    GridDev g, Walk walk, unsigned char* __restrict__ seg, int64_t nseg, int kahan) {
   __shared__ unsigned bucket_lds[64];
   __shared__ unsigned perm_lds[kWalkBlock];
   const int t = threadIdx.x;
@@ -152,10 +178,7 @@ __global__ __launch_bounds__(kWalkBlock) void walk_segments_kernel(
   const Vec3f s{rec[4], rec[5], rec[6]};
   const Vec3f e{rec[7], rec[8], rec[9]};
   WalkOut w;
-  if (kahan)
-    walk_segment_with<true, false, POW2>(g, fields, s, e, &w);
-  else
-    walk_segment_with<false, false, POW2>(g, fields, s, e, &w);
+  walk(g, s, e, kahan != 0, &w);
   rec[10] = w.tau[0];
   rec[11] = w.tau[1];
   rec[12] = w.tau[2];
@@ -382,10 +405,12 @@ __device__ __forceinline__ void rate_all_nodes(const RateTables& rt, float cl1, 
 template <typename SpecF, typename WeightF>
 __device__ inline void rate_loop_f32(const RateTables& rt, const RayRate& rr, double scale,
                                      float limit, SpecF spec, WeightF weight, double out[6]) {
-  const double tsh = rr.t[0] * rt.cs_last[0] + rr.t[1] * rt.cs_last[1] + rr.t[2] * rt.cs_last[2];
+  const double sh2 = rr.t[2] * rt.cs_last[2];
+  const double sh1 = __builtin_fma(rr.t[1], rt.cs_last[1], sh2);
+  const double tsh = __builtin_fma(rr.t[0], rt.cs_last[0], sh1);
   const float n[3] = {(float)rr.t[0], (float)rr.t[1], (float)rr.t[2]};
-  const float c1 = (float)(-(rr.t[1] * rt.cs_last[1] + rr.t[2] * rt.cs_last[2]));
-  const float c2 = (float)(-(rr.t[2] * rt.cs_last[2]));
+  const float c1 = (float)-sh1;
+  const float c2 = (float)-sh2;
   // Scale of the ray against the rule's test columns, from its columns at the
   // far side of the cell (and, where the half-cell shift made one
   // negative, its negative part).
@@ -422,23 +447,24 @@ __device__ inline void rate_loop_f32(const RateTables& rt, const RayRate& rr, do
   const double fl = fmax(floor(xl), -2000.0);
   const double pre =
       scale * ldexp((double)__builtin_amdgcn_exp2f((float)(xl - fl)), (int)fl);
-  const double p0 = rr.r[0] * rr.d[0] * pre;
-  const double p1 = rr.r[1] * rr.d[1] * pre;
-  const double p2 = rr.r[2] * rr.d[2] * pre;
+  const double p0 = rcp_f64(rr.v[0]) * rr.d[0] * pre;
+  const double p1 = rcp_f64(rr.v[1]) * rr.d[1] * pre;
+  const double p2 = rcp_f64(rr.v[2]) * rr.d[2] * pre;
   double G[3] = {0, 0, 0}, H[3] = {0, 0, 0};
   // largest in-cell optical depth of this ray over the bins.  A wavefront
   // whose rays are all thin runs the thin loop; one with a thicker ray runs
   // the combined loop, in which a thin lane does the thin loop's operations
   // exactly, so a cell's rates do not depend on which rays share its
   // wavefront (tile shape, grid size).
-  const double dmax = rr.d[0] * rt.cs_max[0] + rr.d[1] * rt.cs_max[1] + rr.d[2] * rt.cs_max[2];
+  const float dmax = (float)rr.d[0] * (float)rt.cs_max[0] + (float)rr.d[1] * (float)rt.cs_max[1] +
+                     (float)rr.d[2] * (float)rt.cs_max[2];
   constexpr double kHalfLog2e = 0.5 * 1.4426950408889634;
   constexpr double kLog2eD = 1.4426950408889634;
   const float dl[3] = {(float)(rr.d[0] * -kHalfLog2e), (float)(rr.d[1] * -kHalfLog2e),
                        (float)(rr.d[2] * -kHalfLog2e)};
   const float nl[3] = {(float)(rr.t[0] * -kLog2eD), (float)(rr.t[1] * -kLog2eD),
                        (float)(rr.t[2] * -kLog2eD)};
-  const bool thin = dmax <= kThinMax;
+  const bool thin = dmax <= (float)kThinMax;
   if (nodes) {
     const float cl1 = c1 * -kLog2e, cl2 = c2 * -kLog2e;
     if (__all(thin))
@@ -537,21 +563,33 @@ __global__ __launch_bounds__(kProjectThreads) void project_spectra_kernel(
 
 // Lower bound of the shifted bin optical depth and upper bound of the
 // in-cell optical depth decide whether the FP32 loop is safe.
+// (In FP32: the bounds are far from where the loop would fail, and a column
+// beyond FP32's range is infinite here and fails.)
 __device__ __forceinline__ bool fast_rate_ok(const RateTables& rt, const RayRate& rr) {
-  double lo = 0.0, dmax = 0.0;
+  float lo = 0.0f, dmax = 0.0f;
   bool finite = true;
   for (int s = 0; s < 3; s++) {
-    lo += rr.t[s] >= 0.0 ? -rr.t[s] * rt.cs_last[s] : rr.t[s] * (rt.cs_max[s] - rt.cs_last[s]);
-    dmax += rr.d[s] * rt.cs_max[s];
-    finite = finite && fabs(rr.t[s]) < 1.0e36 && rr.d[s] < 1.0e36;
+    const float t = (float)rr.t[s], d = (float)rr.d[s];
+    const float last = (float)rt.cs_last[s], top = (float)rt.cs_max[s];
+    lo += t >= 0.0f ? -t * last : t * (top - last);
+    dmax += d * top;
+    finite = finite && fabsf(t) < 1.0e36f && d < 1.0e36f;
   }
-  return finite && lo > -60.0 && dmax < 1.0e30;
+  return finite && lo > -60.0f && dmax < 1.0e30f;
 }
 
 __device__ __forceinline__ int wave_min(int v) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) v = min(v, __shfl_xor(v, off, 64));
   return __builtin_amdgcn_readfirstlane(v);
+}
+
+// Orders the LDS accesses of the lanes of a wavefront before and after it (a
+// block of one wavefront needs no barrier: its LDS accesses are in order).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 template <typename T>
@@ -617,7 +655,8 @@ __global__ __launch_bounds__(64) ARGOT_CALL_OCCUPANCY void target_rates_kernel(
       const CallRay R = rays[r];
       u = R.spec;
       const Vec3f src{R.src[0], R.src[1], R.src[2]};
-      ray_rate_setup(g, rt, R.tau, src, tgt, dens, fHI, fHeI, fHeII, &rr);
+      const RayDir dir = ray_dir(tgt.x - src.x, tgt.y - src.y, tgt.z - src.z);
+      ray_rate_setup(g, dir, R.tau, src, tgt, dens, fHI, fHeI, fHeII, &rr);
       wide = !fast_rate_ok(rt, rr);
       if (!wide) {
         const float* s32 = sp.spec32 + (int64_t)u * ng;
@@ -729,7 +768,7 @@ __device__ inline void surr_rates(const RayRate& rr, double q, const float ya[kN
   double m[kNout];
 #pragma unroll
   for (int o = 0; o < kNout; o++) m[o] = 0.5 * (exp10_wide(ya[o]) + exp10_wide(yb[o]));
-  const double p0 = rr.r[0] * rr.d[0] * q, p1 = rr.r[1] * rr.d[1] * q, p2 = rr.r[2] * rr.d[2] * q;
+  const double p0 = rr.d[0] / rr.v[0] * q, p1 = rr.d[1] / rr.v[1] * q, p2 = rr.d[2] / rr.v[2] * q;
   res[0] = p0 * m[0];
   res[1] = p0 * m[3] * kHnuL;
   res[2] = p1 * m[1];
@@ -738,7 +777,7 @@ __device__ inline void surr_rates(const RayRate& rr, double q, const float ya[kN
   res[5] = p2 * m[5] * kHnuL;
 }
 
-template <bool KAHAN, bool CAPTURE, bool SURR, bool NARROW, bool POW2>
+template <bool KAHAN, bool CAPTURE, bool SURR, bool NARROW, bool POW2, bool FLOAT>
 __global__ __launch_bounds__(64) ARGOT_OCCUPANCY_FOR(SURR) void fused_step_kernel(FusedArgs a) {
   const GridDev& g = a.grid;
   const TreeDev& tr = a.tree;
@@ -766,13 +805,15 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY_FOR(SURR) void fused_step_kerne
   // bits); wave-uniform visit counts
   unsigned int my_ray = 0, my_cross = 0, my_fb = 0, my_surr = 0;
   unsigned long long my_visit = 0, my_emit_iter = 0;
-  // The lane's per-cell FP64 sums and its target's density and fractions
-  // live in LDS between rays, so that the walk and the frequency loop have
-  // the registers to themselves.
+  // The targets' per-cell FP64 sums, centres, and densities and fractions live
+  // in LDS between rays, by the target's place in the tile: the walk and the
+  // frequency loop have the registers to themselves, and a ray can be worked
+  // by any lane.
   __shared__ double acc_lds[6][64];
-  // (the surrogate variant reads the target's fields from the mesh at each
-  // ray instead, so that with the network's LDS it still fits 16 wavefronts
-  // per CU)
+  // (the surrogate variant passes centres between lanes and reads the
+  // target's fields from the mesh at each ray instead, so that with the
+  // network's LDS it still fits 16 wavefronts per CU)
+  __shared__ float4 tgt_lds[SURR ? 1 : 64];
   __shared__ float4 cell_lds[SURR ? 1 : 64];
   float* lds = nullptr;
   if constexpr (SURR) {
@@ -794,22 +835,44 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY_FOR(SURR) void fused_step_kerne
       ty = (int)((t / ntz) % nty);
       tx = (int)(t / ((int64_t)ntz * nty));
     }
+    // The lane's own target: it follows the tree for it and adds its sums to
+    // the mesh at the end.
     const int ix = tx * TX + ((lane >> (by + bz)) & (TX - 1));
     const int iy = ty * TY + ((lane >> bz) & (TY - 1));
     const int iz = tz * TZ + (lane & (TZ - 1));
     const bool valid = ix < g.nx && iy < g.ny && iz < g.nz;
     const int64_t cell = (int64_t)iz + (int64_t)g.nz * ((int64_t)iy + (int64_t)g.ny * ix);
-    const Vec3f tgt{cell_centre(g.gxmin, ix + g.ox, g.dx), cell_centre(g.gymin, iy + g.oy, g.dy),
-                    cell_centre(g.gzmin, iz + g.oz, g.dz)};
+    float4 mine;
     {
       float4 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       if (valid)
         f = make_float4(*mesh_f(a.mesh, cell, kOffDens), *mesh_f(a.mesh, cell, kOffFHI),
                         *mesh_f(a.mesh, cell, kOffFHeI), *mesh_f(a.mesh, cell, kOffFHeII));
-      if constexpr (!SURR) cell_lds[lane] = f;
+      mine = make_float4(cell_centre(g.gxmin, ix + g.ox, g.dx),
+                         cell_centre(g.gymin, iy + g.oy, g.dy),
+                         cell_centre(g.gzmin, iz + g.oz, g.dz), 0.0f);
+      if constexpr (!SURR) {
+        cell_lds[lane] = f;
+        tgt_lds[lane] = mine;
+      }
 #pragma unroll
       for (int k = 0; k < 6; k++) acc_lds[k][lane] = 0.0;
     }
+    wave_sync();
+    const auto centre_of = [&](int t) {
+      if constexpr (SURR)
+        return make_float4(__shfl(mine.x, t, 64), __shfl(mine.y, t, 64), __shfl(mine.z, t, 64),
+                           0.0f);
+      else
+        return tgt_lds[t];
+    };
+    // A place in the tile, to pick the axis that rays from a node run along.
+    const float4 far = centre_of(63);
+    const auto target_cell = [&](int t) {
+      const int jx = tx * TX + (t >> (by + bz)), jy = ty * TY + ((t >> bz) & (TY - 1)),
+                jz = tz * TZ + (t & (TZ - 1));
+      return (int64_t)jz + (int64_t)g.nz * ((int64_t)jy + (int64_t)g.ny * jx);
+    };
     int p = valid ? 0 : tr.nnode;
     int seq = 0;
     for (;;) {
@@ -820,20 +883,44 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY_FOR(SURR) void fused_step_kerne
       const NodeLink ln = tr.link[u];
       const bool here = (p == u);
       // setup_light_ray_to (setup_light_ray_tree.c:346-354), FP32
-      const float ddx = tgt.x - cx, ddy = tgt.y - cy, ddz = tgt.z - cz;
+      const float4 own = SURR ? mine : tgt_lds[lane];
+      const float ddx = own.x - cx, ddy = own.y - cy, ddz = own.z - cz;
       const float r2 = ddx * ddx + ddy * ddy + ddz * ddz;
       const bool accept = r2 * g.theta_sq > len2;
       const bool leaf = ln.n <= 1;
       const bool emit = here && (accept || ln.n == 1);
       if (here) p = (accept || leaf || ln.first < 0) ? ln.skip : ln.first;
       my_visit++;
-      my_emit_iter += __ballot(emit) != 0 ? 1ull : 0ull;
+      const unsigned long long emitting = __ballot(emit);
+      if (emitting == 0) continue;
+      my_emit_iter++;
+      // Which target's ray each lane works: targets that follow one another
+      // along the axis the rays run along mostly (from the node to the tile)
+      // go to neighbouring lanes.  Their rays share most of their cells, and
+      // the vector memory path serves a 12-B gather four neighbouring lanes at
+      // a time, a cycle for each cache line the four touch: 26 lines for the
+      // 16 groups instead of 31 with lanes in mesh order (rays from random
+      // sources on 256^3; 13% fewer cache accesses counted on 4096 clumped
+      // ones, 1.5% of the time: issue bounds the kernel as much).  Bricks of
+      // 2 x 2 x 2 cells would touch 24, but their alternating strides cost
+      // registers, and what they spilled cost 30%.
+      const float ax = fabsf(far.x - cx), ay = fabsf(far.y - cy), az = fabsf(far.z - cz);
+      int t = lane;
+      if (ax > ay && ax > az)
+        t = ((lane & (TX - 1)) << (by + bz)) | (lane >> bx);
+      else if (ay > az)
+        t = ((lane >> (by + bz)) << (by + bz)) | ((lane & (TY - 1)) << bz) |
+            ((lane >> by) & (TZ - 1));
+      const bool work = (emitting >> t) & 1ull;
+      const bool node = (__ballot(accept) >> t) & 1ull;   // the ray comes from the node's centre
+      const float4 tc = centre_of(t);
+      const Vec3f tgt{tc.x, tc.y, tc.z};
       Vec3f src{0.0f, 0.0f, 0.0f}, st{0.0f, 0.0f, 0.0f};
       WalkOut w{};
       RayRate rr{};
       double res[6] = {0, 0, 0, 0, 0, 0};
-      if (emit) {
-        if (accept) {
+      if (work) {
+        if (node) {
           src = Vec3f{cx, cy, cz};
         } else {
           src = Vec3f{tr.src_pos[4 * ln.src + 0], tr.src_pos[4 * ln.src + 1],
@@ -842,16 +929,22 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY_FOR(SURR) void fused_step_kerne
         // a ray the reference refuses (calc_ray_segment.c:212) is counted
         // where it happens, on the path of sources outside the box
         segment_start(g, src, tgt, &st, &a.ctr->noverflow);
-        walk_segment<KAHAN, CAPTURE, NARROW, POW2>(g, a.nf, st, tgt, &w);
+        const RayDir dir = ray_dir(tgt.x - src.x, tgt.y - src.y, tgt.z - src.z);
+        RayDir along = dir;   // from the segment's start: the source, if inside the box
+        if (st.x != src.x || st.y != src.y || st.z != src.z)
+          along = ray_dir(tgt.x - st.x, tgt.y - st.y, tgt.z - st.z);
+        walk_segment<KAHAN, CAPTURE, NARROW, POW2, FLOAT>(g, a.nf, along, st, tgt, &w);
         float4 f;
-        if constexpr (SURR)
-          f = make_float4(*mesh_f(a.mesh, cell, kOffDens), *mesh_f(a.mesh, cell, kOffFHI),
-                          *mesh_f(a.mesh, cell, kOffFHeI), *mesh_f(a.mesh, cell, kOffFHeII));
-        else
-          f = cell_lds[lane];
-        ray_rate_setup(g, rt, w.tau, src, tgt, f.x, f.y, f.z, f.w, &rr);
+        if constexpr (SURR) {
+          const int64_t tcell = target_cell(t);
+          f = make_float4(*mesh_f(a.mesh, tcell, kOffDens), *mesh_f(a.mesh, tcell, kOffFHI),
+                          *mesh_f(a.mesh, tcell, kOffFHeI), *mesh_f(a.mesh, tcell, kOffFHeII));
+        } else {
+          f = cell_lds[t];
+        }
+        ray_rate_setup(g, dir, w.tau, src, tgt, f.x, f.y, f.z, f.w, &rr);
       }
-      bool exact = emit;
+      bool exact = work;
       if constexpr (SURR) {
         // The network runs on the whole wavefront (MFMA) and serves the
         // visit only when every emitting lane can use it; otherwise every
@@ -860,9 +953,8 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY_FOR(SURR) void fused_step_kerne
         // visit that ran both would cost twice as much.
         const double qn = a.surr.node_q[u];
         float xa[3] = {0.0f, 0.0f, 0.0f}, xb[3] = {0.0f, 0.0f, 0.0f};
-        const bool use = emit && surr_inputs(a.surr, rt, rr, qn, xa, xb);
-        const unsigned long long emitting = __ballot(emit);
-        if (emitting != 0 && __ballot(use) == emitting) {
+        const bool use = work && surr_inputs(a.surr, rt, rr, qn, xa, xb);
+        if (__ballot(use) == __ballot(work)) {
           float ya[kNout], yb[kNout];
           mlp_forward(a.surr.net, xa[0], xa[1], xa[2], ya, lds);
           mlp_forward(a.surr.net, xb[0], xb[1], xb[2], yb, lds);
@@ -885,19 +977,20 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY_FOR(SURR) void fused_step_kerne
       // sums; this loop serves the rays FP32 cannot)
       rate_f64_wave(rt, rr, wide, [&](int, int k) { return (double)sp[k] * sc; }, res);
       if (wide) my_fb++;
-      if (emit) {
+      const int nth = CAPTURE ? __shfl(seq, t, 64) : 0;
+      if (work) {
 #pragma unroll
-        for (int k = 0; k < 6; k++) acc_lds[k][lane] += res[k];
+        for (int k = 0; k < 6; k++) acc_lds[k][t] += res[k];
         my_ray++;
         my_cross += (unsigned int)w.ncross;
         if (CAPTURE) {
           const unsigned long long slot = atomicAdd(&a.ctr->nrecord, 1ull);
           if (slot < (unsigned long long)a.rec_cap) {
             RayRecord& R = a.rec[slot];
-            R.target = cell;
-            R.seq = seq;
-            R.kind = accept ? 0 : 1;
-            R.id = accept ? u : ln.src;
+            R.target = target_cell(t);
+            R.seq = nth;
+            R.kind = node ? 0 : 1;
+            R.id = node ? u : ln.src;
             R.ncross = w.ncross;
             R.start[0] = st.x; R.start[1] = st.y; R.start[2] = st.z;
             R.src[0] = src.x; R.src[1] = src.y; R.src[2] = src.z;
@@ -907,8 +1000,9 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY_FOR(SURR) void fused_step_kerne
             for (int k = 0; k < 6; k++) R.rate[k] = res[k];
           }
         }
-        seq++;
       }
+      if (CAPTURE && emit) seq++;
+      wave_sync();   // the sums of this visit before another lane's
     }
     if (valid) {
       float* r = mesh_fw(a.mesh, cell, kOffRates);
@@ -1061,33 +1155,57 @@ static bool pow2_cells(const GridDev& g) {
   return true;
 }
 
-template <typename Fields>
-static void launch_walk(const GridDev& g, const Fields& f, void* seg, int64_t nseg, int kahan,
-                        bool pow2, hipStream_t s) {
-  if (pow2)
-    walk_segments_kernel<true><<<nblocks(nseg, kWalkBlock), kWalkBlock, 0, s>>>(
-        g, f, static_cast<unsigned char*>(seg), nseg, kahan);
-  else
-    walk_segments_kernel<false><<<nblocks(nseg, kWalkBlock), kWalkBlock, 0, s>>>(
-        g, f, static_cast<unsigned char*>(seg), nseg, kahan);
+// How the walk takes a mesh: its float form up to 2^24 cells (byte offsets of
+// 16-B records are exact in FP32 up to there) where the cell sizes leave its
+// FP32 quotients room, 32-bit offsets below 2^28 cells, and 64-bit addresses
+// and face counters otherwise (and always when wide is set).
+enum class WalkForm { kFloat, kNarrow, kWide };
+static WalkForm walk_form(const GridDev& g, int wide) {
+  const int64_t ncell = (int64_t)g.nx * g.ny * g.nz;
+  if (wide || ncell >= kNarrowCells) return WalkForm::kWide;
+  for (float h : {g.dx, g.dy, g.dz})
+    if (!(h > 1.0e-12f && h < 1.0e6f)) return WalkForm::kNarrow;
+  return ncell <= kFloatCells ? WalkForm::kFloat : WalkForm::kNarrow;
+}
+
+template <typename Walk>
+static void launch_walk(const GridDev& g, const Walk& w, void* seg, int64_t nseg, int kahan,
+                        hipStream_t s) {
+  walk_segments_kernel<<<nblocks(nseg, kWalkBlock), kWalkBlock, 0, s>>>(
+      g, w, static_cast<unsigned char*>(seg), nseg, kahan);
 }
 
 hipError_t launch_walk_segments(const GridDev& g, const float4* nf, void* seg, int64_t nseg,
                                 int kahan, int wide, hipStream_t s) {
   if (nseg <= 0) return hipSuccess;
-  if (!wide && (int64_t)g.nx * g.ny * g.nz < kNarrowCells)
-    launch_walk(g, PackedFields<true>{nf, (uint32_t)(g.nx * g.nyz * 16)}, seg, nseg, kahan,
-                pow2_cells(g), s);
-  else
-    launch_walk(g, PackedFields<false>{nf, 0u}, seg, nseg, kahan, false, s);
+  const bool pow2 = pow2_cells(g);
+  switch (walk_form(g, wide)) {
+    case WalkForm::kFloat:
+      if (pow2)
+        launch_walk(g, WalkPacked<true, true, true>{nf}, seg, nseg, kahan, s);
+      else
+        launch_walk(g, WalkPacked<true, false, true>{nf}, seg, nseg, kahan, s);
+      break;
+    case WalkForm::kNarrow:
+      if (pow2)
+        launch_walk(g, WalkPacked<true, true, false>{nf}, seg, nseg, kahan, s);
+      else
+        launch_walk(g, WalkPacked<true, false, false>{nf}, seg, nseg, kahan, s);
+      break;
+    case WalkForm::kWide:
+      launch_walk(g, WalkPacked<false, false, false>{nf}, seg, nseg, kahan, s);
+  }
   return hipGetLastError();
 }
 
 hipError_t launch_walk_segments_mesh(const GridDev& g, const void* mesh, double helium_fact,
                                      void* seg, int64_t nseg, int kahan, hipStream_t s) {
   if (nseg <= 0) return hipSuccess;
-  launch_walk(g, MeshFields{static_cast<const unsigned char*>(mesh), helium_fact}, seg, nseg,
-              kahan, pow2_cells(g), s);
+  const MeshFields f{static_cast<const unsigned char*>(mesh), helium_fact};
+  if (pow2_cells(g))
+    launch_walk(g, WalkMesh<true>{f}, seg, nseg, kahan, s);
+  else
+    launch_walk(g, WalkMesh<false>{f}, seg, nseg, kahan, s);
   return hipGetLastError();
 }
 
@@ -1133,34 +1251,41 @@ hipError_t launch_reset_counters(StepCounters* ctr, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <bool SURR, bool NARROW, bool POW2>
+template <bool SURR, bool NARROW, bool POW2, bool FLOAT>
 static void launch_fused(const FusedArgs& a, int kahan, int capture, int nblock, hipStream_t s) {
   if (capture) {
     if (kahan)
-      fused_step_kernel<true, true, SURR, NARROW, POW2><<<nblock, 64, 0, s>>>(a);
+      fused_step_kernel<true, true, SURR, NARROW, POW2, FLOAT><<<nblock, 64, 0, s>>>(a);
     else
-      fused_step_kernel<false, true, SURR, NARROW, POW2><<<nblock, 64, 0, s>>>(a);
+      fused_step_kernel<false, true, SURR, NARROW, POW2, FLOAT><<<nblock, 64, 0, s>>>(a);
   } else {
     if (kahan)
-      fused_step_kernel<true, false, SURR, NARROW, POW2><<<nblock, 64, 0, s>>>(a);
+      fused_step_kernel<true, false, SURR, NARROW, POW2, FLOAT><<<nblock, 64, 0, s>>>(a);
     else
-      fused_step_kernel<false, false, SURR, NARROW, POW2><<<nblock, 64, 0, s>>>(a);
+      fused_step_kernel<false, false, SURR, NARROW, POW2, FLOAT><<<nblock, 64, 0, s>>>(a);
   }
 }
 
-// Cell-field addressing and face arithmetic: 32-bit offsets on meshes of
-// fewer than 2^28 cells, with face positions where the cell sizes allow;
-// otherwise (and always when wide is set) 64-bit addresses and face counters.
 template <bool SURR>
 static void launch_fused_form(const FusedArgs& a, int kahan, int capture, int wide, int nblock,
                               hipStream_t s) {
-  const bool narrow = !wide && (int64_t)a.grid.nx * a.grid.ny * a.grid.nz < kNarrowCells;
-  if (narrow && pow2_cells(a.grid))
-    launch_fused<SURR, true, true>(a, kahan, capture, nblock, s);
-  else if (narrow)
-    launch_fused<SURR, true, false>(a, kahan, capture, nblock, s);
-  else
-    launch_fused<SURR, false, false>(a, kahan, capture, nblock, s);
+  const bool pow2 = pow2_cells(a.grid);
+  switch (walk_form(a.grid, wide)) {
+    case WalkForm::kFloat:
+      if (pow2)
+        launch_fused<SURR, true, true, true>(a, kahan, capture, nblock, s);
+      else
+        launch_fused<SURR, true, false, true>(a, kahan, capture, nblock, s);
+      break;
+    case WalkForm::kNarrow:
+      if (pow2)
+        launch_fused<SURR, true, true, false>(a, kahan, capture, nblock, s);
+      else
+        launch_fused<SURR, true, false, false>(a, kahan, capture, nblock, s);
+      break;
+    case WalkForm::kWide:
+      launch_fused<SURR, false, false, false>(a, kahan, capture, nblock, s);
+  }
 }
 
 // nblock: the persistent grid; a mesh of fewer tiles gets a block per tile

@@ -282,6 +282,9 @@ GridDev make_grid(const run_param* r) {
   d.dx = r->delta_x;
   d.dy = r->delta_y;
   d.dz = r->delta_z;
+  d.rdx = 1.0f / d.dx;
+  d.rdy = 1.0f / d.dy;
+  d.rdz = 1.0f / d.dz;
   d.lunit = r->lunit;
   d.denstonh = r->denstonh;
   d.helium_fact = g_helium_fact;
@@ -1725,6 +1728,11 @@ int argot_hip_segment_start(const struct run_param* r, const float* src, int ix,
   start[1] = st.y;
   start[2] = st.z;
   return n;
+}
+
+// The walk's quotients a[i]/b[i] (div_exact), on the host.
+void argot_hip_quotients(const float* a, const float* b, float* q, int64_t n) {
+  for (int64_t i = 0; i < n; i++) q[i] = div_exact(a[i], b[i], 1.0f / b[i]);
 }
 
 // The quadrature rule of run_param's tables on the host: cross-sections
