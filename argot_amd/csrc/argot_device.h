@@ -739,23 +739,34 @@ struct RayRate {
   double v[3];    // n_s V_sh + TINY
 };
 
-// dir: ray_dir of tgt - src.
-__device__ inline void ray_rate_setup(const GridDev& g, const RayDir& dir, const float tau[3],
-                                      Vec3f src, Vec3f tgt, float dens, float fHI, float fHeI,
-                                      float fHeII, RayRate* rr) {
+// The ray's chord through a cell and its length (delta_length and the
+// distance, calc_photoion_rate.c:52-90,163-170).  dir: ray_dir of d = target
+// - source.
+struct Chord {
+  float delta, dist;
+};
+__device__ inline Chord ray_chord(const GridDev& g, const RayDir& dir, float dx, float dy,
+                                  float dz) {
+  Chord c;
+  c.delta = fminf(fabsf(div_exact(g.dx, dir.xo, dir.hx)),
+                  fminf(fabsf(div_exact(g.dy, dir.yo, dir.hy)),
+                        fabsf(div_exact(g.dz, dir.zo, dir.hz))));
+  c.dist = dir.dist;
+  if (!dir.plain) {
+    c.delta = delta_length(g, dx, dy, dz);
+    c.dist = (float)__builtin_sqrt((double)(dx * dx + dy * dy + dz * dz));
+  }
+  return c;
+}
+
+__device__ inline void ray_rate_setup(const GridDev& g, const Chord& c, const float tau[3],
+                                      float dens, float fHI, float fHeI, float fHeII,
+                                      RayRate* rr) {
   const double col = g.lunit * g.denstonh;
   rr->t[0] = (double)tau[0] * col;
   rr->t[1] = (double)tau[1] * col;
   rr->t[2] = (double)tau[2] * col;
-  float delta = fminf(fabsf(div_exact(g.dx, dir.xo, dir.hx)),
-                      fminf(fabsf(div_exact(g.dy, dir.yo, dir.hy)),
-                            fabsf(div_exact(g.dz, dir.zo, dir.hz))));
-  float dist = dir.dist;
-  if (!dir.plain) {
-    const float dx = tgt.x - src.x, dy = tgt.y - src.y, dz = tgt.z - src.z;
-    delta = delta_length(g, dx, dy, dz);
-    dist = (float)__builtin_sqrt((double)(dx * dx + dy * dy + dz * dz));
-  }
+  const float delta = c.delta, dist = c.dist;
   const double nH = (double)dens * g.denstonh;
   const double nHI = nH * (double)fHI;
   rr->d[0] = nHI * (double)delta * g.lunit;

@@ -599,20 +599,18 @@ __device__ __forceinline__ T wave_sum(T v) {
   return v;
 }
 
-// ARGOT_WAVES_PER_EU (build option, 6 by default) caps the register budget
-// of the exact-rate fused kernels so that this many wavefronts fit per SIMD:
-// their walks wait on gathers, and more wavefronts hide more of that wait
-// than the spilled registers cost (on 256^3 / 4096 sources, 140 ms at 6
-// against 143 ms at 5, 148 ms at 4 and 149 ms at 8).  The surrogate variant,
-// whose LDS holds about 4 wavefronts per SIMD, and the per-call rate kernel,
-// which does not walk, keep the budget of 4.
+// ARGOT_WAVES_PER_EU (build option, 4 by default) caps the register budget of
+// the fused and the per-call rate kernels so that this many wavefronts fit per
+// SIMD.  Their issue and the gathers' cache lines bound them, so registers
+// (spills are instructions) count for more than wavefronts: on 256^3 cells and
+// 4096 sources 3, 4, 5 and 6 wavefronts take 84, 81, 87 and 90 ms, on 128^3 and
+// 1024 with Kahan sums 27.0, 28.0, 30.6 and 32.1, on 72 x 58 x 87 and 250 4.2, 4.3,
+// 4.8 and 5.3 (each with the grid that fills it).
 #if defined(ARGOT_WAVES_PER_EU) && ARGOT_WAVES_PER_EU > 0
-#define ARGOT_OCCUPANCY_FOR(SURR) \
-  __attribute__((amdgpu_waves_per_eu((SURR) ? 4 : ARGOT_WAVES_PER_EU)))
+#define ARGOT_OCCUPANCY __attribute__((amdgpu_waves_per_eu(ARGOT_WAVES_PER_EU)))
 #else
-#define ARGOT_OCCUPANCY_FOR(SURR)
+#define ARGOT_OCCUPANCY
 #endif
-#define ARGOT_CALL_OCCUPANCY __attribute__((amdgpu_waves_per_eu(4)))
 
 // calc_photoion_rate_cuda (calc_photoion_rate_cuda.cu:92-216 with the
 // per-target merge of calc_photoion_rate.c:403-425): one lane per target
@@ -624,7 +622,7 @@ __device__ __forceinline__ T wave_sum(T v) {
 // its next ray at each pass, whichever spectra the wavefront's rays have.
 // Each ray's arithmetic is the fused kernel's, so a ray list taken from the
 // fused step gives its bits.
-__global__ __launch_bounds__(64) ARGOT_CALL_OCCUPANCY void target_rates_kernel(
+__global__ __launch_bounds__(64) ARGOT_OCCUPANCY void target_rates_kernel(
     GridDev g, RateTables rt, unsigned char* __restrict__ mesh, const CallTarget* __restrict__ tg,
     int64_t ntarget, const CallRay* __restrict__ rays, CallSpectra sp) {
   const int lane = threadIdx.x;
@@ -649,27 +647,28 @@ __global__ __launch_bounds__(64) ARGOT_CALL_OCCUPANCY void target_rates_kernel(
     const bool more = r < rend;
     bool wide = false;   // FP32 cannot serve this ray
     int u = 0;
-    RayRate rr{};
-    double res[6] = {0, 0, 0, 0, 0, 0};
+    RayRate rr;
+    double res[6];
     if (more) {
       const CallRay R = rays[r];
       u = R.spec;
       const Vec3f src{R.src[0], R.src[1], R.src[2]};
-      const RayDir dir = ray_dir(tgt.x - src.x, tgt.y - src.y, tgt.z - src.z);
-      ray_rate_setup(g, dir, R.tau, src, tgt, dens, fHI, fHeI, fHeII, &rr);
+      const Vec3f d{tgt.x - src.x, tgt.y - src.y, tgt.z - src.z};
+      const Chord chord = ray_chord(g, ray_dir(d.x, d.y, d.z), d.x, d.y, d.z);
+      ray_rate_setup(g, chord, R.tau, dens, fHI, fHeI, fHeII, &rr);
       wide = !fast_rate_ok(rt, rr);
-      if (!wide) {
-        const float* s32 = sp.spec32 + (int64_t)u * ng;
-        const F4* w = reinterpret_cast<const F4*>(sp.weight + (int64_t)u * kRuleWeights);
-        rate_loop_f32(rt, rr, sp.scale[u], sp.limit[u], [&](int k) { return s32[k]; },
-                      [&](int i) { return w[i]; }, res);
-      }
     }
     rate_f64_wave(rt, rr, wide,
                   [&](int owner, int k) {
                     return sp.spec64[(int64_t)__shfl(u, owner, 64) * ng + k];
                   },
                   res);
+    if (more && !wide) {
+      const float* s32 = sp.spec32 + (int64_t)u * ng;
+      const F4* w = reinterpret_cast<const F4*>(sp.weight + (int64_t)u * kRuleWeights);
+      rate_loop_f32(rt, rr, sp.scale[u], sp.limit[u], [&](int k) { return s32[k]; },
+                    [&](int i) { return w[i]; }, res);
+    }
     if (more) {
 #pragma unroll
       for (int k = 0; k < 6; k++) acc[k] += res[k];
@@ -778,7 +777,7 @@ __device__ inline void surr_rates(const RayRate& rr, double q, const float ya[kN
 }
 
 template <bool KAHAN, bool CAPTURE, bool SURR, bool NARROW, bool POW2, bool FLOAT>
-__global__ __launch_bounds__(64) ARGOT_OCCUPANCY_FOR(SURR) void fused_step_kernel(FusedArgs a) {
+__global__ __launch_bounds__(64) ARGOT_OCCUPANCY void fused_step_kernel(FusedArgs a) {
   const GridDev& g = a.grid;
   const TreeDev& tr = a.tree;
   const RateTables& rt = a.rates;
@@ -917,8 +916,8 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY_FOR(SURR) void fused_step_kerne
       const Vec3f tgt{tc.x, tc.y, tc.z};
       Vec3f src{0.0f, 0.0f, 0.0f}, st{0.0f, 0.0f, 0.0f};
       WalkOut w{};
-      RayRate rr{};
-      double res[6] = {0, 0, 0, 0, 0, 0};
+      RayRate rr;      // (of working lanes; no other lane's is used)
+      double res[6];
       if (work) {
         if (node) {
           src = Vec3f{cx, cy, cz};
@@ -929,8 +928,11 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY_FOR(SURR) void fused_step_kerne
         // a ray the reference refuses (calc_ray_segment.c:212) is counted
         // where it happens, on the path of sources outside the box
         segment_start(g, src, tgt, &st, &a.ctr->noverflow);
-        const RayDir dir = ray_dir(tgt.x - src.x, tgt.y - src.y, tgt.z - src.z);
-        RayDir along = dir;   // from the segment's start: the source, if inside the box
+        const Vec3f d{tgt.x - src.x, tgt.y - src.y, tgt.z - src.z};
+        RayDir along = ray_dir(d.x, d.y, d.z);
+        // (formed here, so that two numbers are kept through the walk)
+        const Chord chord = ray_chord(g, along, d.x, d.y, d.z);
+        // from the segment's start: the source, if inside the box
         if (st.x != src.x || st.y != src.y || st.z != src.z)
           along = ray_dir(tgt.x - st.x, tgt.y - st.y, tgt.z - st.z);
         walk_segment<KAHAN, CAPTURE, NARROW, POW2, FLOAT>(g, a.nf, along, st, tgt, &w);
@@ -942,7 +944,7 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY_FOR(SURR) void fused_step_kerne
         } else {
           f = cell_lds[t];
         }
-        ray_rate_setup(g, dir, w.tau, src, tgt, f.x, f.y, f.z, f.w, &rr);
+        ray_rate_setup(g, chord, w.tau, f.x, f.y, f.z, f.w, &rr);
       }
       bool exact = work;
       if constexpr (SURR) {
@@ -968,15 +970,16 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY_FOR(SURR) void fused_step_kerne
       const float* sp = tr.spec + (int64_t)u * rt.ngrid;
       const double sc = ldc(tr.spec_scale + u);
       const bool wide = exact && !fast_rate_ok(rt, rr);   // FP32 cannot serve this ray
+      // the node spectrum as spec * spec_scale (within 6e-8 of the double
+      // sums; this loop serves the rays FP32 cannot).  It comes first, so that
+      // the ray's FP64 quantities need not outlive the FP32 loop.
+      rate_f64_wave(rt, rr, wide, [&](int, int k) { return (double)sp[k] * sc; }, res);
+      if (wide) my_fb++;
       if (exact && !wide) {
         const F4* wt = reinterpret_cast<const F4*>(tr.weight + (int64_t)u * kRuleWeights);
         rate_loop_f32(rt, rr, sc, ldc(tr.limit + u), [&](int k) { return ldc(sp + k); },
                       [&](int i) { return ldc(wt + i); }, res);
       }
-      // the node spectrum as spec * spec_scale (within 6e-8 of the double
-      // sums; this loop serves the rays FP32 cannot)
-      rate_f64_wave(rt, rr, wide, [&](int, int k) { return (double)sp[k] * sc; }, res);
-      if (wide) my_fb++;
       const int nth = CAPTURE ? __shfl(seq, t, 64) : 0;
       if (work) {
 #pragma unroll
