@@ -143,6 +143,8 @@ struct ChemCounters {
   unsigned long long niter;
   unsigned long long next;   // cell queue of the persistent chemistry kernel
   unsigned long long nstopped;   // cells ended by the NaN or sub-step guard
+  unsigned int npaused;      // cells handed on to the row kernel (beyond its list: none)
+  unsigned int next_paused;  // its queue
 };
 
 }  // namespace argot

@@ -84,129 +84,272 @@ struct KSet {
   float k1, k2, k3, k4, k5, k6;
 };
 
-// k01, k03, k05 (collisional ionization), reaction_rate.cu:33-62,108-136,
-// 167-192; k02, k06 (case-B recombination, Hui & Gnedin 1997), :98-103,
-// 200-203; k04, :152-164.
+// A cell's arithmetic is done by one lane, or by the 16 lanes of a DPP row
+// together: a cell beside a source takes thousands of sub-steps one after the
+// other, and when only such cells are left, what counts is how long one
+// sub-step takes.  The fits are then spread over the row, a fit or a term of
+// the cooling sum per lane, and everything else is done by all 16 lanes alike.
+// Both ways form each term with the same operations and add the terms in the
+// same tree, so a cell's result does not depend on which it went through.
+
+// Sum over the row, in every lane: ((t0 + t1) + (t2 + t3)) + ... as tree_sum.
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+  union { double d; int i[2]; } a, b;
+  a.d = v;
+  b.i[0] = __builtin_amdgcn_mov_dpp(a.i[0], CTRL, 0xf, 0xf, true);
+  b.i[1] = __builtin_amdgcn_mov_dpp(a.i[1], CTRL, 0xf, 0xf, true);
+  return v + b.d;
+}
+__device__ __forceinline__ double row_sum(double v) {
+  v = dpp_add<0xb1>(v);    // quad_perm [1,0,3,2]
+  v = dpp_add<0x4e>(v);    // quad_perm [2,3,0,1]
+  v = dpp_add<0x141>(v);   // row_half_mirror: the other quad of the half row
+  return dpp_add<0x140>(v);   // row_mirror: the other half
+}
+__device__ __forceinline__ double tree_sum(const double (&t)[16]) {
+  const double a = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+  const double b = ((t[8] + t[9]) + (t[10] + t[11])) + ((t[12] + t[13]) + (t[14] + t[15]));
+  return a + b;
+}
+// Value of lane `from` of each row, in all its lanes.
+template <int FROM>
+__device__ __forceinline__ float row_pick(float v) {
+  return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x10 | (FROM << 5)));
+}
+
+constexpr double kLnKtoEV = -9.359277830950614;   // ln(K_to_eV)
+constexpr double kLnB274 = 1.0079579203999789;    // ln(2.740)
+constexpr double kLnLamHeII = 13.254566388120152;
+constexpr double kX6 = 1.7584044112379005;        // (631515/157807)^0.407
+constexpr double kLog10e = 0.43429448190325182765;
+
+// Fits of k01, k03, k05 (collisional ionization), reaction_rate.cu:33-62,
+// 108-136, 167-192, by powers of ln(T in eV).
+constexpr double kIon1[9] = {-32.71396786375,      13.53655609057,     -5.739328757388,
+                             1.563154982022,       -0.2877056004391,   0.03482559773736999,
+                             -0.00263197617559,    0.0001119543953861, -2.039149852002e-6};
+constexpr double kIon3[9] = {-44.09864886561001, 23.91596563469,      -10.75323019821,
+                             3.058038757198,     -0.5685118909884001, 0.06795391233790001,
+                             -0.005009056101857001, 0.0002067236157507, -3.649161410833e-6};
+constexpr double kIon5[9] = {-68.71040990212001, 43.93347632635,      -18.48066993568,
+                             4.701626486759002,  -0.7692466334492,    0.08113042097303,
+                             -0.005324020628287001, 0.0001975705312221, -3.165581065665e-6};
+
+// k02, k06 (case-B recombination, Hui & Gnedin 1997), :98-103,200-203; k04,
+// :152-164.
 __device__ inline KSet rate_coefficients(float T) {
-  constexpr double c1[9] = {-32.71396786375,      13.53655609057,     -5.739328757388,
-                            1.563154982022,       -0.2877056004391,   0.03482559773736999,
-                            -0.00263197617559,    0.0001119543953861, -2.039149852002e-6};
-  constexpr double c3[9] = {-44.09864886561001, 23.91596563469,      -10.75323019821,
-                            3.058038757198,     -0.5685118909884001, 0.06795391233790001,
-                            -0.005009056101857001, 0.0002067236157507, -3.649161410833e-6};
-  constexpr double c5[9] = {-68.71040990212001, 43.93347632635,      -18.48066993568,
-                            4.701626486759002,  -0.7692466334492,    0.08113042097303,
-                            -0.005324020628287001, 0.0001975705312221, -3.165581065665e-6};
-  // ln(K_to_eV), ln(2.740)
-  constexpr double kLnKtoEV = -9.359277830950614, kLnB = 1.007957920399979;
   const double t = (double)T;
   const double tev = t * kKtoEV;
   const double L = log(tev);
   KSet K;
-  K.k1 = (float)exp(poly_left(c1, L));
+  K.k1 = (float)exp(poly_left(kIon1, L));
   K.k3 = 0.0f;
   K.k5 = 0.0f;
   if (tev > 0.8) {
-    K.k3 = (float)exp(poly_left(c3, L));
-    K.k5 = (float)exp(poly_left(c5, L));
+    K.k3 = (float)exp(poly_left(kIon3, L));
+    K.k5 = (float)exp(poly_left(kIon5, L));
   }
   const double l2 = (kLnLamHII + kLnKtoEV) - L;     // ln lam_HII
   const double l6 = (kLnLamHeIII + kLnKtoEV) - L;   // ln lam_HeIII
-  const double x2 = exp(0.407 * (l2 - kLnB));
-  constexpr double kX6 = 1.7584044112379005;        // (631515/157807)^0.407
+  const double x2 = exp(0.407 * (l2 - kLnB274));
   const double x6 = x2 * kX6;
   K.k2 = (float)(2.753e-14 * exp(1.5 * l2 - 2.242 * log(1.0 + x2)));
   K.k6 = (float)(1.3765e-14 * exp(1.5 * l6 - 2.242 * log(1.0 + x6)));
-  if (t > 500.3) {
-    constexpr double kLnLamHeII = 13.254566388120152;
+  if (t > 500.3)
     K.k4 = (float)(1.26e-14 * exp(0.75 * ((kLnLamHeII + kLnKtoEV) - L)));
-  } else {
-    constexpr double kLog10e = 0.43429448190325182765;
+  else
     K.k4 = (float)((1.12e-10 - 2.1e-11 * ((L - kLnKtoEV) * kLog10e)) / sqrt(t));
-  }
   return K;
 }
 
 // ------------------------------------------------------------- cooling ---
 
-// What heat - cool of one cell depends on besides the temperature, formed
-// once per energy update.
-struct CoolTerms {
-  double heat;                          // photoheating [erg cm^-3 s^-1]
-  double hii, heii, heiii, hi, hei;     // ion densities times n_e
-  double ions;                          // (n_HII + n_HeII + n_HeIII) n_e
-  double ne;
-  double compt, tcmb;                   // Compton: compt * (T - tcmb) * n_e
-  double scale;                         // to code units: convfact / dens
+// Terms of the cooling sum, each w * exp(p ln T + q 1e5/T + r z) with w the
+// densities times a constant (times 1/(1 + sqrt(T/1e5)) for 5 to 10), and
+// z = ln(1 + x) for the two Hui & Gnedin fits, (5.5 - log10 T)^2 for the Gaunt
+// factor: calc_heatcool_rate_dev (heatcool_rate.cu:10-74) with
+// cooling_rate.cu's case-B functions.
+//   0 creh2, 1 crehe3, 2 crehe2 (two branches at 980 K), 3 and 4 crexihe2,
+//   5 cioh1, 6 ciohe1, 7 ciohe2, 8 cexh1, 9 cexhe1, 10 cexhe2,
+//   11 and 12 bremsstrahlung (constant part and Gaunt factor)
+constexpr int kTerms = 13;
+constexpr double kTermP[kTerms] = {-0.97, -0.97, 0.15, -1.5, -1.5, 0.5, 0.5,
+                                   0.5,   0.0,   -0.1687, -0.397, 0.5, 0.5};
+constexpr double kTermQ[kTerms] = {0.0,       0.0,      0.0,      -4.7,     -5.64, -1.578091, -2.853354,
+                                   -6.31515, -1.18348, -0.13179, -4.73638, 0.0,   0.0};
+constexpr double kColdP = 0.35;              // term 2 below 980 K
+constexpr double kColdW = 1.7e-26;
+// constants of w: creh2 and crehe3 hold lam^1.97 without its temperature
+constexpr double kTermW[kTerms] = {
+    3.435e-30 * 68129912473.377426, 3.435e-30 * 1046610102391.0461,
+    1.9e-25 * 0.35481338923357547, 1.24e-13, 1.24e-13 * 0.3, 1.27e-21, 9.38e-22, 4.95e-22,
+    7.5e-19, 9.1e-27, 5.54e-17, 1.42e-27 * 1.1, 1.42e-27 * 0.34};
+constexpr double kRecR = -3.72, kGauntR = -1.0 / 3.0;
+constexpr double kLnB225 = 0.8109302162163288;    // ln 2.25
+constexpr double kX3 = 1.6844137772424854;        // (631515/157807)^0.376
+
+// Constants of a lane of a row: its term of the cooling sum (lanes beyond have
+// weight 0) and its fit among two sets of rate coefficients (lanes 0 to 5: k1,
+// k2, k3, k4, k5, k6 at one temperature, 8 to 13 at another).
+struct RowLane {
+  int sub;
+  double p, pc, q, r, x;     // cooling term (pc: below 980 K)
+  double ion[9];             // collisional ionization fit
+  double lam, xk, kw;        // Hui & Gnedin fit; constant factor
 };
 
-__device__ __forceinline__ CoolTerms cool_terms(const State& c, float zred, double nH,
-                                                double helium_fact, double scale) {
-  CoolTerms k;
+__device__ inline RowLane row_lane() {
+  RowLane r;
+  r.sub = threadIdx.x & 15;
+  r.p = r.pc = r.q = r.r = r.x = 0.0;
+#pragma unroll
+  for (int i = 0; i < kTerms; i++)
+    if (r.sub == i) {
+      r.p = kTermP[i];
+      r.pc = i == 2 ? kColdP : kTermP[i];
+      r.q = kTermQ[i];
+      r.r = i < 2 ? kRecR : i == 12 ? kGauntR : 0.0;
+      r.x = i == 0 ? 1.0 : i == 1 ? kX3 : 0.0;
+    }
+  const int f = r.sub & 7;
+#pragma unroll
+  for (int i = 0; i < 9; i++) r.ion[i] = f == 0 ? kIon1[i] : f == 2 ? kIon3[i] : kIon5[i];
+  r.lam = f == 1 ? kLnLamHII + kLnKtoEV : f == 5 ? kLnLamHeIII + kLnKtoEV : kLnLamHeII + kLnKtoEV;
+  r.xk = f == 5 ? kX6 : 1.0;
+  r.kw = f == 1 ? 2.753e-14 : f == 5 ? 1.3765e-14 : f == 3 ? 1.26e-14 : 1.0;
+  return r;
+}
+
+// Rate coefficients at two temperatures, by the row.
+__device__ inline void row_coefficients(const RowLane& r, float T0, float T1, KSet* K0, KSet* K1) {
+  const int f = r.sub & 7;
+  const double t = (double)(r.sub < 8 ? T0 : T1);
+  const double tev = t * kKtoEV;
+  const double L = log(tev);
+  const double l2 = (kLnLamHII + kLnKtoEV) - L;
+  const double l = r.lam - L;
+  const double x2 = exp(0.407 * (l2 - kLnB274));
+  const bool rec = f == 1 || f == 5;
+  const double arg = rec ? 1.5 * l - 2.242 * log(1.0 + x2 * r.xk)
+                         : f == 3 ? 0.75 * l : poly_left(r.ion, L);
+  float v = (float)(r.kw * exp(arg));
+  if ((f == 2 || f == 4) && !(tev > 0.8)) v = 0.0f;
+  if (f == 3 && !(t > 500.3))
+    v = (float)((1.12e-10 - 2.1e-11 * ((L - kLnKtoEV) * kLog10e)) / sqrt(t));
+  *K0 = KSet{row_pick<0>(v), row_pick<1>(v), row_pick<2>(v),
+             row_pick<3>(v), row_pick<4>(v), row_pick<5>(v)};
+  *K1 = KSet{row_pick<8>(v), row_pick<9>(v), row_pick<10>(v),
+             row_pick<11>(v), row_pick<12>(v), row_pick<13>(v)};
+}
+
+// What heat - cool of one cell depends on besides the temperature, formed
+// once per energy update.  w: the terms' weights (a row's lane: its own), wc:
+// term 2's below 980 K.
+struct CoolCell {
+  double heat;              // photoheating [erg cm^-3 s^-1]
+  double compt, tcmb;       // Compton cooling: compt (T - tcmb)
+  double scale;             // to code units: convfact / dens
+};
+struct CoolTerms : CoolCell {
+  double w[kTerms], wc;
+};
+struct CoolRow : CoolCell {
+  const RowLane& r;
+  double w, wc;
+};
+
+__device__ __forceinline__ void cool_cell(const State& c, float zred, double nH,
+                                          double helium_fact, double scale, CoolCell* k,
+                                          double (&n)[6]) {
   const double nHe = nH * helium_fact;
   const double nHI = nH * (double)c.fHI, nHII = nH * (double)c.fHII;
   const double nHeI = nHe * (double)c.fHeI, nHeII = nHe * (double)c.fHeII;
   const double nHeIII = nHe * (double)c.fHeIII;
-  k.ne = nH * (double)c.felec;
-  k.heat = (double)c.HeatHI * nHI;
-  k.heat += (double)c.HeatHeI * nHeI + (double)c.HeatHeII * nHeII;
-  k.hi = nHI * k.ne;
-  k.hii = nHII * k.ne;
-  k.hei = nHeI * k.ne;
-  k.heii = nHeII * k.ne;
-  k.heiii = nHeIII * k.ne;
-  k.ions = k.hii + (k.heii + k.heiii);
+  const double ne = nH * (double)c.felec;
+  k->heat = (double)c.HeatHI * nHI;
+  k->heat += (double)c.HeatHeI * nHeI + (double)c.HeatHeII * nHeII;
   const double z1 = 1.0 + (double)zred;
-  k.compt = 5.406e-36 * (z1 * z1 * z1 * z1);
-  k.tcmb = 2.73 * z1;
-  k.scale = scale;
+  k->compt = 5.406e-36 * (z1 * z1 * z1 * z1) * ne;
+  k->tcmb = 2.73 * z1;
+  k->scale = scale;
+  // densities times n_e: HI, HII, HeI, HeII, HeIII, and n_HeI n_e^2 (the
+  // reference gives cexhe1 another n_e)
+  n[0] = nHI * ne;
+  n[1] = nHII * ne;
+  n[2] = nHeI * ne;
+  n[3] = nHeII * ne;
+  n[4] = nHeIII * ne;
+  n[5] = n[2] * ne;
+}
+
+__device__ __forceinline__ CoolTerms cool_terms(const State& c, float zred, double nH,
+                                                double helium_fact, double scale) {
+  CoolTerms k;
+  double n[6];
+  cool_cell(c, zred, nH, helium_fact, scale, &k, n);
+  const double ions = n[1] + (n[3] + n[4]);
+  const double d[kTerms] = {n[1], n[4], n[3], n[3], n[3], n[0], n[2],
+                            n[3], n[0], n[5], n[3], ions, ions};
+#pragma unroll
+  for (int i = 0; i < kTerms; i++) k.w[i] = kTermW[i] * d[i];
+  k.wc = kColdW * n[3];
   return k;
 }
 
-// heat - cool of one cell in code units, calc_heatcool_rate_dev
-// (heatcool_rate.cu:10-74) with cooling_rate.cu's case-B functions:
-// recombination creh2 / crehe2 / crexihe2 / crehe3, collisional ionization
-// cioh1 / ciohe1 / ciohe2 and excitation cexh1 / cexhe1 / cexhe2,
-// bremsstrahlung with its Gaunt factor, Compton cooling off the CMB.
-// cexhe1 carries another factor n_e, which the reference gives it
-// ((cexhe1 n_e n_HeI + ...) n_e).  3 logarithms and 12 exponentials.
+__device__ __forceinline__ CoolRow cool_terms(const State& c, float zred, double nH,
+                                              double helium_fact, double scale,
+                                              const RowLane& r) {
+  CoolRow k{{}, r, 0.0, 0.0};
+  double n[6];
+  cool_cell(c, zred, nH, helium_fact, scale, &k, n);
+  const double ions = n[1] + (n[3] + n[4]);
+  const double d[kTerms] = {n[1], n[4], n[3], n[3], n[3], n[0], n[2],
+                            n[3], n[0], n[5], n[3], ions, ions};
+#pragma unroll
+  for (int i = 0; i < kTerms; i++)
+    if (r.sub == i) k.w = kTermW[i] * d[i];
+  k.wc = r.sub == 2 ? kColdW * n[3] : k.w;
+  return k;
+}
+
+// heat - cool of one cell in code units.
 __device__ __forceinline__ double heatcool_rate(const CoolTerms& k, double T) {
-  constexpr double kLnB = 0.8109302162163288;    // ln 2.25
-  constexpr double kX3 = 1.6844137772424854;      // (631515/157807)^0.376
-  constexpr double kLog10e = 0.43429448190325182765;
   const double L = log(T);
-  const double it5 = 1.0e5 / T;                   // 1 / (T/1e5)
-  const double sq = sqrt(T);
-  const double sq5 = sq * 0.0031622776601683794;  // sqrt(T/1e5)
-  const double l1 = kLnLamHII - L, l3 = kLnLamHeIII - L;
-  const double x1 = exp(0.376 * (l1 - kLnB));
-  const double x3 = x1 * kX3;
-  const double a = 3.435e-30 * T;
-  const double creh2 = a * exp(1.97 * l1 - 3.72 * log(1.0 + x1));
-  const double crehe3 = a * exp(1.97 * l3 - 3.72 * log(1.0 + x3));
-  // pow(T, 0.35) and pow(T/1e3, 0.15), either side of 980 K
-  const bool cold = T < 980.0;
-  const double crehe2 = (cold ? 1.7e-26 : 1.9e-25) *
-                        exp(cold ? 0.35 * L : 0.15 * (L - 6.907755278982137));
-  // exp(-4.7/t5) as the fifth power of exp(-0.94/t5)
-  const double y = exp(-0.94 * it5);
-  const double y2 = y * y;
-  const double rsq = 1.0 / (T * sq * (1.0 + sq5));  // one division for T^-1.5 and 1/(1+sqrt(T5))
-  const double t15 = rsq * (1.0 + sq5);
-  const double r5 = rsq * (T * sq);
-  const double crexihe2 = 1.24e-13 * t15 * (y2 * y2 * y) * (1.0 + 0.3 * y);
-  const double cioh1 = exp(-1.578091 * it5), ciohe1 = exp(-2.853354 * it5);
-  const double ciohe2 = exp(-6.31515 * it5), cexh1 = exp(-1.18348 * it5);
-  const double cexhe1 = exp(-0.1687 * L - 0.13179 * it5);
-  const double cexhe2 = exp(-0.397 * L - 4.73638 * it5);
+  const double it5 = 1.0e5 / T;
+  const double r5 = 1.0 / (1.0 + sqrt(T) * 3.1622776601683794e-3);   // 1/(1 + sqrt(T/1e5))
+  const double x = exp(0.376 * ((kLnLamHII - L) - kLnB225));
   const double lg = 5.5 - L * kLog10e;
-  const double gaunt = 1.1 + 0.34 * exp(-lg * lg * (1.0 / 3.0));
-  const double brems = 1.42e-27 * gaunt * sq;
-  const double col = (k.hi * (1.27e-21 * sq * cioh1 + 7.5e-19 * cexh1) +
-                      k.hei * (9.38e-22 * sq * ciohe1 + 9.1e-27 * cexhe1 * k.ne) +
-                      k.heii * (4.95e-22 * sq * ciohe2 + 5.54e-17 * cexhe2)) * r5;
-  const double cool = creh2 * k.hii + crehe3 * k.heiii + (crehe2 + crexihe2) * k.heii + col +
-                      brems * k.ions + k.compt * (T - k.tcmb) * k.ne;
+  const bool cold = T < 980.0;
+  double t[16];
+#pragma unroll
+  for (int i = 0; i < kTerms; i++) {
+    double arg = (i == 2 && cold ? kColdP : kTermP[i]) * L;
+    if (kTermQ[i] != 0.0) arg = arg + kTermQ[i] * it5;
+    if (i < 2) arg = arg + kRecR * log(1.0 + (i == 0 ? x : x * kX3));
+    if (i == 12) arg = arg + kGauntR * (lg * lg);
+    t[i] = (i == 2 && cold ? k.wc : k.w[i]) * exp(arg);
+    if (i >= 5 && i <= 10) t[i] = t[i] * r5;
+  }
+  for (int i = kTerms; i < 16; i++) t[i] = 0.0;
+  const double cool = tree_sum(t) + k.compt * (T - k.tcmb);
+  return (k.heat - cool) * k.scale;
+}
+
+__device__ __forceinline__ double heatcool_rate(const CoolRow& k, double T) {
+  const RowLane& r = k.r;
+  const double L = log(T);
+  const double it5 = 1.0e5 / T;
+  const double r5 = 1.0 / (1.0 + sqrt(T) * 3.1622776601683794e-3);
+  const double x = exp(0.376 * ((kLnLamHII - L) - kLnB225));
+  const double lg = 5.5 - L * kLog10e;
+  const bool cold = T < 980.0;
+  // (a lane without a factor multiplies by 0 or 1: exact)
+  const double z = r.sub == 12 ? lg * lg : log(1.0 + x * r.x);
+  const double arg = ((cold ? r.pc : r.p) * L + r.q * it5) + r.r * z;
+  double t = (cold ? k.wc : k.w) * exp(arg);
+  t = t * (r.sub >= 5 && r.sub <= 10 ? r5 : 1.0);
+  const double cool = row_sum(t) + k.compt * (T - k.tcmb);
   return (k.heat - cool) * k.scale;
 }
 
@@ -230,8 +373,11 @@ __device__ __forceinline__ double heatcool_rate(const CoolTerms& k, double T) {
 // With the fits above, a 128^3 mesh over 100 kyr (8.0e6 sub-steps, the longest
 // cell's chain setting the time) took 12.4 ms instead of 100 ms, with the same
 // bits in every cell.
+//
+// row: the lane's constants when a row does the cell, nothing otherwise.
+template <typename... Row>
 __device__ inline int advance_heatcool(float dens_cell, float* uene, const State& c,
-                                       const ChemParams& p, float dtime) {
+                                       const ChemParams& p, float dtime, const Row&... row) {
   const double dens = (double)(dens_cell * p.anow3i);
   const double uene_min = (double)p.uene_min, uene_max = (double)p.uene_max;
 
@@ -244,7 +390,7 @@ __device__ inline int advance_heatcool(float dens_cell, float* uene, const State
   }
   const float wmol = (float)mean_mass_inv(c);
   const double nH = dens * p.denstonh;
-  const CoolTerms k = cool_terms(c, p.znow, nH, p.helium_fact, p.convfact / dens);
+  const auto k = cool_terms(c, p.znow, nH, p.helium_fact, p.convfact / dens, row...);
   auto temp = [&](double u) { return u * p.uenetok * (double)wmol; };
   const double dt = (double)dtime;
   const double h0 = heatcool_rate(k, temp(uene_in));
@@ -413,6 +559,52 @@ __device__ inline void cell_begin(CellRun& r, const ChemParams& p, float dtime) 
   r.elapsed = 0.0;
 }
 
+// A cell between two sub-steps: what differs from its prev_chem record and the
+// mesh, and its progress.
+struct CellPaused {
+  double dtime_safe, elapsed;
+  int cell, nsub, niter;
+  float uene;
+  float felec, fHI, fHII, fHeI, fHeII, fHeIII;
+};
+
+__device__ __forceinline__ CellPaused cell_pause(const CellRun& r, int cell) {
+  const State& c = r.c;
+  return {r.dtime_safe, r.elapsed, cell,   r.nsub,  r.niter,  r.uene,
+          c.felec,      c.fHI,     c.fHII, c.fHeI, c.fHeII, c.fHeIII};
+}
+
+// r holds the cell's dens, mesh_uene and prev_chem; continues from s (after
+// at least one sub-step: the densities and coefficients follow from the state).
+__device__ inline void cell_resume(CellRun& r, const CellPaused& s, const ChemParams& p,
+                                   float dtime) {
+  r.nsub = s.nsub;
+  r.niter = s.niter;
+  r.uene = s.uene;
+  r.c.felec = s.felec;
+  r.c.fHI = s.fHI;
+  r.c.fHII = s.fHII;
+  r.c.fHeI = s.fHeI;
+  r.c.fHeII = s.fHeII;
+  r.c.fHeIII = s.fHeIII;
+  r.dtime_p = (double)dtime * p.tunit;
+  const Dens n = number_densities(r.dens, r.c, p);
+  r.nH = n.nH;
+  r.nHe = n.nHe;
+  r.nHI = n.nHI;
+  r.nHII = n.nHII;
+  r.nHeI = n.nHeI;
+  r.nHeII = n.nHeII;
+  r.nHeIII = n.nHeIII;
+  r.ne = n.ne;
+  r.GHI = r.c.GammaHI;
+  r.GHeI = (double)r.c.GammaHeI;
+  r.GHeII = (double)r.c.GammaHeII;
+  r.K = rate_coefficients(temperature(r.uene, r.c, p));
+  r.dtime_safe = s.dtime_safe;
+  r.elapsed = s.elapsed;
+}
+
 // The reference sub-steps until the elapsed time reaches dtime.  Two
 // guards stop a cell earlier, where the reference would run for an
 // unbounded time: a state that has turned NaN (e.g. an infinite rate in a
@@ -434,7 +626,8 @@ __device__ __forceinline__ bool cell_stopped(const CellRun& r) {
   return r.elapsed < r.dtime_p;
 }
 
-__device__ inline void cell_substep(CellRun& r, const ChemParams& p) {
+template <typename... Row>
+__device__ inline void cell_substep(CellRun& r, const ChemParams& p, const Row&... row) {
   State& c = r.c;
   const KSet& K = r.K;
   if (r.elapsed + r.dtime_safe > r.dtime_p) r.dtime_safe = r.dtime_p - r.elapsed;
@@ -482,7 +675,7 @@ __device__ inline void cell_substep(CellRun& r, const ChemParams& p) {
                     (p.helium_fact * ((double)c.fHeII + 2.0 * (double)c.fHeIII) + kTiny));
 
   r.dtime_safe = dts / p.tunit;
-  r.niter += advance_heatcool(r.dens, &r.uene, c, p, (float)r.dtime_safe);
+  r.niter += advance_heatcool(r.dens, &r.uene, c, p, (float)r.dtime_safe, row...);
 
   // densities, temperature and coefficients for the next sub-step
   const Dens n = number_densities(r.dens, c, p);
@@ -493,11 +686,16 @@ __device__ inline void cell_substep(CellRun& r, const ChemParams& p) {
   r.nHeIII = n.nHeIII;
   r.ne = n.ne;
   const float T = temperature(r.uene, c, p);
-  r.K = rate_coefficients(T);
   // calc_dtime takes the temperature of the mesh's (unchanged) energy;
   // its coefficients equal K only when the two temperatures agree.
   const float Tm = temperature(r.mesh_uene, c, p);
-  const KSet Km = Tm == T ? r.K : rate_coefficients(Tm);
+  KSet Km;
+  if constexpr (sizeof...(Row) == 0) {
+    r.K = rate_coefficients(T);
+    Km = Tm == T ? r.K : rate_coefficients(Tm);
+  } else {
+    row_coefficients(row..., T, Tm, &r.K, &Km);
+  }
   r.dtime_safe = kDtFactor * (double)safe_dtime(n, c, Km);
 }
 

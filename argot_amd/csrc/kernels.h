@@ -71,9 +71,11 @@ hipError_t launch_fused_step(const FusedArgs& a, int kahan, int capture, int sur
 
 // Chemistry (chemistry.hip).  Each launch first resets *ctr on the stream.
 // queue_blocks > 0: the persistent cell-queue kernel on that many blocks;
-// 0: one cell per thread.
+// 0: one cell per thread.  paused: kPausedCells * kPausedBytes bytes.
+constexpr int kPausedCells = 16384, kPausedBytes = 56;
 hipError_t launch_chem_step(void* mesh, int64_t ncell, const ChemParams& p, float dtime,
-                            ChemCounters* ctr, int queue_blocks, int min_refill, hipStream_t s);
+                            ChemCounters* ctr, void* paused, int queue_blocks, int min_refill,
+                            hipStream_t s);
 hipError_t launch_chem_dtime(const void* mesh, int64_t ncell, const ChemParams& p,
                              ChemCounters* ctr, hipStream_t s);
 hipError_t launch_chem_update(void* mesh, int64_t ncell, hipStream_t s);

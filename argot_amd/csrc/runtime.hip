@@ -173,6 +173,7 @@ struct Ctx {
   DevBuf<float> rate_tab;
   DevBuf<float> smooth_in, smooth_out;   // smooth_photoion_rate planes
   DevBuf<ChemCounters> chem_ctr;
+  DevBuf<unsigned char> chem_paused;   // long cells between the chemistry's two kernels
   hipEvent_t ev_c0 = nullptr, ev_c1 = nullptr;
   argot_chem_stats chem_stats{};
   HostTree tree;
@@ -212,6 +213,7 @@ struct Ctx {
     smooth_in.release();
     smooth_out.release();
     chem_ctr.release();
+    chem_paused.release();
     for (hipEvent_t e : {ev0, ev1, ev_mid, ev_c0, ev_c1})
       if (e) (void)hipEventDestroy(e);
     if (mesh) (void)hipFree(mesh);
@@ -1381,11 +1383,12 @@ static void chem_step(Ctx& g, const run_param* r, float dtime, float* diff_chem,
   // A cell integrates until its elapsed time reaches dtime * tunit: that
   // product must be a finite number of seconds.
   const double dtime_p = (double)dtime * r->tunit;
+  HIP_OK(g.chem_paused.reserve((size_t)kPausedCells * kPausedBytes));
   if (!(dtime_p >= -DBL_MAX && dtime_p <= DBL_MAX)) return set_err(ARGOT_ERR_ARG);
   HIP_OK(hipEventRecord(g.ev_c0, g.stream));
   const int qblocks = g_chem_queue ? 4 * g.ncu : 0;
-  HIP_OK(launch_chem_step(g.mesh, g.ncell, chem_params(r), dtime, g.chem_ctr.p, qblocks,
-                          g_chem_queue, g.stream));
+  HIP_OK(launch_chem_step(g.mesh, g.ncell, chem_params(r), dtime, g.chem_ctr.p, g.chem_paused.p,
+                          qblocks, g_chem_queue, g.stream));
   HIP_OK(hipEventRecord(g.ev_c1, g.stream));
   ChemCounters hc;
   HIP_OK(hipMemcpyAsync(&hc, g.chem_ctr.p, sizeof hc, hipMemcpyDeviceToHost, g.stream));
