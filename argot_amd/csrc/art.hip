@@ -10,13 +10,15 @@
 // on, __HELIUM_BB__ off and __USE_ATOMIC__ off.
 //
 // GPU layout: directions run in batches; each direction of a batch owns a
-// float4 accumulator slice {length, I1, I2, I3} over the mesh, so that the
-// rays of all directions in a batch trace in one launch per ray group.
-// Within a ray group no two rays touch the same cell (their start points
-// are two cells apart and a ray moves at most one cell sideways per layer
-// of its dominant axis), so the accumulators need no atomics and the sums
-// keep the reference's group order.  Per-cell rates then accumulate over
-// the batch's directions in the reference's (sorted) direction order.
+// float4 accumulator slice {length, I1, I2, I3} over the mesh.  Within a ray
+// group no two rays touch the same cell (their start points are two cells
+// apart and a ray moves at most one cell sideways per layer of its dominant
+// axis), so the accumulators need no atomics and the sums keep the reference's
+// group order.  A block sweeps one direction's rays through the box layer by
+// layer with the layer's accumulators in LDS (art_sweep_kernel); where its
+// bounds do not hold, a launch per ray group adds to the slices in memory
+// (art_trace_kernel).  Per-cell rates then accumulate over the batch's
+// directions in the reference's (sorted) direction order.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <string.h>
@@ -59,6 +61,13 @@ struct ArtDir {
   float ovr[3];
   int base;
   double rcp[3];   // 1 / (double)ovr: exact FP32 quotient dx/ovr via div_by
+  float rcpf[3];   // 1 / ovr in FP32: the same quotient via div_exact
+  float pad;
+};
+
+// A cell's absorption coefficients and source functions (3 bands).
+struct ArtMedium {
+  float k0, k1, k2, s0, s1, s2;
 };
 
 struct ArtGrid {
@@ -122,7 +131,7 @@ __device__ inline double k06_B(double t) {
 __global__ void art_rmesh_kernel(const unsigned char* __restrict__ mesh, int nx, int ny, int nz,
                                  double denstonh, double uenetok, double helium_fact,
                                  float csHI, float csHeI, float csHeII,
-                                 float4* __restrict__ med, float4* __restrict__ medT) {
+                                 ArtMedium* __restrict__ med, ArtMedium* __restrict__ medT) {
   const int64_t ncell = (int64_t)nx * ny * nz;
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= ncell) return;
@@ -142,30 +151,25 @@ __global__ void art_rmesh_kernel(const unsigned char* __restrict__ mesh, int nx,
   ne += nHeII + 2.0e0 * nHeIII;
   const double aHI = (double)csHI * nHI;
   const double aHeI = (double)csHeI * nHeI, aHeII = (double)csHeII * nHeII;
-  float4 k;
-  k.x = (float)(aHI + kTinyArt);
-  k.y = (float)(aHI * kRcHI2 + aHeI + kTinyArt);
-  k.z = (float)(aHI * kRcHI3 + aHeI * kRcHeI3 + aHeII + kTinyArt);
-  k.w = 0.0f;
+  ArtMedium r;
+  r.k0 = (float)(aHI + kTinyArt);
+  r.k1 = (float)(aHI * kRcHI2 + aHeI + kTinyArt);
+  r.k2 = (float)(aHI * kRcHI3 + aHeI * kRcHeI3 + aHeII + kTinyArt);
   const double t = temper;
-  float4 s;
-  s.x = (float)((k02_A(t) - k02_B(t)) * ne * nHII * kNuLeV * 1.0 * kEVtoErg / (4.0 * kPiArt) /
-                (double)k.x);
-  s.y = (float)((k04_A(t) - k04_B(t)) * ne * nHeII * kNuLeV * 1.8125 * kEVtoErg /
-                (4.0 * kPiArt) / (double)k.y);
-  s.z = (float)((k06_A(t) - k06_B(t)) * ne * nHeIII * kNuLeV * 4.0 * kEVtoErg / (4.0 * kPiArt) /
-                (double)k.z);
-  s.w = 0.0f;
+  r.s0 = (float)((k02_A(t) - k02_B(t)) * ne * nHII * kNuLeV * 1.0 * kEVtoErg / (4.0 * kPiArt) /
+                (double)r.k0);
+  r.s1 = (float)((k04_A(t) - k04_B(t)) * ne * nHeII * kNuLeV * 1.8125 * kEVtoErg /
+                (4.0 * kPiArt) / (double)r.k1);
+  r.s2 = (float)((k06_A(t) - k06_B(t)) * ne * nHeIII * kNuLeV * 4.0 * kEVtoErg / (4.0 * kPiArt) /
+                (double)r.k2);
   // the record in both trace layouts
   const int ix = (int)(c / ((int64_t)ny * nz));
   const int iy = (int)((c / nz) % ny);
   const int iz = (int)(c % nz);
   const int64_t cm = art_index(false, nx, ny, nz, ix, iy, iz);
   const int64_t cT = art_index(true, nx, ny, nz, ix, iy, iz);
-  med[2 * cm] = k;
-  med[2 * cm + 1] = s;
-  medT[2 * cT] = k;
-  medT[2 * cT + 1] = s;
+  med[cm] = r;
+  medT[cT] = r;
 }
 
 
@@ -178,8 +182,8 @@ struct TraceArgs {
   int ndir;
   int group;              // ray group 0..3 (set_boundary_ray's parity classes)
   int nray_max;           // rays per group and direction (largest face / 4)
-  const float4* med;      // [2*ncell]: absorption (3 bands), source function (3 bands)
-  const float4* medT;     // the same, y-fastest layout (z-dominant directions)
+  const ArtMedium* med;
+  const ArtMedium* medT;  // the same, y-fastest layout (z-dominant directions)
   float4* acc;            // [ndir][ncell] {length, I1, I2, I3}, in the direction's layout
   unsigned long long* ncross;
 };
@@ -268,15 +272,15 @@ __global__ __launch_bounds__(256) void art_trace_kernel(TraceArgs a) {
       float I0 = 0.0f, I1 = 0.0f, I2 = 0.0f;
       const bool zdom = base <= 1;
       float4* __restrict__ acc = a.acc + (int64_t)d * g.ncell;
-      const float4* __restrict__ med = zdom ? a.medT : a.med;
+      const ArtMedium* __restrict__ med = zdom ? a.medT : a.med;
       auto cell = [&]() { return art_index(zdom, g.nx, g.ny, g.nz, ix, iy, iz); };
       bool live = !out();
       int64_t pos = 0;
-      float4 kp{}, sp{}, ac{};
+      ArtMedium m{};
+      float4 ac{};
       if (live) {
         pos = cell();
-        kp = med[2 * pos];
-        sp = med[2 * pos + 1];
+        m = med[pos];
         ac = acc[pos];
       }
       // Each pass: the crossing's geometry and the next cell (with the
@@ -329,25 +333,24 @@ __global__ __launch_bounds__(256) void art_trace_kernel(TraceArgs a) {
           }
         }
         int64_t npos = pos;
-        float4 nkp = kp, nsp = sp, nac = ac;
+        ArtMedium nm = m;
+        float4 nac = ac;
         if (cont) {
           // another ray of this group never touches these cells, and this
           // ray never returns to one: the early read of acc is safe
           npos = cell();
-          nkp = med[2 * npos];
-          nsp = med[2 * npos + 1];
+          nm = med[npos];
           nac = acc[npos];
         }
         ac.x += rmin;
-        band<F64>(kp.x * rmin, sp.x, ac.y, I0);
-        band<F64>(kp.y * rmin, sp.y, ac.z, I1);
-        band<F64>(kp.z * rmin, sp.z, ac.w, I2);
+        band<F64>(m.k0 * rmin, m.s0, ac.y, I0);
+        band<F64>(m.k1 * rmin, m.s1, ac.z, I1);
+        band<F64>(m.k2 * rmin, m.s2, ac.w, I2);
         acc[pos] = ac;
         nc++;
         if (wrapped) I0 = I1 = I2 = 0.0f;
         pos = npos;
-        kp = nkp;
-        sp = nsp;
+        m = nm;
         ac = nac;
         live = cont;
       }
@@ -359,6 +362,286 @@ __global__ __launch_bounds__(256) void art_trace_kernel(TraceArgs a) {
   if ((threadIdx.x & 63) == 0 && nc) atomicAdd(a.ncross, nc);
 }
 
+// The same rays swept layer by layer (along the direction's dominant axis D;
+// A and B are the other two, B the fast one of the layout).
+//
+// A launch per ray group reads and writes a record of the slice per crossing,
+// after a pass that clears it: at 128^3 and 768 directions some 170 GB, which
+// bound the trace (31.3 ms of 37 with the clearing, at 5 TB/s).  Here a
+// block takes one tile of a direction's layers, its accumulators stay in LDS
+// while the four groups pass through the layer one after the other, and the
+// slice is written once: 26 GB, and 17 ms with everything below.  What bounds
+// it now is instruction issue (some 170 vector instructions a crossing and 17%
+// of crossings traced by two tiles) and, second, the phases' barriers: 128
+// registers leave one block of 15 wavefronts a compute unit.
+//
+// Tiles: all rays of a direction are translates of one another, so a tile of
+// cells that moves from layer to layer by the direction's own shift meets the
+// rays of its own start cells and of two more on either side, which are traced
+// by both tiles (start fraction + slope <= 1 + rounding: a ray lies less than
+// two cells from its start cell plus the shift, sweep_applies).  Tiles part a
+// layer's cells exactly; a crossing outside the block's tile adds nothing.  An
+// axis that fits goes whole: no halo, and the rays' wrap stays in the tile.
+// A thread carries four rays, one of each group, the same place in the pairs
+// of cells.
+struct SweepOri {
+  int axA, axB, axD;            // 0 x, 1 y, 2 z
+  int nA, nB, nD;
+  uint32_t mA, mD;              // cell index: split(B) + nB * (mA * A + mD * D)
+  int rA, rB, tA, tB;           // cells of a tile along A and B, tiles
+  int hA, hB;                   // halo: 0 (whole axis) or 2
+  int pA, pB;                   // pairs of rays of a full tile along A and B
+  int swap;                     // group bit 0 belongs to A (else to B)
+  float mnA, mxA, mnB, mxB, mnD, mxD, cell;
+  double centreA, centreB;      // start fractions of set_position
+  const ArtMedium* med;
+};
+
+struct SweepArgs {
+  double lunit;
+  const ArtDir* dirs;
+  int64_t ncell;
+  int tiles;                    // largest tile count of the three orientations
+  float4* acc;
+  unsigned long long* ncross;
+  SweepOri ori[3];              // by base / 2: z, x, y dominant
+};
+
+struct SweepRay {
+  float a, b, d;       // position
+  float i0, i1, i2;    // band intensities
+  int ia, ib;          // cell (the layer is the block's)
+};
+
+// One crossing: path length, place in the tile and flags, the cell's record,
+// its medium.
+constexpr uint32_t kStepMine = 1u << 30, kStepWrap = 1u << 31, kStepSlot = kStepMine - 1;
+struct SweepStep {
+  float rmin;
+  uint32_t at, pos;
+  ArtMedium m;
+};
+// Crossings of a layer that are planned ahead: one per face a ray of slope <= 1
+// can meet; those that rounding adds are taken one by one.
+constexpr int kSweepSteps = 3;
+
+typedef float art_f4 __attribute__((ext_vector_type(4)));
+
+// A barrier for what the block shares in LDS only: __syncthreads also waits for
+// every wave's loads of the medium and stores of the slice.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <bool F64, bool WHOLE_B>
+__global__ __launch_bounds__(1024) void art_sweep_kernel(SweepArgs args) {
+  extern __shared__ float4 cells[];   // [lenA][lenB], B split
+  __shared__ unsigned total;
+  const int dn = (int)(blockIdx.x / args.tiles), tile = (int)(blockIdx.x % args.tiles);
+  const ArtDir* const __restrict__ dir = args.dirs + dn;
+  const SweepOri* const __restrict__ po = args.ori + (dir->base >> 1);
+  const SweepOri& o = *po;
+  if (tile >= o.tA * o.tB) return;
+  const int nA = o.nA, nB = o.nB, nD = o.nD;
+  const uint32_t mA = o.mA;
+  const int a0 = (tile / o.tB) * o.rA, b0 = (tile % o.tB) * o.rB;
+  const int lenA = min(o.rA, nA - a0), lenB = min(o.rB, nB - b0);
+  const float mnA = o.mnA, mnB = o.mnB, mnD = o.mnD, mxA = o.mxA, mxB = o.mxB;
+  const float cell = o.cell;
+  const float ovA = dir->ovr[o.axA], ovB = dir->ovr[o.axB], ovD = dir->ovr[o.axD];
+  const float rcA = dir->rcpf[o.axA], rcB = dir->rcpf[o.axB], rcD = dir->rcpf[o.axD];
+  const int sA = ovA > 0.0f ? 1 : 0, stA = ovA > 0.0f ? 1 : -1;
+  const int sB = ovB > 0.0f ? 1 : 0, stB = ovB > 0.0f ? 1 : -1;
+  const int sD = ovD > 0.0f ? 1 : 0;
+  const ArtMedium* __restrict__ med = o.med;
+  float4* __restrict__ acc = args.acc + (int64_t)dn * args.ncell;
+  const int nthread = blockDim.x, tid = threadIdx.x;
+  for (int q = tid; q < lenA * lenB; q += nthread) cells[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (tid == 0) total = 0;
+
+  // the thread's four rays (set_position, set_start_pos.c:195-229)
+  const int pa = tid / o.pB, pb = tid % o.pB;
+  SweepRay ray[4];
+  bool live[4];
+  unsigned nc = 0;
+  unsigned own = 0;   // rays that start in this tile: their crossings count here
+#pragma unroll
+  for (int grp = 0; grp < 4; grp++) {
+    const int da = grp >> 1, db = grp & 1;
+    const int la = 2 * pa + (o.swap ? db : da) - o.hA, lb = 2 * pb + (o.swap ? da : db) - o.hB;
+    live[grp] = la < lenA + o.hA && lb < lenB + o.hB;
+    if (la >= 0 && la < lenA && lb >= 0 && lb < lenB) own |= 1u << grp;
+    SweepRay& r = ray[grp];
+    r = SweepRay{};
+    r.ia = a0 + la;
+    r.ib = b0 + lb;
+    r.ia += r.ia < 0 ? nA : (r.ia >= nA ? -nA : 0);
+    r.ib += r.ib < 0 ? nB : (r.ib >= nB ? -nB : 0);
+    r.a = (float)((double)mnA + (double)(r.ia + o.centreA) * (double)cell);
+    r.b = (float)((double)mnB + (double)(r.ib + o.centreB) * (double)cell);
+    r.d = sD ? mnD : o.mxD;
+  }
+  // A layer: the face that ends it, its first row, the tile's first cell in it
+  // (start cell plus the rays' shift).
+  struct Layer {
+    float face;
+    uint32_t row;
+    int a, b;
+  };
+  const double slA = (double)ovA / fabs((double)ovD), slB = (double)ovB / fabs((double)ovD);
+  auto at_layer = [&](int layer) {
+    const int iD = sD ? layer : nD - 1 - layer;
+    Layer l{cell * (float)(sD + iD), o.mD * (uint32_t)iD, 0, 0};
+    auto start = [&](int first, double centre, double slope, int n) {
+      int v = first + (int)floor(centre + layer * slope) % n;
+      v += v < 0 ? n : (v >= n ? -n : 0);
+      return __builtin_amdgcn_readfirstlane(v);
+    };
+    if (o.tA > 1) l.a = start(a0, o.centreA, slA, nA);
+    if (o.tB > 1) l.b = start(b0, o.centreB, slB, nB);
+    return l;
+  };
+  // One crossing's geometry, and the ray goes on to the next cell.
+  auto cross = [&](SweepRay& r, const Layer& l, SweepStep& st, bool& leave) {
+    const uint32_t sb = (uint32_t)art_split(r.ib, nB);
+    st.pos = __umul24(__umul24(mA, r.ia) + l.row, nB) + sb;
+    int ja = r.ia - l.a;   // place in the tile
+    ja += ja < 0 ? nA : 0;
+    if (WHOLE_B) {
+      st.at = ja < lenA ? kStepMine | (__umul24(ja, nB) + sb) : 0u;
+    } else {
+      int jb = r.ib - l.b;
+      jb += jb < 0 ? nB : 0;
+      st.at = ja < lenA && jb < lenB
+                  ? kStepMine | (uint32_t)(__umul24(ja, lenB) + art_split(jb, lenB))
+                  : 0u;
+    }
+    const float ddA = cell * (float)(sA + r.ia) - (r.a - mnA);
+    const float ddB = cell * (float)(sB + r.ib) - (r.b - mnB);
+    const float ddD = l.face - (r.d - mnD);
+    const float rdA = fmaxf(div_exact(ddA, ovA, rcA), 0.0f);
+    const float rdB = fmaxf(div_exact(ddB, ovB, rcB), 0.0f);
+    const float rdD = fmaxf(div_exact(ddD, ovD, rcD), 0.0f);
+    const float rmin = fminf(fminf(rdA, rdB), rdD);
+    r.a += rmin * ovA;
+    r.b += rmin * ovB;
+    r.d += rmin * ovD;
+    if (rdA == rmin) r.ia += stA;
+    if (rdB == rmin) r.ib += stB;
+    leave = rdD == rmin;
+    st.rmin = (float)((double)rmin * args.lunit);
+    // a side face wraps the ray to the opposite one, where its intensity
+    // restarts at zero after this cell's update (ray_cycle + reset_I)
+    const bool offA = (unsigned)r.ia >= (unsigned)nA, offB = (unsigned)r.ib >= (unsigned)nB;
+    if (offA || offB) {
+      if (offA) {
+        r.a = r.ia < 0 ? mxA : mnA;
+        r.ia = r.ia < 0 ? nA - 1 : 0;
+      }
+      if (offB) {
+        r.b = r.ib < 0 ? mxB : mnB;
+        r.ib = r.ib < 0 ? nB - 1 : 0;
+      }
+      st.at |= kStepWrap;
+    }
+  };
+  auto absorb = [&](SweepRay& r, const SweepStep& st) {
+    float4* const slot = &cells[st.at & kStepSlot];
+    float4 ac = *slot;
+    ac.x += st.rmin;
+    band<F64>(st.m.k0 * st.rmin, st.m.s0, ac.y, r.i0);
+    band<F64>(st.m.k1 * st.rmin, st.m.s1, ac.z, r.i1);
+    band<F64>(st.m.k2 * st.rmin, st.m.s2, ac.w, r.i2);
+    if (st.at & kStepMine) *slot = ac;
+    if (st.at & kStepWrap) r.i0 = r.i1 = r.i2 = 0.0f;
+  };
+  // Every ray's crossings of a layer are planned one phase ahead of the phase
+  // that absorbs them (the geometry never reads the medium), and their media
+  // loaded between the two, so that a load's latency falls on the next phase's
+  // planning: 6.4 ms per 256 directions of 128^3, against 7.0 with each cell's
+  // medium loaded when the ray reaches it.
+  SweepStep step[2][kSweepSteps];
+  bool act[2][kSweepSteps], more[2];
+  auto plan = [&](SweepRay& r, bool on, const Layer& l, int buf, bool mine) {
+    unsigned n = 0;
+#pragma unroll
+    for (int m = 0; m < kSweepSteps; m++) {
+      act[buf][m] = on;
+      if (on) {
+        bool leave;
+        cross(r, l, step[buf][m], leave);
+        on = !leave;
+        n++;
+      }
+    }
+    more[buf] = on;
+    nc += mine ? n : 0u;
+  };
+  auto load = [&](int buf) {
+#pragma unroll
+    for (int m = 0; m < kSweepSteps; m++)
+      if (act[buf][m]) step[buf][m].m = med[step[buf][m].pos];
+  };
+  // the thread's first slot of the layer and the step to its next ones
+  const int qa = tid / lenB, qs = tid % lenB, stepa = nthread / lenB, steps = nthread % lenB;
+  Layer now = at_layer(0);
+  plan(ray[0], live[0], now, 0, own & 1u);
+  load(0);
+  __syncthreads();
+  for (int layer = 0; layer < nD; layer++) {
+    const bool last = layer == nD - 1;
+    const Layer next = at_layer(last ? layer : layer + 1);
+#pragma unroll
+    for (int grp = 0; grp < 4; grp++) {
+      const int cur = grp & 1, nxt = cur ^ 1;
+      SweepRay& r = ray[grp];
+      if (grp < 3)
+        plan(ray[grp + 1], live[grp + 1], now, nxt, (own >> (grp + 1)) & 1u);
+      else
+        plan(ray[0], live[0] && !last, next, nxt, own & 1u);
+#pragma unroll
+      for (int m = 0; m < kSweepSteps; m++)
+        if (act[cur][m]) absorb(r, step[cur][m]);
+      for (bool on = more[cur]; on;) {
+        SweepStep st;
+        bool leave;
+        cross(r, now, st, leave);
+        st.m = med[st.pos];
+        absorb(r, st);
+        nc += (own >> grp) & 1u;
+        on = !leave;
+      }
+      load(nxt);
+      lds_barrier();
+    }
+    // the layer's tile to the slice, and clear
+    for (int q = tid, qA = qa, qS = qs; q < lenA * lenB; q += nthread) {
+      const float4 v = cells[q];
+      cells[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+      const int h = lenB >> 1;
+      int gA = now.a + qA, gB = now.b + (qS < h ? 2 * qS : 2 * (qS - h) + 1);
+      gA -= gA >= nA ? nA : 0;
+      gB -= gB >= nB ? nB : 0;
+      const uint32_t pos =
+          __umul24(__umul24(mA, gA) + now.row, nB) + (uint32_t)art_split(gB, nB);
+      __builtin_nontemporal_store((art_f4){v.x, v.y, v.z, v.w},
+                                  reinterpret_cast<art_f4*>(acc + pos));
+      qA += stepa;
+      qS += steps;
+      if (qS >= lenB) { qS -= lenB; qA++; }
+    }
+    now = next;
+    lds_barrier();
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) nc += __shfl_xor(nc, off, 64);
+  if ((tid & 63) == 0) atomicAdd(&total, nc);
+  __syncthreads();
+  if (tid == 0 && total) atomicAdd(args.ncross, (unsigned long long)total);
+}
+
 __global__ void art_fill_kernel(float4* __restrict__ p, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -368,24 +651,29 @@ __global__ void art_fill_kernel(float4* __restrict__ p, int64_t n) {
 // calc_GH_tot for the batch's directions in order: gh[k][c] (FP32, 6
 // outputs GHI, HHI, GHeI, HHeI, GHeII, HHeII); optionally Kahan-compensated
 // across directions.
-// One block per 32 x 32 (y, z) tile of one x plane, one thread per cell.
+// One block per TILE x TILE (y, z) tile of one x plane, one thread per cell.
 // The slices of x- and y-dominant directions are read in their own layout
 // (z fastest); those of z-dominant directions (y fastest) go through an LDS
 // tile, read along y and used along z, so that every read is a contiguous
-// run.  Each cell's sums take the directions in batch order.
-// Grid: (ceil(ny/32) ceil(nz/32), nx), blocks of kGhTile^2 threads.
-constexpr int kGhTile = 32;
-template <bool KAHAN>
-__global__ __launch_bounds__(kGhTile * kGhTile) void art_gh_kernel(
+// run.  Each cell's sums take the directions in batch order.  TILE 32 reads at
+// the rate of the memory (5 TB/s).  Where its blocks would leave compute units
+// without work (below two per unit), TILE 16 makes four times as many, which
+// take two directions at once (one wavefront's chain of FP64 operations is
+// what lasts) with the next two on their way: 32^3 with 192 directions 120 us
+// instead of 197.  (Fetching ahead at 128^3 costs the wide tile a third: 2.30 ms per 256 directions instead of 1.73.)
+// Grid: (ceil(ny/TILE) ceil(nz/TILE), nx), blocks of TILE^2 threads.
+template <bool KAHAN, int TILE>
+__global__ __launch_bounds__(TILE * TILE) void art_gh_kernel(
     const float4* __restrict__ acc, const ArtDir* __restrict__ dirs, int ndir, int nx, int ny,
-    int nz, const float4* __restrict__ med, float f0, float f1, float f2, float f3, float f4,
+    int nz, const ArtMedium* __restrict__ med, float f0, float f1, float f2, float f3, float f4,
     float f5, float* __restrict__ gh, float* __restrict__ comp) {
-  __shared__ float4 tile[kGhTile][kGhTile + 1];
+  constexpr int P = TILE < 32 ? 2 : 1;   // directions at once
+  __shared__ float4 tile[P][TILE][TILE + 1];
   const int64_t ncell = (int64_t)nx * ny * nz;
-  const int ntz = (nz + kGhTile - 1) / kGhTile;
-  const int y0 = (int)(blockIdx.x / ntz) * kGhTile, z0 = (int)(blockIdx.x % ntz) * kGhTile;
+  const int ntz = (nz + TILE - 1) / TILE;
+  const int y0 = (int)(blockIdx.x / ntz) * TILE, z0 = (int)(blockIdx.x % ntz) * TILE;
   const int ix = blockIdx.y;
-  const int tz = threadIdx.x % kGhTile, ty = threadIdx.x / kGhTile;
+  const int tz = threadIdx.x % TILE, ty = threadIdx.x / TILE;
   const int iy = y0 + ty, iz = z0 + tz;
   const bool valid = iy < ny && iz < nz;
   // this cell's record in the layout of x- and y-dominant directions
@@ -395,8 +683,8 @@ __global__ __launch_bounds__(kGhTile * kGhTile) void art_gh_kernel(
   // cell (y0 + tz, z0 + ty), read along y
   const bool tvalid = y0 + tz < ny && z0 + ty < nz;
   const int64_t ct = tvalid ? art_index(true, nx, ny, nz, ix, y0 + tz, z0 + ty) : 0;
-  const float4 ka = valid ? med[2 * cs] : make_float4(1.0f, 1.0f, 1.0f, 0.0f);
-  const float4 so = valid ? med[2 * cs + 1] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const ArtMedium m = valid ? med[cs] : ArtMedium{1.0f, 1.0f, 1.0f, 0.0f, 0.0f, 0.0f};
+  const float3 ka = make_float3(m.k0, m.k1, m.k2), so = make_float3(m.s0, m.s1, m.s2);
   float s[6], e[6];
 #pragma unroll
   for (int k = 0; k < 6; k++) {
@@ -419,51 +707,78 @@ __global__ __launch_bounds__(kGhTile * kGhTile) void art_gh_kernel(
   double sh1 = so.y;
   sh1 += (double)so.z * kRhHeI3;
   const double sg2 = so.z, sh2 = so.z;
-  for (int d = 0; d < ndir; d++) {
-    float4 a;
-    if (dirs[d].base <= 1) {   // the same for the whole block
-      __syncthreads();         // the previous tile has been read
-      if (tvalid) tile[ty][tz] = acc[(int64_t)d * ncell + ct];
-      __syncthreads();
-      a = tile[tz][ty];
-    } else {
-      a = acc[(int64_t)d * ncell + cs];
+  auto zdom = [&](int d) { return dirs[d].base <= 1; };   // the same for the whole block
+  auto record = [&](int d) {
+    if (d >= ndir) return make_float4(1.0f, 0.0f, 0.0f, 0.0f);
+    return (zdom(d) ? tvalid : valid) ? acc[(int64_t)d * ncell + (zdom(d) ? ct : cs)]
+                                      : make_float4(1.0f, 0.0f, 0.0f, 0.0f);
+  };
+  float4 ahead[P];
+  if (P > 1)
+#pragma unroll
+    for (int p = 0; p < P; p++) ahead[p] = record(p);
+  for (int d = 0; d < ndir; d += P) {
+    float4 a[P];
+    bool turn = false;
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+      a[p] = P > 1 ? ahead[p] : record(d);
+      turn = turn || (d + p < ndir && zdom(d + p));
+    }
+    if (P > 1)
+#pragma unroll
+      for (int p = 0; p < P; p++) ahead[p] = record(d + P + p);
+    if (turn) {
+      lds_barrier();           // the previous tiles have been read
+#pragma unroll
+      for (int p = 0; p < P; p++) tile[p][ty][tz] = a[p];
+      lds_barrier();
+#pragma unroll
+      for (int p = 0; p < P; p++)
+        if (d + p < ndir && zdom(d + p)) a[p] = tile[p][tz][ty];
     }
     if (!valid) continue;
-    const double rl = 1.0 / (double)a.x;
-    const double q1 = (double)div_by(a.y, rkx);   // I_1 / kappa_1 (float, as the reference)
-    const double q2 = (double)div_by(a.z, rky);
-    const double q3 = (double)div_by(a.w, rkz);
-    const double z2 = (double)a.z * rky, w3 = (double)a.w * rkz;
-    double v[6];
-    // HI
-    double Ig = q1;
-    Ig += z2 * kRjHI2;
-    Ig += w3 * kRjHI3;
-    double Ih = q1;
-    Ih += z2 * kRhHI2;
-    Ih += w3 * kRhHI3;
-    v[0] = (Ig * rl + sg0) * f[0];
-    v[1] = (Ih * rl + sh0) * f[1];
-    // HeI
-    Ig = q2;
-    Ig += w3 * kRjHeI3;
-    Ih = q2;
-    Ih += w3 * kRhHeI3;
-    v[2] = (Ig * rl + sg1) * f[2];
-    v[3] = (Ih * rl + sh1) * f[3];
-    // HeII
-    v[4] = (q3 * rl + sg2) * f[4];
-    v[5] = (q3 * rl + sh2) * f[5];
+    double v[P][6];
 #pragma unroll
-    for (int k = 0; k < 6; k++) {
-      if (KAHAN) {
-        const float y = (float)v[k] - e[k];
-        const float t = s[k] + y;
-        e[k] = (t - s[k]) - y;
-        s[k] = t;
-      } else {
-        s[k] = (float)((double)s[k] + v[k]);
+    for (int p = 0; p < P; p++) {
+      const double rl = 1.0 / (double)a[p].x;
+      const double q1 = (double)div_by(a[p].y, rkx);   // I_1 / kappa_1 (float, as the reference)
+      const double q2 = (double)div_by(a[p].z, rky);
+      const double q3 = (double)div_by(a[p].w, rkz);
+      const double z2 = (double)a[p].z * rky, w3 = (double)a[p].w * rkz;
+      // HI
+      double Ig = q1;
+      Ig += z2 * kRjHI2;
+      Ig += w3 * kRjHI3;
+      double Ih = q1;
+      Ih += z2 * kRhHI2;
+      Ih += w3 * kRhHI3;
+      v[p][0] = (Ig * rl + sg0) * f[0];
+      v[p][1] = (Ih * rl + sh0) * f[1];
+      // HeI
+      Ig = q2;
+      Ig += w3 * kRjHeI3;
+      Ih = q2;
+      Ih += w3 * kRhHeI3;
+      v[p][2] = (Ig * rl + sg1) * f[2];
+      v[p][3] = (Ih * rl + sh1) * f[3];
+      // HeII
+      v[p][4] = (q3 * rl + sg2) * f[4];
+      v[p][5] = (q3 * rl + sh2) * f[5];
+    }
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+      if (d + p >= ndir) break;
+#pragma unroll
+      for (int k = 0; k < 6; k++) {
+        if (KAHAN) {
+          const float y = (float)v[p][k] - e[k];
+          const float t = s[k] + y;
+          e[k] = (t - s[k]) - y;
+          s[k] = t;
+        } else {
+          s[k] = (float)((double)s[k] + v[p][k]);
+        }
       }
     }
   }
@@ -494,7 +809,7 @@ __global__ void art_gh_sum_kernel(unsigned char* __restrict__ mesh, int64_t ncel
 
 int g_nside = 8;             // N_SIDE (run_param.h:159)
 int g_heatcool = 1;          // __HEATCOOL__ (src/Makefile:187)
-int g_batch = 0;             // directions per batch; 0: as many as 8 GiB of slices hold, <= 128
+int g_batch = 0;             // directions per batch; 0: as many as 8 GiB of slices hold, <= 256
 int g_kahan = 0;
 int g_exp64 = 0;             // 1: exp/expm1 in FP64 as the reference
 argot_diffuse_stats g_dstats{};
@@ -502,12 +817,13 @@ argot_diffuse_stats g_dstats{};
 struct ArtCtx {
   int nside = 0;
   std::vector<ArtDir> dirs;       // sorted order
+  bool sweep = false;             // sweep_directions(dirs)
   float fact[6] = {0, 0, 0, 0, 0, 0};
   hipStream_t stream = nullptr;
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   ArtDir* d_dirs = nullptr;
-  float4 *med = nullptr, *acc = nullptr;   // med: [2*ncell] absorption, source
-  float4* medT = nullptr;   // y-fastest medium
+  ArtMedium *med = nullptr, *medT = nullptr;   // [ncell]; medT: y-fastest
+  float4* acc = nullptr;
   float *gh = nullptr, *comp = nullptr;
   unsigned long long* ncross = nullptr;
   int64_t ncell = 0;
@@ -524,6 +840,72 @@ ArtCtx a_;
       return;                                                                       \
     }                                                                               \
   } while (0)
+
+// Tiles of art_sweep_kernel for layers of nA x nB cells: the split with the
+// fewest lanes over all tiles, of at most 1024 threads (four rays each) and
+// 64 KiB of LDS a block.  128 x 128: 5 tiles of 26 whole rows (17% more rays
+// than start cells); 256 x 256: 4 x 5 tiles of 64 x 52 (17%); up to 64 x 64
+// one tile.
+constexpr int kSweepThreads = 1024, kSweepCells = 4096;
+void sweep_tiles(SweepOri& o) {
+  int64_t best = 0;
+  auto axis = [](int n, int t, int& r, int& h) {   // n cells in about t tiles
+    r = t == 1 ? n : ((n + t - 1) / t + 1) & ~1;
+    h = r < n ? 2 : 0;
+    return r == n || r + 4 <= n;
+  };
+  for (int ta = 1; ta <= o.nA; ta++) {
+    int rA, hA;
+    if (!axis(o.nA, ta, rA, hA)) continue;
+    const int pA = (rA + 2 * hA) / 2;
+    for (int tb = 1; tb <= o.nB; tb++) {
+      int rB, hB;
+      if (!axis(o.nB, tb, rB, hB)) continue;
+      const int pB = (rB + 2 * hB) / 2;
+      if ((int64_t)pA * pB > kSweepThreads || (int64_t)rA * rB > kSweepCells) continue;
+      const int cA = (o.nA + rA - 1) / rA, cB = (o.nB + rB - 1) / rB;
+      const int64_t lanes = (int64_t)cA * cB * ((pA * pB + 63) & ~63);
+      if (best == 0 || lanes <= best) {   // (of equals the longest runs along B)
+        best = lanes;
+        o.rA = rA; o.rB = rB; o.hA = hA; o.hB = hB; o.pA = pA; o.pB = pB; o.tA = cA; o.tB = cB;
+      }
+      break;   // more tiles along B at this ta only add halo
+    }
+  }
+}
+
+// Whether the sweep's bounds hold for the directions: bases that name their
+// dominant axis and sign, and components (1e-31 at least, make_angles) whose
+// reciprocals and remainders stay normal in FP32.
+bool sweep_directions(const std::vector<ArtDir>& dirs) {
+  for (const ArtDir& d : dirs) {
+    if (d.base < 0 || d.base > 5) return false;
+    const int ax = d.base <= 1 ? 2 : (d.base <= 3 ? 0 : 1);
+    const double lead = (d.base & 1) ? -(double)d.ovr[ax] : (double)d.ovr[ax];
+    if (!(lead > 0.1 && lead < 2.0)) return false;
+    for (int k = 0; k < 3; k++)
+      if (!(fabs((double)d.ovr[k]) <= lead * (1.0 + 1e-5) && fabs((double)d.ovr[k]) >= 9.9e-32))
+        return false;
+  }
+  return true;
+}
+
+// Whether they hold for the box: cell indices in 32 bits, faces where the
+// cells end, and rays whose rounding (at most 3 crossings a layer, each within
+// 2 ulp of the largest coordinate) stays below half a cell of the halo's slack.
+bool sweep_applies(const ArtGrid& g) {
+  const double mn[3] = {g.xmin, g.ymin, g.zmin}, mx[3] = {g.xmax, g.ymax, g.zmax};
+  const double d[3] = {g.dx, g.dy, g.dz};
+  const int n[3] = {g.nx, g.ny, g.nz};
+  double big = 0.0;
+  for (int k = 0; k < 3; k++) {
+    if (!(d[k] > 1e-12 && d[k] < 1e6) || !(fabs(mx[k] - mn[k] - n[k] * d[k]) < 0.05 * d[k])) return false;
+    big = std::max(big, std::max(fabs(mn[k]), fabs(mx[k])));
+  }
+  const double err = 6.0 * ((double)g.nx + g.ny + g.nz) * big * 1.2e-7 / d[0];
+  const int64_t rows = std::max((int64_t)g.nx * g.ny, (int64_t)g.nx * g.nz);   // 24-bit products
+  return err < 0.5 && g.ncell <= ((int64_t)1 << 30) && std::max(rows, (int64_t)g.ny * g.nz) < (1 << 24);
+}
 
 double now_ms() {
   return std::chrono::duration<double, std::milli>(
@@ -712,7 +1094,7 @@ void init_diffuse_gpu(struct cuda_diffuse_param* cd, struct cuda_param* this_cud
   int batch = g_batch;
   if (batch <= 0) {
     const int64_t fit = ((int64_t)8 << 30) / (16 * ncell);
-    batch = (int)std::max<int64_t>(1, std::min<int64_t>(128, fit));
+    batch = (int)std::max<int64_t>(1, std::min<int64_t>(256, fit));
   }
   batch = std::min(batch, nang);
   if (!a_.stream) {
@@ -723,7 +1105,8 @@ void init_diffuse_gpu(struct cuda_diffuse_param* cd, struct cuda_param* this_cud
                   (void*)a_.comp, (void*)a_.ncross, (void*)a_.medT})
     if (p) A_OK(hipFree(p));
   a_.d_dirs = nullptr;
-  a_.med = a_.acc = nullptr;
+  a_.med = nullptr;
+  a_.acc = nullptr;
   a_.medT = nullptr;
   a_.gh = a_.comp = nullptr;
   a_.ncross = nullptr;
@@ -733,9 +1116,9 @@ void init_diffuse_gpu(struct cuda_diffuse_param* cd, struct cuda_param* this_cud
   a_.ncell = 0;
   a_.batch = 0;
   A_OK(hipMalloc(&a_.d_dirs, sizeof(ArtDir) * nang));
-  A_OK(hipMalloc(&a_.med, sizeof(float4) * 2 * ncell));
+  A_OK(hipMalloc(&a_.med, sizeof(ArtMedium) * ncell));
   A_OK(hipMalloc(&a_.acc, sizeof(float4) * ncell * batch));
-  A_OK(hipMalloc(&a_.medT, sizeof(float4) * 2 * ncell));
+  A_OK(hipMalloc(&a_.medT, sizeof(ArtMedium) * ncell));
   A_OK(hipMalloc(&a_.gh, sizeof(float) * 6 * ncell));
   A_OK(hipMalloc(&a_.comp, sizeof(float) * 6 * ncell));
   A_OK(hipMalloc(&a_.ncross, sizeof(unsigned long long)));
@@ -765,11 +1148,16 @@ void send_diffuse_data(struct host_diffuse_param* hd, struct cuda_diffuse_param*
     d.ovr[1] = an.yovr;
     d.ovr[2] = an.zovr;
     d.base = an.base_id;
-    for (int k = 0; k < 3; k++) d.rcp[k] = 1.0 / (double)d.ovr[k];
+    for (int k = 0; k < 3; k++) {
+      d.rcp[k] = 1.0 / (double)d.ovr[k];
+      d.rcpf[k] = 1.0f / d.ovr[k];
+    }
+    d.pad = 0.0f;
   }
   const step_func_factor* sf = hd->step_fact;
   const float f[6] = {sf->HI[0], sf->HI[1], sf->HeI[0], sf->HeI[1], sf->HeII[0], sf->HeII[1]};
   memcpy(a_.fact, f, sizeof f);
+  a_.sweep = sweep_directions(a_.dirs);
   A_OK(hipMemcpy(a_.d_dirs, a_.dirs.data(), sizeof(ArtDir) * nang, hipMemcpyHostToDevice));
 }
 
@@ -825,40 +1213,94 @@ void calc_diffuse_photon_radiation(struct fluid_mesh* mesh, struct run_param* th
   const int nang = (int)a_.dirs.size();
   const int nray_max = std::max(g.nx * g.ny, std::max(g.ny * g.nz, g.nz * g.nx)) / 4;
   float trace_ms = 0.0f, gh_ms = 0.0f;
+  const bool sweep = a_.sweep && sweep_applies(g);
+  SweepArgs sa{};
+  unsigned sweep_threads = 0, sweep_lds = 0;
+  bool sweep_whole = true;   // B whole in every orientation
+  if (sweep) {
+    const int n[3] = {g.nx, g.ny, g.nz};
+    const float mn[3] = {g.xmin, g.ymin, g.zmin}, mx[3] = {g.xmax, g.ymax, g.zmax};
+    const double centre[3] = {0.521212345, 0.508512345, 0.468287655};
+    sa.lunit = g.lunit;
+    sa.ncell = nc;
+    sa.acc = a_.acc;
+    sa.ncross = a_.ncross;
+    // {A, B, D, group bit of A} for z-, x- and y-dominant directions
+    const int axes[3][4] = {{0, 1, 2, 0}, {1, 2, 0, 0}, {0, 2, 1, 1}};
+    for (int k = 0; k < 3; k++) {
+      SweepOri& o = sa.ori[k];
+      o.axA = axes[k][0];
+      o.axB = axes[k][1];
+      o.axD = axes[k][2];
+      o.swap = axes[k][3];
+      o.nA = n[o.axA];
+      o.nB = n[o.axB];
+      o.nD = n[o.axD];
+      o.mA = k == 2 ? (uint32_t)o.nD : 1u;
+      o.mD = k == 2 ? 1u : (uint32_t)o.nA;
+      o.mnA = mn[o.axA];
+      o.mxA = mx[o.axA];
+      o.mnB = mn[o.axB];
+      o.mxB = mx[o.axB];
+      o.mnD = mn[o.axD];
+      o.mxD = mx[o.axD];
+      o.cell = g.dx;
+      o.centreA = centre[o.axA];
+      o.centreB = centre[o.axB];
+      o.med = k == 0 ? a_.medT : a_.med;
+      sweep_tiles(o);
+      sa.tiles = std::max(sa.tiles, o.tA * o.tB);
+      sweep_whole = sweep_whole && o.tB == 1;
+      sweep_threads = std::max(sweep_threads, (unsigned)(o.pA * o.pB + 63) & ~63u);
+      sweep_lds = std::max(sweep_lds, (unsigned)(sizeof(float4) * o.rA * o.rB));
+    }
+  }
   for (int d0 = 0; d0 < nang; d0 += a_.batch) {
     const int nd = std::min(a_.batch, nang - d0);
-    const int64_t nacc = (int64_t)nd * nc;
-    art_fill_kernel<<<(unsigned)((nacc + 255) / 256), 256, 0, st>>>(a_.acc, nacc);
     A_OK(hipEventRecord(a_.ev[1], st));
-    TraceArgs ta;
-    ta.g = g;
-    ta.dirs = a_.d_dirs + d0;
-    ta.ndir = nd;
-    ta.nray_max = nray_max;
-    ta.med = a_.med;
-    ta.medT = a_.medT;
-    ta.acc = a_.acc;
-    ta.ncross = a_.ncross;
-    const int64_t nthread = (int64_t)nd * nray_max;
-    for (int grp = 0; grp < 4; grp++) {
-      ta.group = grp;
-      if (g_exp64)
-        art_trace_kernel<true><<<(unsigned)((nthread + 255) / 256), 256, 0, st>>>(ta);
-      else
-        art_trace_kernel<false><<<(unsigned)((nthread + 255) / 256), 256, 0, st>>>(ta);
+    if (sweep) {
+      sa.dirs = a_.d_dirs + d0;
+      const unsigned nblock = (unsigned)(sa.tiles * nd);
+      const auto kernel = g_exp64 ? (sweep_whole ? art_sweep_kernel<true, true>
+                                                 : art_sweep_kernel<true, false>)
+                                  : (sweep_whole ? art_sweep_kernel<false, true>
+                                                 : art_sweep_kernel<false, false>);
+      kernel<<<nblock, sweep_threads, sweep_lds, st>>>(sa);
+    } else {
+      const int64_t nacc = (int64_t)nd * nc;
+      art_fill_kernel<<<(unsigned)((nacc + 255) / 256), 256, 0, st>>>(a_.acc, nacc);
+      TraceArgs ta;
+      ta.g = g;
+      ta.dirs = a_.d_dirs + d0;
+      ta.ndir = nd;
+      ta.nray_max = nray_max;
+      ta.med = a_.med;
+      ta.medT = a_.medT;
+      ta.acc = a_.acc;
+      ta.ncross = a_.ncross;
+      const int64_t nthread = (int64_t)nd * nray_max;
+      for (int grp = 0; grp < 4; grp++) {
+        ta.group = grp;
+        if (g_exp64)
+          art_trace_kernel<true><<<(unsigned)((nthread + 255) / 256), 256, 0, st>>>(ta);
+        else
+          art_trace_kernel<false><<<(unsigned)((nthread + 255) / 256), 256, 0, st>>>(ta);
+      }
     }
+    A_OK(hipGetLastError());
     A_OK(hipEventRecord(a_.ev[2], st));
     const float* f = a_.fact;
-    const dim3 ghgrid((unsigned)(((g.ny + kGhTile - 1) / kGhTile) * ((g.nz + kGhTile - 1) / kGhTile)),
+    auto sums = [&](auto kernel, int tile) {
+      const dim3 grid((unsigned)(((g.ny + tile - 1) / tile) * ((g.nz + tile - 1) / tile)),
                       (unsigned)g.nx);
+      kernel<<<grid, tile * tile, 0, st>>>(a_.acc, a_.d_dirs + d0, nd, g.nx, g.ny, g.nz, a_.med,
+                                           f[0], f[1], f[2], f[3], f[4], f[5], a_.gh, a_.comp);
+    };
+    const bool wide = (int64_t)((g.ny + 31) / 32) * ((g.nz + 31) / 32) * g.nx >= 512;
     if (g_kahan)
-      art_gh_kernel<true><<<ghgrid, kGhTile * kGhTile, 0, st>>>(
-          a_.acc, a_.d_dirs + d0, nd, g.nx, g.ny, g.nz, a_.med, f[0], f[1], f[2], f[3], f[4],
-          f[5], a_.gh, a_.comp);
+      wide ? sums(art_gh_kernel<true, 32>, 32) : sums(art_gh_kernel<true, 16>, 16);
     else
-      art_gh_kernel<false><<<ghgrid, kGhTile * kGhTile, 0, st>>>(
-          a_.acc, a_.d_dirs + d0, nd, g.nx, g.ny, g.nz, a_.med, f[0], f[1], f[2], f[3], f[4],
-          f[5], a_.gh, a_.comp);
+      wide ? sums(art_gh_kernel<false, 32>, 32) : sums(art_gh_kernel<false, 16>, 16);
     A_OK(hipGetLastError());
     A_OK(hipEventRecord(a_.ev[3], st));
     A_OK(hipEventSynchronize(a_.ev[3]));
@@ -887,7 +1329,8 @@ void free_diffuse_gpu(struct cuda_diffuse_param* cd, struct cuda_param* this_cud
                   (void*)a_.comp, (void*)a_.ncross, (void*)a_.medT})
     if (p) (void)hipFree(p);
   a_.d_dirs = nullptr;
-  a_.med = a_.acc = nullptr;
+  a_.med = nullptr;
+  a_.acc = nullptr;
   a_.medT = nullptr;
   a_.gh = a_.comp = nullptr;
   a_.ncross = nullptr;
