@@ -60,8 +60,8 @@ hipError_t launch_target_rates(const GridDev& g, const RateTables& rt, void* mes
                               const CallTarget* tg, int64_t ntarget, const CallRay* rays,
                               const CallSpectra& sp, hipStream_t s);
 hipError_t launch_reset_counters(StepCounters* ctr, hipStream_t s);
-// smooth_photoion_rate on one rank; tmp_in/tmp_out: 6*ncell floats each.
-// On return (stream order) tmp_out holds the smoothed rates as six planes.
+// smooth_photoion_rate on one rank; tmp_in: 6*ncell floats; tmp_out: null, or
+// 6*ncell floats that get the smoothed rates as six planes too.
 hipError_t launch_smooth_rates(void* mesh, int nx, int ny, int nz, float* tmp_in, float* tmp_out,
                                hipStream_t s);
 hipError_t launch_copy_probe(const float4* src, float4* dst, int64_t n, int nblock,

@@ -1432,10 +1432,8 @@ static void step_radiation_tree_body(struct fluid_mesh* mesh, struct radiation_s
   int iter = 1;
   for (;;) {
     HIP_OK(g.smooth_in.reserve(6 * (size_t)g.ncell));
-    HIP_OK(g.smooth_out.reserve(6 * (size_t)g.ncell));
     HIP_OK(hipEventRecord(g.ev_c0, g.stream));
-    HIP_OK(launch_smooth_rates(g.mesh, g.nx, g.ny, g.nz, g.smooth_in.p, g.smooth_out.p,
-                               g.stream));
+    HIP_OK(launch_smooth_rates(g.mesh, g.nx, g.ny, g.nz, g.smooth_in.p, nullptr, g.stream));
     HIP_OK(hipEventRecord(g.ev_c1, g.stream));
     HIP_OK(hipEventSynchronize(g.ev_c1));
     float ms_s = 0.0f;
@@ -1566,8 +1564,9 @@ static void smooth_photoion_rate_body(struct fluid_mesh* mesh, struct run_param*
   if (this_run->nnode_x > 1 || this_run->nnode_y > 1 || this_run->nnode_z > 1)
     return set_err(ARGOT_ERR_ARG);   // the halo exchange of several ranks is not built
   HIP_OK(g.smooth_in.reserve(6 * (size_t)g.ncell));
-  HIP_OK(g.smooth_out.reserve(6 * (size_t)g.ncell));
-  HIP_OK(launch_smooth_rates(g.mesh, g.nx, g.ny, g.nz, g.smooth_in.p, g.smooth_out.p, g.stream));
+  if (mesh) HIP_OK(g.smooth_out.reserve(6 * (size_t)g.ncell));
+  HIP_OK(launch_smooth_rates(g.mesh, g.nx, g.ny, g.nz, g.smooth_in.p,
+                             mesh ? g.smooth_out.p : nullptr, g.stream));
   if (mesh) {
     std::vector<float> soa(6 * (size_t)g.ncell);
     HIP_OK(hipMemcpyAsync(soa.data(), g.smooth_out.p, sizeof(float) * soa.size(),
