@@ -23,6 +23,9 @@ struct FusedArgs {
 hipError_t launch_pack_fields(const void* mesh, int64_t ncell, double helium_fact, float4* nf,
                               hipStream_t s);
 hipError_t launch_zero_rates(void* mesh, int64_t ncell, hipStream_t s);
+// launch_pack_fields and launch_zero_rates in one pass, and the counters to zero.
+hipError_t launch_begin_step(void* mesh, int64_t ncell, double helium_fact, float4* nf,
+                             StepCounters* ctr, hipStream_t s);
 hipError_t launch_add_rates(void* mesh, const float* rate, int64_t ncell, hipStream_t s);
 // rate[6c + k] := prev_chem rate k of cell c, and back
 hipError_t launch_get_rates(const void* mesh, float* rate, int64_t ncell, hipStream_t s);
@@ -59,7 +62,6 @@ struct CallSpectra {
 hipError_t launch_target_rates(const GridDev& g, const RateTables& rt, void* mesh,
                               const CallTarget* tg, int64_t ntarget, const CallRay* rays,
                               const CallSpectra& sp, hipStream_t s);
-hipError_t launch_reset_counters(StepCounters* ctr, hipStream_t s);
 // smooth_photoion_rate on one rank; tmp_in: 6*ncell floats; tmp_out: null, or
 // 6*ncell floats that get the smoothed rates as six planes too.
 hipError_t launch_smooth_rates(void* mesh, int nx, int ny, int nz, float* tmp_in, float* tmp_out,

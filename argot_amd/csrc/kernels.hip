@@ -75,6 +75,29 @@ __global__ void zero_rates_kernel(unsigned char* __restrict__ mesh, int64_t ncel
   for (int k = 0; k < 6; k++) r[k] = 0.0f;
 }
 
+// What a step begins with, in one pass over the records: the packed fields, the
+// rates to zero, the counters of the fused kernel.  256^3: 1.04 ms (5.1 TB/s
+// over the records read and written) instead of 0.53 and 0.85 in two passes;
+// 64^3: 14 us instead of 29 in three launches.
+__global__ void begin_step_kernel(unsigned char* __restrict__ mesh, int64_t ncell,
+                                  double helium_fact, float4* __restrict__ nf,
+                                  StepCounters* __restrict__ ctr) {
+  if (blockIdx.x == 0) {
+    const int i = threadIdx.x;
+    if (i < kNumQueues) ctr->queue[i] = StepCounters::Queue{0, 0, 0, 0, 0, 0, 0};
+    if (i == 0) {
+      ctr->nrecord = 0;
+      ctr->noverflow = 0;
+    }
+  }
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= ncell) return;
+  nf[c] = form_fields(mesh, c, helium_fact);
+  float* r = mesh_fw(mesh, c, kOffRates);
+#pragma unroll
+  for (int k = 0; k < 6; k++) r[k] = 0.0f;
+}
+
 __global__ void add_rates_kernel(unsigned char* __restrict__ mesh, const float* __restrict__ rate,
                                  int64_t ncell) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1132,15 +1155,6 @@ hipError_t launch_copy_probe(const float4* src, float4* dst, int64_t n, int nblo
   return hipGetLastError();
 }
 
-__global__ void reset_counters_kernel(StepCounters* ctr) {
-  const int i = threadIdx.x;
-  if (i < kNumQueues) ctr->queue[i] = StepCounters::Queue{0, 0, 0, 0, 0, 0, 0};
-  if (i == 0) {
-    ctr->nrecord = 0;
-    ctr->noverflow = 0;
-  }
-}
-
 // ------------------------------------------------------------------------
 // Launch wrappers (host side).
 
@@ -1155,6 +1169,14 @@ hipError_t launch_pack_fields(const void* mesh, int64_t ncell, double helium_fac
 
 hipError_t launch_zero_rates(void* mesh, int64_t ncell, hipStream_t s) {
   zero_rates_kernel<<<nblocks(ncell, 256), 256, 0, s>>>(static_cast<unsigned char*>(mesh), ncell);
+  return hipGetLastError();
+}
+
+hipError_t launch_begin_step(void* mesh, int64_t ncell, double helium_fact, float4* nf,
+                             StepCounters* ctr, hipStream_t s) {
+  static_assert(kNumQueues <= 256, "one block clears the queues");
+  begin_step_kernel<<<nblocks(ncell, 256), 256, 0, s>>>(static_cast<unsigned char*>(mesh), ncell,
+                                                        helium_fact, nf, ctr);
   return hipGetLastError();
 }
 
@@ -1267,11 +1289,6 @@ hipError_t launch_set_rates(void* mesh, const float* rate, int64_t ncell, hipStr
   if (ncell <= 0) return hipSuccess;
   set_rates_kernel<<<nblocks(ncell, 256), 256, 0, s>>>(static_cast<unsigned char*>(mesh), rate,
                                                       ncell);
-  return hipGetLastError();
-}
-
-hipError_t launch_reset_counters(StepCounters* ctr, hipStream_t s) {
-  reset_counters_kernel<<<1, 64, 0, s>>>(ctr);
   return hipGetLastError();
 }
 
