@@ -662,7 +662,13 @@ void send_run_param_data(struct run_param* this_run, struct cuda_mem_space* cuda
   Ctx& g = *cp;
   t_last = cp;
   HIP_OK(hipMemcpy(g.run_dev, this_run, sizeof(struct run_param), hipMemcpyHostToDevice));
-  upload_tables(g, this_run);
+  try {
+    upload_tables(g, this_run);
+  } catch (const std::bad_alloc&) {
+    set_err(ARGOT_ERR_NOMEM);
+  } catch (...) {
+    set_err(ARGOT_ERR_ARG);
+  }
 }
 
 void allocate_pinned_segment(struct ray_segment** seg, uint64_t nseg) {
