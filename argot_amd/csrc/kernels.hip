@@ -973,9 +973,8 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY void fused_step_kernel(FusedArg
       if constexpr (SURR) {
         // The network runs on the whole wavefront (MFMA) and serves the
         // visit only when every emitting lane can use it; otherwise every
-        // lane takes the exact integral below.  Two 64x64 network
-        // evaluations cost about as much as the exact 256-bin loop, so a
-        // visit that ran both would cost twice as much.
+        // lane takes the exact integral below: a visit that ran both would
+        // pay for both.
         const double qn = a.surr.node_q[u];
         float xa[3] = {0.0f, 0.0f, 0.0f}, xb[3] = {0.0f, 0.0f, 0.0f};
         const bool use = work && surr_inputs(a.surr, rt, rr, qn, xa, xb);

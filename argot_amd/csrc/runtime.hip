@@ -1240,8 +1240,9 @@ static void point_source_pass(Ctx& g, struct radiation_src* src, struct run_para
   const HostTree& T = g.tree;
   const int nn = T.nnode();
   // The tree's arrays one after the other in one buffer, through one pinned
-  // copy: five pageable ones, each with its own staging, took 45 us of a 16^3
-  // step and 0.8 ms of the 4096-source one.  (The copy has ended when the pass
+  // copy.  With five pageable ones, each with its own staging, and three
+  // launches before them a 16^3 step took 307 us instead of 202, the 256^3 one
+  // with 4096 sources 81 ms instead of 80.  (The copy has ended when the pass
   // returns: it waits for the stream.)
   size_t bytes = 0;
   auto section = [&](size_t n) {
