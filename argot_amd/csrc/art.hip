@@ -62,7 +62,7 @@ struct ArtDir {
   int base;
   double rcp[3];   // 1 / (double)ovr: exact FP32 quotient dx/ovr via div_by
   float rcpf[3];   // 1 / ovr in FP32: the same quotient via div_exact
-  float pad;
+  int order;       // the batch's direction that this place of the launch sweeps
 };
 
 // A cell's absorption coefficients and source functions (3 bands).
@@ -370,16 +370,21 @@ __global__ __launch_bounds__(256) void art_trace_kernel(TraceArgs a) {
 // bound the trace (31.3 ms of 37 with the clearing, at 5 TB/s).  Here a
 // block takes one tile of a direction's layers, its accumulators stay in LDS
 // while the four groups pass through the layer one after the other, and the
-// slice is written once: 26 GB, and 17 ms with everything below.  What bounds
-// it now is instruction issue (some 170 vector instructions a crossing and 17%
-// of crossings traced by two tiles) and, second, the phases' barriers: 128
-// registers leave one block of 15 wavefronts a compute unit.
+// slice is written once: 26 GB, and 15.5 to 16.5 ms with everything below.
+// What bounds it now is the memory again: 13 GB of medium (each direction reads
+// it once; nearly nothing is shared between directions) and 8.6 GB of slices
+// for 256 directions, 4.1 TB/s of the 4.75 that a copy reaches.  Blocks of 512
+// threads leave two to a compute unit at 115 registers, so that one runs while
+// the other meets a barrier (1024 threads and one block: 5% slower; 640 threads
+// and 96 registers spill: 36 ms a pass instead of 21).
 //
 // Tiles: all rays of a direction are translates of one another, so a tile of
 // cells that moves from layer to layer by the direction's own shift meets the
-// rays of its own start cells and of two more on either side, which are traced
-// by both tiles (start fraction + slope <= 1 + rounding: a ray lies less than
-// two cells from its start cell plus the shift, sweep_applies).  Tiles part a
+// rays of its own start cells and of two more on the side they come from, which
+// two tiles trace: with p the ray's place at the layer's entry and a shift of
+// floor(p - 1/4), a ray of slope up to 1 touches the cells 0 to 2 from its start
+// cell plus the shift, also where rounding moved it by 0.2 cells (sweep_applies;
+// the mirror image for slopes below 0).  Tiles part a
 // layer's cells exactly; a crossing outside the block's tile adds nothing.  An
 // axis that fits goes whole: no halo, and the rays' wrap stays in the tile.
 // A thread carries four rays, one of each group, the same place in the pairs
@@ -389,7 +394,7 @@ struct SweepOri {
   int nA, nB, nD;
   uint32_t mA, mD;              // cell index: split(B) + nB * (mA * A + mD * D)
   int rA, rB, tA, tB;           // cells of a tile along A and B, tiles
-  int hA, hB;                   // halo: 0 (whole axis) or 2
+  int hA, hB;                   // halo rays: 0 (whole axis) or 2
   int pA, pB;                   // pairs of rays of a full tile along A and B
   int swap;                     // group bit 0 belongs to A (else to B)
   float mnA, mxA, mnB, mxB, mnD, mxD, cell;
@@ -421,9 +426,10 @@ struct SweepStep {
   uint32_t at, pos;
   ArtMedium m;
 };
-// Crossings of a layer that are planned ahead: one per face a ray of slope <= 1
-// can meet; those that rounding adds are taken one by one.
-constexpr int kSweepSteps = 3;
+// Crossings of a layer that are planned ahead.  A fifth of a ray's layers have a
+// third one; it is taken by itself, as are those that rounding could add (three
+// planned ahead: 3% slower).
+constexpr int kSweepSteps = 2;
 
 typedef float art_f4 __attribute__((ext_vector_type(4)));
 
@@ -436,10 +442,10 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 template <bool F64, bool WHOLE_B>
-__global__ __launch_bounds__(1024) void art_sweep_kernel(SweepArgs args) {
+__global__ __launch_bounds__(512, 4) void art_sweep_kernel(SweepArgs args) {
   extern __shared__ float4 cells[];   // [lenA][lenB], B split
   __shared__ unsigned total;
-  const int dn = (int)(blockIdx.x / args.tiles), tile = (int)(blockIdx.x % args.tiles);
+  const int dn = args.dirs[blockIdx.x / args.tiles].order, tile = (int)(blockIdx.x % args.tiles);
   const ArtDir* const __restrict__ dir = args.dirs + dn;
   const SweepOri* const __restrict__ po = args.ori + (dir->base >> 1);
   const SweepOri& o = *po;
@@ -470,8 +476,9 @@ __global__ __launch_bounds__(1024) void art_sweep_kernel(SweepArgs args) {
 #pragma unroll
   for (int grp = 0; grp < 4; grp++) {
     const int da = grp >> 1, db = grp & 1;
-    const int la = 2 * pa + (o.swap ? db : da) - o.hA, lb = 2 * pb + (o.swap ? da : db) - o.hB;
-    live[grp] = la < lenA + o.hA && lb < lenB + o.hB;
+    const int la = 2 * pa + (o.swap ? db : da) - (sA ? o.hA : 0),
+              lb = 2 * pb + (o.swap ? da : db) - (sB ? o.hB : 0);
+    live[grp] = la < lenA + (sA ? 0 : o.hA) && lb < lenB + (sB ? 0 : o.hB);
     if (la >= 0 && la < lenA && lb >= 0 && lb < lenB) own |= 1u << grp;
     SweepRay& r = ray[grp];
     r = SweepRay{};
@@ -495,7 +502,7 @@ __global__ __launch_bounds__(1024) void art_sweep_kernel(SweepArgs args) {
     const int iD = sD ? layer : nD - 1 - layer;
     Layer l{cell * (float)(sD + iD), o.mD * (uint32_t)iD, 0, 0};
     auto start = [&](int first, double centre, double slope, int n) {
-      int v = first + (int)floor(centre + layer * slope) % n;
+      int v = first + (int)floor(centre + layer * slope + (slope > 0.0 ? -0.25 : 0.25)) % n;
       v += v < 0 ? n : (v >= n ? -n : 0);
       return __builtin_amdgcn_readfirstlane(v);
     };
@@ -842,34 +849,36 @@ ArtCtx a_;
   } while (0)
 
 // Tiles of art_sweep_kernel for layers of nA x nB cells: the split with the
-// fewest lanes over all tiles, of at most 1024 threads (four rays each) and
-// 64 KiB of LDS a block.  128 x 128: 5 tiles of 26 whole rows (17% more rays
-// than start cells); 256 x 256: 4 x 5 tiles of 64 x 52 (17%); up to 64 x 64
-// one tile.
-constexpr int kSweepThreads = 1024, kSweepCells = 4096;
+// fewest lanes over all tiles, of at most 512 threads (four rays each) and
+// 64 KiB of LDS a block; whole rows along B count for a tenth less, since their
+// lanes read and write long runs and need one place instead of two (128^3:
+// 6.4 ms per 256 directions with A whole, 5.7 with B whole).  128 x 128: 11
+// tiles of 12 rows, 256 x 256: 11 x 4 tiles of 24 x 64 (both 20% more lanes than
+// rays); up to 32 x 64 one tile.
+constexpr int kSweepThreads = 512, kSweepCells = 4096;
 void sweep_tiles(SweepOri& o) {
   int64_t best = 0;
   auto axis = [](int n, int t, int& r, int& h) {   // n cells in about t tiles
     r = t == 1 ? n : ((n + t - 1) / t + 1) & ~1;
     h = r < n ? 2 : 0;
-    return r == n || r + 4 <= n;
+    return r == n || r + h <= n;
   };
   for (int ta = 1; ta <= o.nA; ta++) {
     int rA, hA;
     if (!axis(o.nA, ta, rA, hA)) continue;
-    const int pA = (rA + 2 * hA) / 2;
+    const int pA = (rA + hA) / 2;
     for (int tb = 1; tb <= o.nB; tb++) {
       int rB, hB;
       if (!axis(o.nB, tb, rB, hB)) continue;
-      const int pB = (rB + 2 * hB) / 2;
+      const int pB = (rB + hB) / 2;
       if ((int64_t)pA * pB > kSweepThreads || (int64_t)rA * rB > kSweepCells) continue;
       const int cA = (o.nA + rA - 1) / rA, cB = (o.nB + rB - 1) / rB;
-      const int64_t lanes = (int64_t)cA * cB * ((pA * pB + 63) & ~63);
+      const int64_t lanes = (int64_t)cA * cB * ((pA * pB + 63) & ~63) * (cB == 1 ? 9 : 10);
       if (best == 0 || lanes <= best) {   // (of equals the longest runs along B)
         best = lanes;
         o.rA = rA; o.rB = rB; o.hA = hA; o.hB = hB; o.pA = pA; o.pB = pB; o.tA = cA; o.tB = cB;
       }
-      break;   // more tiles along B at this ta only add halo
+      break;   // more at this ta only add halo
     }
   }
 }
@@ -890,9 +899,31 @@ bool sweep_directions(const std::vector<ArtDir>& dirs) {
   return true;
 }
 
+// The order in which a batch's directions are swept: by base, then by crossings
+// a layer (1 + the slopes), most first.  Directions that go through the layers
+// alike and at one pace find more of one another's medium in the L2, and the
+// longest go first: 20.7 ms a pass at 128^3 instead of 21.9 in batch order.
+void sweep_order(std::vector<ArtDir>& dirs, int batch) {
+  auto crossings = [&](const ArtDir& d) {
+    const float* o = d.ovr;
+    return (fabsf(o[0]) + fabsf(o[1]) + fabsf(o[2])) /
+           std::max(fabsf(o[0]), std::max(fabsf(o[1]), fabsf(o[2])));
+  };
+  std::vector<int> ord;
+  for (size_t d0 = 0; d0 < dirs.size(); d0 += batch) {
+    ord.resize(std::min<size_t>(batch, dirs.size() - d0));
+    for (size_t i = 0; i < ord.size(); i++) ord[i] = (int)i;
+    std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) {
+      const ArtDir &p = dirs[d0 + a], &q = dirs[d0 + b];
+      return p.base != q.base ? p.base < q.base : crossings(p) > crossings(q);
+    });
+    for (size_t i = 0; i < ord.size(); i++) dirs[d0 + i].order = ord[i];
+  }
+}
+
 // Whether they hold for the box: cell indices in 32 bits, faces where the
 // cells end, and rays whose rounding (at most 3 crossings a layer, each within
-// 2 ulp of the largest coordinate) stays below half a cell of the halo's slack.
+// an ulp of the largest coordinate) stays below 0.2 cells.
 bool sweep_applies(const ArtGrid& g) {
   const double mn[3] = {g.xmin, g.ymin, g.zmin}, mx[3] = {g.xmax, g.ymax, g.zmax};
   const double d[3] = {g.dx, g.dy, g.dz};
@@ -902,9 +933,9 @@ bool sweep_applies(const ArtGrid& g) {
     if (!(d[k] > 1e-12 && d[k] < 1e6) || !(fabs(mx[k] - mn[k] - n[k] * d[k]) < 0.05 * d[k])) return false;
     big = std::max(big, std::max(fabs(mn[k]), fabs(mx[k])));
   }
-  const double err = 6.0 * ((double)g.nx + g.ny + g.nz) * big * 1.2e-7 / d[0];
+  const double err = 3.0 * std::max(g.nx, std::max(g.ny, g.nz)) * big * 1.2e-7 / d[0];
   const int64_t rows = std::max((int64_t)g.nx * g.ny, (int64_t)g.nx * g.nz);   // 24-bit products
-  return err < 0.5 && g.ncell <= ((int64_t)1 << 30) && std::max(rows, (int64_t)g.ny * g.nz) < (1 << 24);
+  return err < 0.2 && g.ncell <= ((int64_t)1 << 30) && std::max(rows, (int64_t)g.ny * g.nz) < (1 << 24);
 }
 
 double now_ms() {
@@ -1152,8 +1183,8 @@ void send_diffuse_data(struct host_diffuse_param* hd, struct cuda_diffuse_param*
       d.rcp[k] = 1.0 / (double)d.ovr[k];
       d.rcpf[k] = 1.0f / d.ovr[k];
     }
-    d.pad = 0.0f;
   }
+  sweep_order(a_.dirs, a_.batch);
   const step_func_factor* sf = hd->step_fact;
   const float f[6] = {sf->HI[0], sf->HI[1], sf->HeI[0], sf->HeI[1], sf->HeII[0], sf->HeII[1]};
   memcpy(a_.fact, f, sizeof f);

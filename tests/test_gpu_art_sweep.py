@@ -37,10 +37,10 @@ def box(shape, seed):
     return dataclasses.replace(w, **fields)
 
 
-# one tile of 4096 cells and just past it, tiles along one axis and both, a
-# last tile of two cells, the smallest even axes
+# one tile and just past it, tiles along either axis and both, short last
+# tiles, the smallest even axes
 @pytest.mark.parametrize("shape", [(64, 64, 2), (66, 66, 4), (4, 128, 66), (130, 6, 70),
-                                   (2, 2, 200), (68, 72, 96)])
+                                   (2, 2, 200), (68, 72, 96), (6, 4, 600), (40, 12, 300)])
 @pytest.mark.parametrize("exp64", [False, True])
 def test_tiled_sweep_matches_oracle(require_gpu, monkeypatch, shape, exp64):
     print(f"art sweep {shape} exp64={exp64}", flush=True)
@@ -62,7 +62,7 @@ def test_tiled_sweep_matches_oracle(require_gpu, monkeypatch, shape, exp64):
     compare(w, run_param, monkeypatch, g, 20, exp64)
 
 
-@pytest.mark.parametrize("lo", [500.0, 1000.0, -2000.0])   # below and above the sweep's bound
+@pytest.mark.parametrize("lo", [500.0, 1500.0, -4000.0])   # below and above the sweep's bound
 @pytest.mark.parametrize("exp64", [False, True])
 def test_far_box_matches_oracle(require_gpu, monkeypatch, lo, exp64):
     print(f"art far box {lo} exp64={exp64}", flush=True)
