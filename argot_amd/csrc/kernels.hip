@@ -1056,8 +1056,8 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY void fused_step_kernel(FusedArg
 // interior cell) and the results go straight back into prev_chem.  The floor is
 // passing over the records twice, whose rates lie in nearly every one of the
 // mesh's cache lines.  128^3: 65 us for the gather (5 TB/s) and 77 for the
-// rest; 65 + 90 + 69 with a scatter pass of its own and a thread per plane and
-// cell, 65 + 165 with a thread per cell that reads all its 162 neighbours.
+// rest, against 65 + 90 + 69 with a scatter pass of its own and a thread per
+// plane and cell.
 __global__ void gather_rates_kernel(const unsigned char* __restrict__ mesh, int64_t ncell,
                                     float* __restrict__ soa) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1068,9 +1068,11 @@ __global__ void gather_rates_kernel(const unsigned char* __restrict__ mesh, int6
 }
 
 // Blocks of consecutive (y, z) cells; a thread takes kSmoothX cells along x,
-// whose stencils share most of their rows (81 loads a cell instead of 162).
+// whose stencils share rows (108 loads a cell instead of 162).  A call on 128^3
+// cells takes 150, 144 and 146 us with 1, 2 and 4 cells a thread, on 16^3 20,
+// 20 and 22, where 4 are too long a chain.
 // out: the smoothed planes too, when the caller wants them (else null).
-constexpr int kSmoothX = 4;
+constexpr int kSmoothX = 2;
 __global__ __launch_bounds__(256) void smooth_rates_kernel(int nx, int ny, int nz, int x0,
                                                            const float* __restrict__ in,
                                                            unsigned char* __restrict__ mesh,

@@ -408,7 +408,7 @@ def chem_leg(step, dtime=1.0e-3):
            "cells_per_s": ncell / (cs["ms_kernel"] * 1e-3),
            "substeps": int(cs["nsub"]), "bisections": int(cs["niter"]),
            "substeps_per_s": cs["nsub"] / (cs["ms_kernel"] * 1e-3),
-           "heatcool_evals_per_s": cs["niter"] / (cs["ms_kernel"] * 1e-3),
+           "bisections_per_s": cs["niter"] / (cs["ms_kernel"] * 1e-3),
            "cells_stopped": int(cs["nstopped"]),
            "max_diff_chem": float(dc), "max_diff_uene": float(du)}
     log(f"chemistry: {out}")
