@@ -371,7 +371,7 @@ def rate_call_leg(step, rec):
            "ms_call": float(np.mean(walls[1:])), "ms_kernel": kms_,
            "rays_per_s_kernel": n / (kms_ * 1e-3),
            "rays_per_s_call": n / (np.mean(walls[1:]) * 1e-3),
-           "roofline": {"bound": "valu (FP32 frequency loop, 256 bins per ray)",
+           "roofline": {"bound": "valu (FP32 frequency integral)",
                         "achieved": bytes_ / (kms_ * 1e-3) / 1e9, "peak": HBM_PEAK_GBS,
                         "unit": "GB/s", "frac": bytes_ / (kms_ * 1e-3) / 1e9 / HBM_PEAK_GBS}}
     log(f"rate call: {out}")
