@@ -849,13 +849,13 @@ ArtCtx a_;
   } while (0)
 
 // Tiles of art_sweep_kernel for layers of nA x nB cells: the split with the
-// fewest lanes over all tiles, of at most 512 threads (four rays each) and
-// 64 KiB of LDS a block; whole rows along B count for a tenth less, since their
-// lanes read and write long runs and need one place instead of two (128^3:
-// 6.4 ms per 256 directions with A whole, 5.7 with B whole).  128 x 128: 11
-// tiles of 12 rows, 256 x 256: 11 x 4 tiles of 24 x 64 (both 20% more lanes than
-// rays); up to 32 x 64 one tile.
-constexpr int kSweepThreads = 512, kSweepCells = 4096;
+// fewest lanes over all tiles, of at most 512 threads a block (four rays each,
+// so at most 2048 cells or 32 KiB of LDS).  Whole rows along B count for a
+// tenth less, since their lanes read and write long runs and need one place
+// instead of two (128^3: 6.4 ms per 256 directions with A whole, 5.7 with B
+// whole).  128 x 128: 11 tiles of 12 rows, 256 x 256: 11 x 4 tiles of 24 x 64
+// (both 20% more lanes than rays); up to 32 x 64 one tile.
+constexpr int kSweepThreads = 512;
 void sweep_tiles(SweepOri& o) {
   int64_t best = 0;
   auto axis = [](int n, int t, int& r, int& h) {   // n cells in about t tiles
@@ -871,7 +871,7 @@ void sweep_tiles(SweepOri& o) {
       int rB, hB;
       if (!axis(o.nB, tb, rB, hB)) continue;
       const int pB = (rB + hB) / 2;
-      if ((int64_t)pA * pB > kSweepThreads || (int64_t)rA * rB > kSweepCells) continue;
+      if ((int64_t)pA * pB > kSweepThreads) continue;
       const int cA = (o.nA + rA - 1) / rA, cB = (o.nB + rB - 1) / rB;
       const int64_t lanes = (int64_t)cA * cB * ((pA * pB + 63) & ~63) * (cB == 1 ? 9 : 10);
       if (best == 0 || lanes <= best) {   // (of equals the longest runs along B)
