@@ -104,6 +104,8 @@ def lib():
     L.argot_hip_quotients.argtypes = 3 * [C.c_void_p] + [C.c_int64]
     L.argot_hip_rate_rule.argtypes = [rp, C.c_void_p, C.c_int] + 4 * [C.c_void_p]
     L.argot_hip_rate_rule.restype = C.c_int
+    L.argot_hip_rate_limits.argtypes = [C.c_void_p, rp, C.c_void_p, C.c_int, C.c_void_p,
+                                        C.c_void_p]
     L.argot_hip_tree_build.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_void_p,
                                        C.c_float]
     L.argot_hip_tree_build.restype = C.c_void_p

@@ -50,8 +50,9 @@ struct RateTables {
   // quadrature form (rate_rule.h): cross-sections at its nodes, and the
   // first-bin cross-sections that scale a ray against a spectrum's limit
   const float* qsig;   // [3*kRuleNodes] sigma_s, species-major
-  const float* qdsig;  // [3*kRuleNodes] sigma_s - sigma_s(last bin)
+  const float* qdsig;  // [3*kRuleNodes] sigma_s - sigma_s(last bin of the node's range)
   float edge[9];       // [range][species]
+  float end[3];        // sigma_HI at the end of range 1; sigma_HI, sigma_HeI at the end of range 2
 };
 
 // Source tree in depth-first pre-order (children in octant order), as
@@ -70,7 +71,7 @@ struct TreeDev {
   const float* spec;         // [nnode*ngrid] spectrum / spec_scale, FP32
   const double* spec_scale;  // [nnode] max over bins of the spectrum
   const float* weight;       // [nnode*kRuleWeights] quadrature weights of spec (rate_rule.h)
-  const float* limit;        // [nnode] thickest ray the quadrature serves (0: none)
+  const float* limit;        // [nnode*kRuleLimits] thickest rays the quadrature serves (0: none)
   const float* src_pos;      // [4*nsrc]
 };
 

@@ -38,14 +38,15 @@ hipError_t launch_walk_segments(const GridDev& g, const float4* nf, void* seg, i
 // crossing (no packed-field buffer; identical optical depths).
 hipError_t launch_walk_segments_mesh(const GridDev& g, const void* mesh, double helium_fact,
                                      void* seg, int64_t nseg, int kahan, hipStream_t s);
-// The quadrature rule's matrices on the device (rate_rule.h).
+// The quadrature rule on the device (rate_rule.h).
 struct RuleDev {
   int usable;
   int start[4];
-  const double* project;   // [ngrid][kRuleW3]
-  const float* test;       // [ngrid][kRuleTests][2]
+  const double* lag;       // [ngrid][kRuleN3]
+  const float* rate;       // [6][ngrid]
+  const float* test;       // by range: [bins][rule_columns][2]
 };
-// Quadrature weights [nspec * kRuleWeights] and limits [nspec] of spectra
+// Quadrature weights [nspec * kRuleWeights] and limits [nspec * kRuleLimits] of spectra
 // [nspec * ngrid].
 hipError_t launch_project_spectra(const RuleDev& rule, const float* spec, int nspec, int ngrid,
                                   float* weight, float* limit, hipStream_t s);
@@ -55,7 +56,7 @@ struct CallSpectra {
   const double* spec64;    // [nspec * ngrid] as given
   const double* scale;     // [nspec] the spectrum's maximum
   const float* weight;     // quadrature weights of spec32, and
-  const float* limit;      // the thickest ray they serve
+  const float* limit;      // the thickest rays they serve
 };
 // calc_photoion_rate_cuda: ntarget targets, each with its consecutive rays
 // (rays[first .. first + count)), rates added to the mesh's prev_chem.

@@ -353,14 +353,17 @@ typedef float F4 __attribute__((ext_vector_type(4)));
 // Nodes [o, o + N) of the quadrature form for one bin range with NS active
 // species: the same f as the bin loops above (thin form, and in MIXED
 // wavefronts the direct form by lane and node), at the range's nodes, summed
-// with the spectrum's weight rows G_s, H_s.  w(i): the i-th four weights of
-// the range; cl: -log2(e) times the range's constant optical depth.
+// with the spectrum's weight rows G_s, H_s into g, h.  w(i): the i-th four
+// weights of the range.  The optical depths are those beyond the depth at the range's last
+// bin, whose attenuation the caller puts in: the sums come from there, and what FP32
+// rounds off an optical depth is relative to its size.  (Taken beyond the depth
+// at the last bin of all, a ray of 100 at the HI edge has 25 at the end of the
+// first range and its rates errors of 2e-6, as large as the bin loops'.)
 template <int NS, int N, bool MIXED, typename WeightF>
-__device__ __forceinline__ void rate_nodes(const RateTables& rt, int o, float cl,
-                                           const float nl[3], const float dl[3], bool thin,
-                                           WeightF w, double G[3], double H[3]) {
+__device__ __forceinline__ void rate_nodes(const RateTables& rt, int o, const float nl[3],
+                                           const float dl[3], bool thin, WeightF w, float g[NS],
+                                           float h[NS]) {
   constexpr float kHalfLog2eN = -0.5f * kLog2e;
-  float g[NS], h[NS];
 #pragma unroll
   for (int s = 0; s < NS; s++) g[s] = h[s] = 0.0f;
 #pragma unroll 1
@@ -378,12 +381,12 @@ __device__ __forceinline__ void rate_nodes(const RateTables& rt, int o, float cl
       float yl = 0.0f;
 #pragma unroll
       for (int s = 0; s < NS; s++) yl = __builtin_fmaf(dl[s], sg[s][i], yl);
-      float z = NS < 3 ? yl + cl : yl;
+      float z = yl;
 #pragma unroll
       for (int s = 0; s < NS; s++) z = __builtin_fmaf(nl[s], ds[s][i], z);
       float f = __builtin_amdgcn_exp2f(z) * sinhc_l(yl);
       if constexpr (MIXED) {
-        float zt = cl;
+        float zt = 0.0f;
 #pragma unroll
         for (int s = 0; s < NS; s++) zt = __builtin_fmaf(nl[s], ds[s][i], zt);
         const float om = 1.0f - __builtin_amdgcn_exp2f(yl + yl);
@@ -398,22 +401,54 @@ __device__ __forceinline__ void rate_nodes(const RateTables& rt, int o, float cl
       }
     }
   }
-#pragma unroll
-  for (int s = 0; s < NS; s++) {
-    G[s] += g[s];
-    H[s] += h[s];
-  }
 }
 
-template <bool MIXED, typename WeightF>
-__device__ __forceinline__ void rate_all_nodes(const RateTables& rt, float cl1, float cl2,
-                                               const float nl[3], const float dl[3], bool thin,
-                                               WeightF w, double G[3], double H[3]) {
-  rate_nodes<1, kRuleN1, MIXED>(rt, 0, cl1, nl, dl, thin, w, G, H);
-  rate_nodes<2, kRuleN2, MIXED>(rt, kRuleN1, cl2, nl, dl, thin,
-                                [&](int i) { return w(kRuleW1 / 4 + i); }, G, H);
-  rate_nodes<3, kRuleN3, MIXED>(rt, kRuleN1 + kRuleN2, 0.0f, nl, dl, thin,
-                                [&](int i) { return w((kRuleW1 + kRuleW2) / 4 + i); }, G, H);
+// exp(x) 2^e as 2^n 2^f, n = floor(x log2 e) and f in [0, 1): the FP32
+// exponential of f (relative error about 1e-7) times an exact power of two, in
+// FP64 range.  The library exponential's polynomial would hold a dozen FP64
+// constants in registers across the kernel, which the register budget spills.
+// (fast_rate_ok bounds x above.)
+__device__ __forceinline__ double exp_scaled(double x, int e) {
+  constexpr double kLog2eD = 1.4426950408889634;
+  const double xl = x * kLog2eD;
+  const double fl = fmax(floor(xl), -2000.0);
+  return ldexp((double)__builtin_amdgcn_exp2f((float)(xl - fl)), (int)fl + e);
+}
+
+// One range of the frequency integral: by N nodes from node o on, or bin by bin.
+// unit: the nodes' unit in that of G, H.  loose: the nodes serve only if their sums
+// are at most kRuleShare of G[0], H[0] (else they are dropped for the bins).
+template <int NS, int N, bool FOLD, typename SpecF, typename WeightF>
+__device__ __forceinline__ void rate_range(const RateTables& rt, bool nodes, bool loose,
+                                           bool all_thin, int k0, int k1, int o, double unit,
+                                           float cst, const float n[3], const float nl[3],
+                                           const float dl[3], bool thin, SpecF spec, WeightF w,
+                                           double G[3], double H[3]) {
+  if (nodes) {
+    float g[NS], h[NS];
+    if (all_thin)
+      rate_nodes<NS, N, false>(rt, o, nl, dl, thin, w, g, h);
+    else
+      rate_nodes<NS, N, true>(rt, o, nl, dl, thin, w, g, h);
+    const double g0 = (double)g[0] * unit, h0 = (double)h[0] * unit;
+    if (NS == 1 && loose && !(g0 <= kRuleShare * G[0] && h0 <= kRuleShare * H[0])) {
+      nodes = false;
+    } else {
+      G[0] += g0;
+      H[0] += h0;
+#pragma unroll
+      for (int s = 1; s < NS; s++) {
+        G[s] = __builtin_fma((double)g[s], unit, G[s]);
+        H[s] = __builtin_fma((double)h[s], unit, H[s]);
+      }
+    }
+  }
+  if (!nodes) {
+    if (all_thin)
+      rate_bins_thin<NS, FOLD>(rt, k0, k1, cst, n, nl, dl, spec, G, H);
+    else
+      rate_bins_mixed<NS, FOLD>(rt, k0, k1, cst, n, nl, dl, thin, spec, G, H);
+  }
 }
 
 // FP32 frequency integral (photon-conserving form, calc_photoion_rate.c:327-386
@@ -422,22 +457,23 @@ __device__ __forceinline__ void rate_all_nodes(const RateTables& rt, float cl1, 
 // The optical depth is shifted by its last-bin value tsh (folded back in
 // FP64): tau_k - tsh = sum_s N_s (sigma_s(k) - sigma_s(last)).  Bins below
 // the HeI and HeII edges skip the absent species.
-// A ray within its spectrum's limit takes the sums as quadratures over the
-// rule's 44 nodes (rate_rule.cpp), any other ray bin by bin; which one
-// depends on the ray alone, not on its wavefront.
-template <typename SpecF, typename WeightF>
+// In a range within whose limit of its spectrum it lies a ray takes the sums as
+// quadratures over the range's nodes (rate_rule.cpp), in any other bin by bin;
+// which one depends on the ray alone, not on its wavefront.  limit(i): the
+// spectrum's limits (kRuleLimits).
+template <typename LimitF, typename SpecF, typename WeightF>
 __device__ inline void rate_loop_f32(const RateTables& rt, const RayRate& rr, double scale,
-                                     float limit, SpecF spec, WeightF weight, double out[6]) {
+                                     LimitF limit, SpecF spec, WeightF weight, double out[6]) {
   const double sh2 = rr.t[2] * rt.cs_last[2];
   const double sh1 = __builtin_fma(rr.t[1], rt.cs_last[1], sh2);
   const double tsh = __builtin_fma(rr.t[0], rt.cs_last[0], sh1);
   const float n[3] = {(float)rr.t[0], (float)rr.t[1], (float)rr.t[2]};
   const float c1 = (float)-sh1;
   const float c2 = (float)-sh2;
-  // Scale of the ray against the rule's test columns, from its columns at the
-  // far side of the cell (and, where the half-cell shift made one
-  // negative, its negative part).
-  float lam = 0.0f, neg = 0.0f;
+  // Scale of the ray against the rule's test columns in each range, from its
+  // columns at the far side of the cell (and, where the half-cell shift made
+  // one negative, its negative part).
+  bool nodes[3], loose = false;   // loose: the first range's nodes, for a small share
   {
     float tf[3], tn[3];
 #pragma unroll
@@ -453,23 +489,14 @@ __device__ inline void rate_loop_f32(const RateTables& rt, const RayRate& rr, do
         e = __builtin_fmaf(fabsf(tf[s]), rt.edge[3 * g + s], e);
         m = __builtin_fmaf(tn[s], rt.edge[3 * g + s], m);
       }
-      lam = fmaxf(lam, e);
-      neg = fmaxf(neg, m);
+      const float top = limit(g);
+      nodes[g] = e <= top && m <= kRuleNegative && top > 0.0f;
+      if (g == 0) loose = !nodes[0] && e <= limit(3) && m <= kRuleNegative && limit(3) > 0.0f;
     }
   }
-  const bool nodes = lam <= limit && neg <= kRuleNegative && limit > 0.0f;
   // per-ray prefactors first (same operations as after the loop), so that
   // only they, not the ray's FP64 quantities, stay live through the bins
-  // exp(-tsh) as 2^n 2^f, n = floor(-tsh log2 e) and f in [0, 1): the FP32
-  // exponential of f (relative error about 1e-7, below the loop's own) times
-  // an exact power of two, in FP64 range.  The library exponential's
-  // polynomial would hold a dozen FP64 constants in registers across the
-  // kernel, which the register budget spills.
-  constexpr double kLog2eP = 1.4426950408889634;
-  const double xl = -tsh * kLog2eP;
-  const double fl = fmax(floor(xl), -2000.0);
-  const double pre =
-      scale * ldexp((double)__builtin_amdgcn_exp2f((float)(xl - fl)), (int)fl);
+  const double pre = scale * exp_scaled(-tsh, 0);
   const double p0 = rcp_f64(rr.v[0]) * rr.d[0] * pre;
   const double p1 = rcp_f64(rr.v[1]) * rr.d[1] * pre;
   const double p2 = rcp_f64(rr.v[2]) * rr.d[2] * pre;
@@ -488,26 +515,19 @@ __device__ inline void rate_loop_f32(const RateTables& rt, const RayRate& rr, do
   const float nl[3] = {(float)(rr.t[0] * -kLog2eD), (float)(rr.t[1] * -kLog2eD),
                        (float)(rr.t[2] * -kLog2eD)};
   const bool thin = dmax <= (float)kThinMax;
-  if (nodes) {
-    const float cl1 = c1 * -kLog2e, cl2 = c2 * -kLog2e;
-    if (__all(thin))
-      rate_all_nodes<false>(rt, cl1, cl2, nl, dl, thin, weight, G, H);
-    else
-      rate_all_nodes<true>(rt, cl1, cl2, nl, dl, thin, weight, G, H);
-#pragma unroll
-    for (int s = 0; s < 3; s++) {
-      G[s] *= 1.0 / kRuleScale;
-      H[s] *= 1.0 / kRuleScale;
-    }
-  } else if (__all(thin)) {
-    rate_bins_thin<1, false>(rt, 0, rt.k_he1, c1, n, nl, dl, spec, G, H);
-    rate_bins_thin<2, false>(rt, rt.k_he1, rt.k_he2, c2, n, nl, dl, spec, G, H);
-    rate_bins_thin<3, true>(rt, rt.k_he2, rt.ngrid, 0.0f, n, nl, dl, spec, G, H);
-  } else {
-    rate_bins_mixed<1, false>(rt, 0, rt.k_he1, c1, n, nl, dl, thin, spec, G, H);
-    rate_bins_mixed<2, false>(rt, rt.k_he1, rt.k_he2, c2, n, nl, dl, thin, spec, G, H);
-    rate_bins_mixed<3, true>(rt, rt.k_he2, rt.ngrid, 0.0f, n, nl, dl, thin, spec, G, H);
-  }
+  const bool all_thin = __all(thin);
+  // (the sums are in units of exp(-tsh), the nodes' weights in those of kRuleScale)
+  const double unit1 = exp_scaled(tsh - rr.t[0] * rt.end[0], -kRuleExponent);
+  const double unit2 = exp_scaled(
+      tsh - __builtin_fma(rr.t[0], rt.end[1], rr.t[1] * rt.end[2]), -kRuleExponent);
+  rate_range<3, kRuleN3, true>(rt, nodes[2], false, all_thin, rt.k_he2, rt.ngrid, kRuleN1 + kRuleN2,
+                               1.0 / kRuleScale, 0.0f, n, nl, dl, thin, spec,
+                               [&](int i) { return weight((kRuleW1 + kRuleW2) / 4 + i); }, G, H);
+  rate_range<2, kRuleN2, false>(rt, nodes[1], false, all_thin, rt.k_he1, rt.k_he2, kRuleN1, unit2,
+                                c2, n, nl, dl, thin, spec,
+                                [&](int i) { return weight(kRuleW1 / 4 + i); }, G, H);
+  rate_range<1, kRuleN1, false>(rt, nodes[0] || loose, loose, all_thin, 0, rt.k_he1, 0, unit1, c1,
+                                n, nl, dl, thin, spec, weight, G, H);
   out[0] = p0 * G[0];
   out[1] = p0 * H[0] * kHnuL;
   out[2] = p1 * G[1];
@@ -517,70 +537,106 @@ __device__ inline void rate_loop_f32(const RateTables& rt, const RayRate& rr, do
 }
 
 // Quadrature weights and limits of nspec spectra (rows of ngrid floats,
-// scaled to their maximum): the rule's projection matrices times the
-// spectrum.  A block takes NB spectra, so that each matrix entry it reads
-// serves NB of them; 448 threads, one per weight (192) and per test column and
-// rate (210).
-constexpr int kProjectThreads = 448;
-static_assert(kRuleWeights + kRuleTests <= kProjectThreads, "one thread per output");
+// scaled to their maximum): a thread per weight (192) and per test (560), a
+// wavefront's all of one range, so that its loop has uniform bounds and eight of
+// its loads in flight: the chain of loads over the 153 bins of the last range is
+// what a launch on few spectra takes (23 us on the tree of 16 sources; with bounds
+// that differ between lanes, and loads waited for one by one, 50).  A block takes NB
+// spectra, so that each entry it reads of the rule's tables serves NB of them.
+// first thread of each kind: weights by range, then tests by range
+constexpr int wave_up(int n) { return (n + 63) & ~63; }
+constexpr int kAtW2 = wave_up(kRuleW1), kAtW3 = kAtW2 + wave_up(kRuleW2),
+              kAtT1 = kAtW3 + wave_up(kRuleW3), kAtT2 = kAtT1 + wave_up(rule_tests(0)),
+              kAtT3 = kAtT2 + wave_up(rule_tests(1)),
+              kProjectThreads = kAtT3 + wave_up(rule_tests(2));
+static_assert(kProjectThreads <= 1024, "one block");
 template <int NB>
 __global__ __launch_bounds__(kProjectThreads) void project_spectra_kernel(
     RuleDev rule, const float* __restrict__ spec, int nspec, int ngrid,
     float* __restrict__ weight, float* __restrict__ limit) {
   __shared__ float sp[kNgridMax][NB];
-  __shared__ unsigned fail[NB];
+  __shared__ float rate[6][kNgridMax + 1];   // (rows in different banks)
+  __shared__ unsigned fail[kRuleLimits * NB];
   const int t = threadIdx.x;
   const int u0 = blockIdx.x * NB;
   for (int i = t; i < NB * ngrid; i += kProjectThreads) {
     const int j = i / ngrid, k = i % ngrid;
     sp[k][j] = u0 + j < nspec ? spec[(int64_t)(u0 + j) * ngrid + k] : 0.0f;
   }
-  if (t < NB) fail[t] = 0u;
+  if (rule.usable)
+    for (int i = t; i < 6 * ngrid; i += kProjectThreads) rate[i / ngrid][i % ngrid] = rule.rate[i];
+  if (t < kRuleLimits * NB) fail[t] = 0u;
   __syncthreads();
-  if (t < kRuleWeights) {
-    const int g = t < kRuleW1 ? 0 : t < kRuleW1 + kRuleW2 ? 1 : 2;
-    const int o = t - (g == 0 ? 0 : g == 1 ? kRuleW1 : kRuleW1 + kRuleW2);
+  const int wave = __builtin_amdgcn_readfirstlane(t) & ~63;   // its first thread
+  if (wave < kAtT1) {
+    const int g = wave < kAtW2 ? 0 : wave < kAtW3 ? 1 : 2;
+    const int o = t - (g == 0 ? 0 : g == 1 ? kAtW2 : kAtW3);
+    const int nn = g == 0 ? kRuleN1 : g == 1 ? kRuleN2 : kRuleN3;
+    const int row = min(o / nn, 2 * g + 1), node = o % nn;   // (lanes beyond the rows: the last)
+    const double* __restrict__ lag = rule.lag + node;
     double w[NB];
 #pragma unroll
     for (int j = 0; j < NB; j++) w[j] = 0.0;
-#pragma unroll 8
-    for (int k = rule.start[g]; k < rule.start[g + 1]; k++) {
-      const double m = rule.project[(int64_t)k * kRuleW3 + o];
+    const int first = rule.start[g], last = rule.start[g + 1];
+    constexpr int kAhead = NB > 4 ? 2 : 8;   // (more spill where a block holds many sums)
+    for (int k0 = first; k0 < last; k0 += kAhead) {
+      double l[kAhead];
 #pragma unroll
-      for (int j = 0; j < NB; j++) w[j] += (double)sp[k][j] * m;
+      for (int i = 0; i < kAhead; i++) l[i] = lag[min(k0 + i, last - 1) * kRuleN3];
+      __builtin_amdgcn_sched_barrier(0);   // (the loads go out together)
+#pragma unroll
+      for (int i = 0; i < kAhead; i++) {
+        const int k = min(k0 + i, last - 1);
+        const double m = k0 + i < last ? (double)rate[row][k] * l[i] : 0.0;
+#pragma unroll
+        for (int j = 0; j < NB; j++) w[j] += (double)sp[k][j] * m;
+      }
     }
+    const int at = g == 0 ? 0 : g == 1 ? kRuleW1 : kRuleW1 + kRuleW2;
 #pragma unroll
     for (int j = 0; j < NB; j++)
-      if (u0 + j < nspec) weight[(int64_t)(u0 + j) * kRuleWeights + t] = (float)w[j];
-  } else if (t < kRuleWeights + kRuleTests) {
-    const int c = t - kRuleWeights;
+      if (u0 + j < nspec && o < 2 * (g + 1) * nn)
+        weight[(int64_t)(u0 + j) * kRuleWeights + at + o] = (float)w[j];
+  } else if (rule.usable) {
+    const int g = wave < kAtT2 ? 0 : wave < kAtT3 ? 1 : 2;
+    const int q = t - (g == 0 ? kAtT1 : g == 1 ? kAtT2 : kAtT3);
+    const int ncol = g == 2 ? rule_columns(2) : g == 1 ? rule_columns(1) : rule_columns(0);
+    const int mixes = g == 2 ? kRuleMixes[2] : g == 1 ? kRuleMixes[1] : kRuleMixes[0];
+    const int c = min(q / (2 * (g + 1)), ncol - 1);   // (lanes beyond the tests repeat one)
+    const int row = q % (2 * (g + 1));
+    const int first = rule.start[g], last = rule.start[g + 1];
+    const float2* __restrict__ f =
+        reinterpret_cast<const float2*>(rule.test) + c +
+        (g > 0 ? (rule.start[1] - rule.start[0]) * rule_columns(0) : 0) +
+        (g > 1 ? (rule.start[2] - rule.start[1]) * rule_columns(1) : 0);
     float sum[NB], err[NB];
 #pragma unroll
     for (int j = 0; j < NB; j++) sum[j] = err[j] = 0.0f;
 #pragma unroll 8
-    for (int k = 0; k < ngrid; k++) {
-      const float2 m = reinterpret_cast<const float2*>(rule.test)[(int64_t)k * kRuleTests + c];
+    for (int k = first; k < last; k++) {
+      const float2 m = f[(k - first) * ncol];
+      const float r = rate[row][k];
 #pragma unroll
       for (int j = 0; j < NB; j++) {
-        sum[j] = __builtin_fmaf(sp[k][j], m.x, sum[j]);
-        err[j] = __builtin_fmaf(sp[k][j], m.y, err[j]);
+        const float v = sp[k][j] * r;
+        sum[j] = __builtin_fmaf(v, m.x, sum[j]);
+        err[j] = __builtin_fmaf(v, m.y, err[j]);
       }
     }
-    const int level = c / 6 / kRuleMixes;
+    const int level = c / mixes;
 #pragma unroll
-    for (int j = 0; j < NB; j++)
-      if (!(fabsf(err[j]) <= kRuleTol * sum[j]))
-        atomicOr(&fail[j], 1u << (level < kRuleLevels ? level : 0));
+    for (int j = 0; j < NB; j++) {
+      if (!(fabsf(err[j]) <= kRuleTol * sum[j])) atomicOr(&fail[kRuleLimits * j + g], 1u << level);
+      if (g == 0 && !(fabsf(err[j]) <= kRuleLoose * sum[j]))
+        atomicOr(&fail[kRuleLimits * j + 3], 1u << level);
+    }
   }
   __syncthreads();
-  if (t < NB && u0 + t < nspec) {
-    constexpr float kLevel[kRuleLevels] = {0.2f, 0.4f, 0.7f, 1.0f, 1.7f, 3.0f};
+  if (t < kRuleLimits * NB && u0 + t / kRuleLimits < nspec) {
     const unsigned f = rule.usable ? fail[t] : 1u;
-    float lim = 0.0f;
-#pragma unroll
-    for (int l = kRuleLevels - 1; l >= 0; l--)
-      if ((f & ((2u << l) - 1u)) == 0u && lim == 0.0f) lim = kLevel[l];
-    limit[u0 + t] = lim;
+    const int g = t % kRuleLimits;
+    const float lim[3] = {rule_limit(0, f), rule_limit(1, f), rule_limit(2, f)};
+    limit[(int64_t)kRuleLimits * u0 + t] = g == 1 ? lim[1] : g == 2 ? lim[2] : lim[0];
   }
 }
 
@@ -689,7 +745,8 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY void target_rates_kernel(
     if (more && !wide) {
       const float* s32 = sp.spec32 + (int64_t)u * ng;
       const F4* w = reinterpret_cast<const F4*>(sp.weight + (int64_t)u * kRuleWeights);
-      rate_loop_f32(rt, rr, sp.scale[u], sp.limit[u], [&](int k) { return s32[k]; },
+      rate_loop_f32(rt, rr, sp.scale[u], [&](int k) { return sp.limit[kRuleLimits * (int64_t)u + k]; },
+                    [&](int k) { return s32[k]; },
                     [&](int i) { return w[i]; }, res);
     }
     if (more) {
@@ -999,7 +1056,8 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY void fused_step_kernel(FusedArg
       if (wide) my_fb++;
       if (exact && !wide) {
         const F4* wt = reinterpret_cast<const F4*>(tr.weight + (int64_t)u * kRuleWeights);
-        rate_loop_f32(rt, rr, sc, ldc(tr.limit + u), [&](int k) { return ldc(sp + k); },
+        rate_loop_f32(rt, rr, sc, [&](int k) { return ldc(tr.limit + kRuleLimits * u + k); },
+                      [&](int k) { return ldc(sp + k); },
                       [&](int i) { return ldc(wt + i); }, res);
       }
       const int nth = CAPTURE ? __shfl(seq, t, 64) : 0;

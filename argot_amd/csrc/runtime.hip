@@ -183,7 +183,7 @@ struct Ctx {
   DevBuf<float> weight;
   RuleDev rule{};
   const float *qsig = nullptr, *qdsig = nullptr;
-  float edge[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  float edge[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, end[3] = {0, 0, 0};
   // tree
   DevBuf<unsigned char> tree_buf;   // links, centres, spectra, their scales, source positions
   PinBuf tree_stage;
@@ -331,6 +331,7 @@ RateTables rate_tables(const Ctx& g) {
   t.qsig = g.qsig;
   t.qdsig = g.qdsig;
   memcpy(t.edge, g.edge, sizeof t.edge);
+  memcpy(t.end, g.end, sizeof t.end);
   return t;
 }
 
@@ -422,20 +423,23 @@ void upload_tables(Ctx& g, const run_param* r) {
   g.rule.usable = rule.usable ? 1 : 0;
   for (int k = 0; k < 4; k++) g.rule.start[k] = rule.usable ? rule.start[k] : 0;
   memcpy(g.edge, rule.edge, sizeof g.edge);
-  // project (double), then test, sig and dsig (float; sizes multiples of 4)
-  const size_t np = rule.project.size(), nt = rule.test.size(), ns = rule.sig.size();
-  std::vector<double> buf(np + (nt + 2 * ns) / 2);
-  std::copy(rule.project.begin(), rule.project.end(), buf.begin());
-  float* const f = reinterpret_cast<float*>(buf.data() + np);
-  std::copy(rule.test.begin(), rule.test.end(), f);
-  std::copy(rule.sig.begin(), rule.sig.end(), f + nt);
-  std::copy(rule.dsig.begin(), rule.dsig.end(), f + nt + ns);
+  memcpy(g.end, rule.end, sizeof g.end);
+  // lag (double), then sig, dsig, rate and test (float; even numbers of them)
+  const size_t nl = rule.lag.size(), ns = rule.sig.size(), nr = rule.rate.size();
+  std::vector<double> buf(nl + (2 * ns + nr + rule.test.size()) / 2);
+  std::copy(rule.lag.begin(), rule.lag.end(), buf.begin());
+  float* const f = reinterpret_cast<float*>(buf.data() + nl);
+  std::copy(rule.sig.begin(), rule.sig.end(), f);
+  std::copy(rule.dsig.begin(), rule.dsig.end(), f + ns);
+  std::copy(rule.rate.begin(), rule.rate.end(), f + 2 * ns);
+  std::copy(rule.test.begin(), rule.test.end(), f + 2 * ns + nr);
   HIP_OK(g.rule_buf.reserve(buf.size()));
   HIP_OK(hipMemcpy(g.rule_buf.p, buf.data(), buf.size() * sizeof(double), hipMemcpyHostToDevice));
-  g.rule.project = g.rule_buf.p;
-  g.rule.test = reinterpret_cast<const float*>(g.rule_buf.p + np);
-  g.qsig = g.rule.test + nt;
+  g.rule.lag = g.rule_buf.p;
+  g.qsig = reinterpret_cast<const float*>(g.rule_buf.p + nl);
   g.qdsig = g.qsig + ns;
+  g.rule.rate = g.qdsig + ns;
+  g.rule.test = g.rule.rate + nr;
 }
 
 // The caller's context, ready and for a mesh of this_run's size, or null
@@ -1077,7 +1081,7 @@ static void calc_photoion_rate_cuda_body(struct cuda_mem_space* cuda_mem, struct
   HIP_OK(hipMemcpyAsync(d, stage, off_tab, hipMemcpyHostToDevice, g.stream));
   HIP_OK(hipMemcpyAsync(d + off_tab, tab, tab_bytes, hipMemcpyHostToDevice, g.stream));
   const RateTables rt = rate_tables(g);
-  HIP_OK(g.weight.reserve((size_t)nspec * (kRuleWeights + 1)));
+  HIP_OK(g.weight.reserve((size_t)nspec * (kRuleWeights + kRuleLimits)));
   float* const limit = g.weight.p + (size_t)nspec * kRuleWeights;
   const CallSpectra spectra{
       reinterpret_cast<const float*>(d + off_tab),
@@ -1272,7 +1276,7 @@ static void point_source_pass(Ctx& g, struct radiation_src* src, struct run_para
   const float* const spec32 = reinterpret_cast<const float*>(tree + at_spec);
   const double t_built = now_ms();
   // Every spectrum's quadrature weights, on the stream before the fused kernel.
-  HIP_OK(g.weight.reserve((size_t)nn * (kRuleWeights + 1)));
+  HIP_OK(g.weight.reserve((size_t)nn * (kRuleWeights + kRuleLimits)));
   float* const limit = g.weight.p + (size_t)nn * kRuleWeights;
   HIP_OK(launch_project_spectra(g.rule, spec32, nn, ARGOT_NGRID_NU, g.weight.p, limit,
                                 g.stream));
@@ -1778,8 +1782,9 @@ void argot_hip_quotients(const float* a, const float* b, float* q, int64_t n) {
 
 // The quadrature rule of run_param's tables on the host: cross-sections
 // sigma_s and sigma_s - sigma_s(last) at its nodes [3 * 44 each], and the
-// weights [nspec * 192] and limits [nspec] of FP32 spectra [nspec * 256].
-// Returns the number of nodes, 0 where the tables have no rule.
+// weights [nspec * 192] and limits [nspec] (the smallest of the three ranges')
+// of FP32 spectra [nspec * 256].  Returns the number of nodes, 0 where the
+// tables have no rule.
 int argot_hip_rate_rule(const struct run_param* r, const float* spec, int nspec, float* sig,
                         float* dsig, float* weight, float* limit) {
   try {
@@ -1787,13 +1792,56 @@ int argot_hip_rate_rule(const struct run_param* r, const float* spec, int nspec,
     RateRule rule;
     build_rate_rule(t.sig.data(), t.hsig.data(), ARGOT_NGRID_NU, t.k_he1, t.k_he2, &rule);
     memcpy(sig, rule.sig.data(), sizeof(float) * rule.sig.size());
-    memcpy(dsig, rule.dsig.data(), sizeof(float) * rule.dsig.size());
-    project_spectra_host(rule, spec, nspec, ARGOT_NGRID_NU, weight, limit);
+    for (int i = 0; i < 3 * kRuleNodes; i++)
+      dsig[i] = rule.node[i] > 0.0
+                    ? (float)(rule.node[i] - (double)t.sig[(i / kRuleNodes + 1) * ARGOT_NGRID_NU - 1])
+                    : 0.0f;
+    std::vector<float> lim(kRuleLimits * (size_t)nspec);
+    project_spectra_host(rule, spec, nspec, ARGOT_NGRID_NU, weight, lim.data());
+    for (int u = 0; u < nspec; u++)
+      limit[u] = *std::min_element(&lim[kRuleLimits * u], &lim[kRuleLimits * u] + 3);
     return rule.usable ? kRuleNodes : 0;
   } catch (const std::bad_alloc&) {
     set_err(ARGOT_ERR_NOMEM);
   }
   return 0;
+}
+
+// Weights [nspec * 192] and limits [nspec * 4] (rate_rule.h) that the rule of
+// run_param's tables gives FP32 spectra [nspec * 256]: formed on the host where
+// cuda_mem is null, else by the context's kernel and its tables.
+static void argot_hip_rate_limits_body(struct cuda_mem_space* cuda_mem, const struct run_param* r,
+                                       const float* spec, int nspec, float* weight,
+                                       float* limits) {
+  if (!cuda_mem) {
+    const HostTables t = host_tables(r);
+    RateRule rule;
+    build_rate_rule(t.sig.data(), t.hsig.data(), ARGOT_NGRID_NU, t.k_he1, t.k_he2, &rule);
+    return project_spectra_host(rule, spec, nspec, ARGOT_NGRID_NU, weight, limits);
+  }
+  Ctx* const cp = find_ctx(cuda_mem);
+  if (!cp || !cp->ready) return set_err(ARGOT_ERR_STATE);
+  Ctx& g = *cp;
+  const size_t ns = (size_t)nspec * ARGOT_NGRID_NU, nw = (size_t)nspec * kRuleWeights;
+  HIP_OK(g.weight.reserve(ns + nw + kRuleLimits * (size_t)nspec));
+  float* const w = g.weight.p + ns;
+  HIP_OK(hipMemcpyAsync(g.weight.p, spec, sizeof(float) * ns, hipMemcpyHostToDevice, g.stream));
+  HIP_OK(launch_project_spectra(g.rule, g.weight.p, nspec, ARGOT_NGRID_NU, w, w + nw, g.stream));
+  HIP_OK(hipMemcpyAsync(weight, w, sizeof(float) * nw, hipMemcpyDeviceToHost, g.stream));
+  HIP_OK(hipMemcpyAsync(limits, w + nw, sizeof(float) * kRuleLimits * nspec, hipMemcpyDeviceToHost,
+                        g.stream));
+  HIP_OK(hipStreamSynchronize(g.stream));
+}
+
+void argot_hip_rate_limits(struct cuda_mem_space* cuda_mem, const struct run_param* r,
+                           const float* spec, int nspec, float* weight, float* limits) {
+  t_err = ARGOT_OK;
+  if (nspec <= 0 || !spec || !weight || !limits || (!cuda_mem && !r)) return set_err(ARGOT_ERR_ARG);
+  try {
+    argot_hip_rate_limits_body(cuda_mem, r, spec, nspec, weight, limits);
+  } catch (const std::bad_alloc&) {
+    set_err(ARGOT_ERR_NOMEM);
+  }
 }
 
 // Product tree on the host: build from nsrc sources and list the rays of a
