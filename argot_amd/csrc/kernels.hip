@@ -234,6 +234,25 @@ __device__ __forceinline__ float sinhc_l(float yl) {
   p = __builtin_fmaf(u, p, kSh1);
   return __builtin_fmaf(u, p, kSh0);
 }
+// The same of degree 5 for the quadrature's nodes (minimax relative error
+// 3.3e-9).  44 nodes average their roundings less than 256 bins do; with this
+// the errors of their rates against 64 bits are still well below the bins': root
+// mean square 0.7e-7 to 1.4e-7 over spectra and columns within the limits, 2.7e-7
+// to 4.4e-7 by bins, where the other polynomial's 3.3e-7 at y = 0 dominates.
+constexpr float kTh0 = (float)9.9999999673e-01;
+constexpr float kTh1 = (float)(1.6666670980e-01 / kL2);
+constexpr float kTh2 = (float)(8.3332447187e-03 / (kL2 * kL2));
+constexpr float kTh3 = (float)(1.9847749592e-04 / (kL2 * kL2 * kL2));
+constexpr float kTh4 = (float)(2.7347502032e-06 / (kL2 * kL2 * kL2 * kL2));
+constexpr float kTh5 = (float)(2.8118837888e-08 / (kL2 * kL2 * kL2 * kL2 * kL2));
+__device__ __forceinline__ float sinhc5_l(float yl) {
+  const float u = yl * yl;
+  float p = __builtin_fmaf(u, kTh5, kTh4);
+  p = __builtin_fmaf(u, p, kTh3);
+  p = __builtin_fmaf(u, p, kTh2);
+  p = __builtin_fmaf(u, p, kTh1);
+  return __builtin_fmaf(u, p, kTh0);
+}
 
 // Bins [k0, k1) of a ray whose in-cell optical depth is at most kThinMax in
 // every bin: exp(-tau) (1 - exp(-dtau)) / dtau = exp(-(tau + y)) sinh(y)/y with
@@ -384,7 +403,7 @@ __device__ __forceinline__ void rate_nodes(const RateTables& rt, int o, const fl
       float z = yl;
 #pragma unroll
       for (int s = 0; s < NS; s++) z = __builtin_fmaf(nl[s], ds[s][i], z);
-      float f = __builtin_amdgcn_exp2f(z) * sinhc_l(yl);
+      float f = __builtin_amdgcn_exp2f(z) * sinhc5_l(yl);
       if constexpr (MIXED) {
         float zt = 0.0f;
 #pragma unroll

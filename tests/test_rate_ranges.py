@@ -255,3 +255,33 @@ def rates_of(step, src, row, idx, tau):
     finally:
         L.deallocate_pinned_light_ray_IO(io)
     return step.rates()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("temp", [3e4, 1e5, 4e5])
+@pytest.mark.parametrize("cell", [0.005, 0.3])
+def test_node_sums_round_like_fp32(require_gpu, temp, cell):
+    """Rays within all limits: the error's root mean square is that of FP32
+    rounding (some six roundings of at most 6e-8 on depths of up to 4 where the
+    sums come from), with no offset of the forms."""
+    w = small_workload(n=16, nsrc=2, seed=81)
+    n = w.n ** 3
+    rng = np.random.default_rng(82)
+    w.dens = (cell * (0.1 + rng.random(w.dens.shape))).astype(np.float32)
+    step, P = R.PointSourceStep(w), oracle_problem(w)
+    nu, sig, _ = arrays(step.run)
+    spec = blackbody(nu, temp).astype(np.float32)
+    _, lims = limits(None, step.run, spec[None])
+    far = columns(rng, sig, n, 0.9 * lims[0, :3].min())
+    idx = np.stack(np.unravel_index(np.arange(n), w.dens.shape), 1)
+    src = rng.uniform(-0.1, 1.1, (n, 3)).astype(np.float32)
+    tau = (far / (w.lunit * w.denstonh)).astype(np.float32)
+    row = 1.0e58 * spec.astype(np.float64)
+    print(f"rounding of node sums: {temp:.0e} K, cells {cell}", flush=True)
+    got = rates_of(step, src, row, idx, tau)
+    want = np.array([P.ray_rate(src[i], row, *(int(v) for v in idx[i]), tau[i], mode=1)
+                     for i in range(n)])
+    fin = np.isfinite(want) & (want > 1e-30) & (want < 1e37)
+    assert fin.all(1).mean() > 0.4
+    err = (got[fin] - want[fin]) / want[fin]
+    assert np.sqrt(np.mean(err ** 2)) < 2e-7, np.sqrt(np.mean(err ** 2))
