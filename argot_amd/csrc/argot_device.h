@@ -787,13 +787,6 @@ __device__ inline void ray_rate_setup(const GridDev& g, const Chord& c, const fl
   rr->v[2] = nHeII * vsh + kRateTiny;
 }
 
-// 1/v to about an ulp of double: the estimate and two Newton steps.
-__device__ __forceinline__ double rcp_f64(double v) {
-  double y = __builtin_amdgcn_rcp(v);
-  y = __builtin_fma(__builtin_fma(-v, y, 1.0), y, y);
-  return __builtin_fma(__builtin_fma(-v, y, 1.0), y, y);
-}
-
 __device__ __forceinline__ double lane_value(double v, int lane) { return __shfl(v, lane, 64); }
 
 // The reference's frequency loop in FP64, calc_photoion_rate.c:285-387,

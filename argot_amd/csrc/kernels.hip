@@ -516,24 +516,23 @@ __device__ inline void rate_loop_f32(const RateTables& rt, const RayRate& rr, do
   // per-ray prefactors first (same operations as after the loop), so that
   // only they, not the ray's FP64 quantities, stay live through the bins
   const double pre = scale * exp_scaled(-tsh, 0);
-  const double p0 = rcp_f64(rr.v[0]) * rr.d[0] * pre;
-  const double p1 = rcp_f64(rr.v[1]) * rr.d[1] * pre;
-  const double p2 = rcp_f64(rr.v[2]) * rr.d[2] * pre;
+  const double p0 = 1.0 / rr.v[0] * rr.d[0] * pre;
+  const double p1 = 1.0 / rr.v[1] * rr.d[1] * pre;
+  const double p2 = 1.0 / rr.v[2] * rr.d[2] * pre;
   double G[3] = {0, 0, 0}, H[3] = {0, 0, 0};
   // largest in-cell optical depth of this ray over the bins.  A wavefront
   // whose rays are all thin runs the thin loop; one with a thicker ray runs
   // the combined loop, in which a thin lane does the thin loop's operations
   // exactly, so a cell's rates do not depend on which rays share its
   // wavefront (tile shape, grid size).
-  const float dmax = (float)rr.d[0] * (float)rt.cs_max[0] + (float)rr.d[1] * (float)rt.cs_max[1] +
-                     (float)rr.d[2] * (float)rt.cs_max[2];
+  const double dmax = rr.d[0] * rt.cs_max[0] + rr.d[1] * rt.cs_max[1] + rr.d[2] * rt.cs_max[2];
   constexpr double kHalfLog2e = 0.5 * 1.4426950408889634;
   constexpr double kLog2eD = 1.4426950408889634;
   const float dl[3] = {(float)(rr.d[0] * -kHalfLog2e), (float)(rr.d[1] * -kHalfLog2e),
                        (float)(rr.d[2] * -kHalfLog2e)};
   const float nl[3] = {(float)(rr.t[0] * -kLog2eD), (float)(rr.t[1] * -kLog2eD),
                        (float)(rr.t[2] * -kLog2eD)};
-  const bool thin = dmax <= (float)kThinMax;
+  const bool thin = dmax <= kThinMax;
   const bool all_thin = __all(thin);
   // (the sums are in units of exp(-tsh), the nodes' weights in those of kRuleScale)
   const double unit1 = exp_scaled(tsh - rr.t[0] * rt.end[0], -kRuleExponent);
@@ -661,19 +660,15 @@ __global__ __launch_bounds__(kProjectThreads) void project_spectra_kernel(
 
 // Lower bound of the shifted bin optical depth and upper bound of the
 // in-cell optical depth decide whether the FP32 loop is safe.
-// (In FP32: the bounds are far from where the loop would fail, and a column
-// beyond FP32's range is infinite here and fails.)
 __device__ __forceinline__ bool fast_rate_ok(const RateTables& rt, const RayRate& rr) {
-  float lo = 0.0f, dmax = 0.0f;
+  double lo = 0.0, dmax = 0.0;
   bool finite = true;
   for (int s = 0; s < 3; s++) {
-    const float t = (float)rr.t[s], d = (float)rr.d[s];
-    const float last = (float)rt.cs_last[s], top = (float)rt.cs_max[s];
-    lo += t >= 0.0f ? -t * last : t * (top - last);
-    dmax += d * top;
-    finite = finite && fabsf(t) < 1.0e36f && d < 1.0e36f;
+    lo += rr.t[s] >= 0.0 ? -rr.t[s] * rt.cs_last[s] : rr.t[s] * (rt.cs_max[s] - rt.cs_last[s]);
+    dmax += rr.d[s] * rt.cs_max[s];
+    finite = finite && fabs(rr.t[s]) < 1.0e36 && rr.d[s] < 1.0e36;
   }
-  return finite && lo > -60.0f && dmax < 1.0e30f;
+  return finite && lo > -60.0 && dmax < 1.0e30;
 }
 
 __device__ __forceinline__ int wave_min(int v) {
