@@ -921,21 +921,27 @@ void sweep_order(std::vector<ArtDir>& dirs, int batch) {
   }
 }
 
-// Whether they hold for the box: cell indices in 32 bits, faces where the
-// cells end, and rays whose rounding (at most 3 crossings a layer, each within
-// an ulp of the largest coordinate) stays below 0.2 cells.
+// Whether they hold for the box: cell indices in 32 bits, and rays that stay
+// within 0.2 cells of where the tiles expect them.  What moves a ray: rounding (at
+// most 3 crossings a layer, each within an ulp of the largest coordinate), and the
+// part by which an axis' extent differs from its cells, once at the entry and once
+// at each of up to nD/n + 1 wraps through its side faces, which put the ray back
+// on the box's face.
 bool sweep_applies(const ArtGrid& g) {
   const double mn[3] = {g.xmin, g.ymin, g.zmin}, mx[3] = {g.xmax, g.ymax, g.zmax};
   const double d[3] = {g.dx, g.dy, g.dz};
   const int n[3] = {g.nx, g.ny, g.nz};
-  double big = 0.0;
+  const int longest = std::max(g.nx, std::max(g.ny, g.nz));
+  double big = 0.0, off = 0.0;
   for (int k = 0; k < 3; k++) {
-    if (!(d[k] > 1e-12 && d[k] < 1e6) || !(fabs(mx[k] - mn[k] - n[k] * d[k]) < 0.05 * d[k])) return false;
+    if (!(d[k] > 1e-12 && d[k] < 1e6)) return false;
+    off = std::max(off, fabs(mx[k] - mn[k] - n[k] * d[k]) / d[k] * (2.0 + (double)longest / n[k]));
     big = std::max(big, std::max(fabs(mn[k]), fabs(mx[k])));
   }
-  const double err = 3.0 * std::max(g.nx, std::max(g.ny, g.nz)) * big * 1.2e-7 / d[0];
+  const double err = off + 3.0 * longest * big * 1.2e-7 / d[0];
   const int64_t rows = std::max((int64_t)g.nx * g.ny, (int64_t)g.nx * g.nz);   // 24-bit products
-  return err < 0.2 && g.ncell <= ((int64_t)1 << 30) && std::max(rows, (int64_t)g.ny * g.nz) < (1 << 24);
+  return err < 0.2 && g.ncell <= ((int64_t)1 << 30) &&
+         std::max(rows, (int64_t)g.ny * g.nz) < (1 << 24);
 }
 
 double now_ms() {
