@@ -180,6 +180,7 @@ struct Ctx {
   // quadrature rule of the tables (one buffer), and the weights and limits
   // of the spectra in use (one buffer)
   DevBuf<double> rule_buf;
+  std::shared_ptr<const RateRule> rule_kept;   // the one in rule_buf
   DevBuf<float> weight;
   RuleDev rule{};
   const float *qsig = nullptr, *qdsig = nullptr;
@@ -220,6 +221,7 @@ struct Ctx {
     hsig.release();
     dsig.release();
     rule_buf.release();
+    rule_kept.reset();
     weight.release();
     tree_buf.release();
     tree_stage.release();
@@ -419,11 +421,12 @@ void upload_tables(Ctx& g, const run_param* r) {
   HIP_OK(hipMemcpy(g.dsig.p, t.dsig.data(), 3 * ng * sizeof(float), hipMemcpyHostToDevice));
   const std::shared_ptr<const RateRule> kept = rate_rule(t);
   const RateRule& rule = *kept;
-  g.rule = RuleDev{};
-  g.rule.usable = rule.usable ? 1 : 0;
-  for (int k = 0; k < 4; k++) g.rule.start[k] = rule.usable ? rule.start[k] : 0;
-  memcpy(g.edge, rule.edge, sizeof g.edge);
-  memcpy(g.end, rule.end, sizeof g.end);
+  // (A program may send its run parameters every step, mostly with the tables
+  // unchanged.  A rule is never written again and the context holds on to its
+  // own, so the same object has the same contents.)
+  if (g.rule_kept == kept) return;
+  g.rule_kept.reset();
+  g.rule = RuleDev{};   // (none, and every ray by bins, should the upload fail)
   // lag (double), then sig, dsig, rate and test (float; even numbers of them)
   const size_t nl = rule.lag.size(), ns = rule.sig.size(), nr = rule.rate.size();
   std::vector<double> buf(nl + (2 * ns + nr + rule.test.size()) / 2);
@@ -435,11 +438,16 @@ void upload_tables(Ctx& g, const run_param* r) {
   std::copy(rule.test.begin(), rule.test.end(), f + 2 * ns + nr);
   HIP_OK(g.rule_buf.reserve(buf.size()));
   HIP_OK(hipMemcpy(g.rule_buf.p, buf.data(), buf.size() * sizeof(double), hipMemcpyHostToDevice));
+  g.rule.usable = rule.usable ? 1 : 0;
+  for (int k = 0; k < 4; k++) g.rule.start[k] = rule.usable ? rule.start[k] : 0;
+  memcpy(g.edge, rule.edge, sizeof g.edge);
+  memcpy(g.end, rule.end, sizeof g.end);
   g.rule.lag = g.rule_buf.p;
   g.qsig = reinterpret_cast<const float*>(g.rule_buf.p + nl);
   g.qdsig = g.qsig + ns;
   g.rule.rate = g.qdsig + ns;
   g.rule.test = g.rule.rate + nr;
+  g.rule_kept = kept;
 }
 
 // The caller's context, ready and for a mesh of this_run's size, or null
