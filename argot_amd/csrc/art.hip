@@ -842,6 +842,7 @@ ArtCtx a_;
   do {                                                                              \
     hipError_t _e = (expr);                                                         \
     if (_e != hipSuccess) {                                                         \
+      (void)hipGetLastError(); /* else the next launch reports it */                \
       argot_hip_internal_set_error(_e == hipErrorOutOfMemory ? ARGOT_ERR_NOMEM      \
                                                              : ARGOT_ERR_HIP);      \
       return;                                                                       \
@@ -1154,11 +1155,21 @@ void init_diffuse_gpu(struct cuda_diffuse_param* cd, struct cuda_param* this_cud
   a_.batch = 0;
   A_OK(hipMalloc(&a_.d_dirs, sizeof(ArtDir) * nang));
   A_OK(hipMalloc(&a_.med, sizeof(ArtMedium) * ncell));
-  A_OK(hipMalloc(&a_.acc, sizeof(float4) * ncell * batch));
   A_OK(hipMalloc(&a_.medT, sizeof(ArtMedium) * ncell));
   A_OK(hipMalloc(&a_.gh, sizeof(float) * 6 * ncell));
   A_OK(hipMalloc(&a_.comp, sizeof(float) * 6 * ncell));
   A_OK(hipMalloc(&a_.ncross, sizeof(unsigned long long)));
+  // The slices last: where the default batch does not fit what is left, a
+  // smaller one does (the rates are the same).
+  hipError_t e = hipMalloc(&a_.acc, sizeof(float4) * ncell * batch);
+  while (e == hipErrorOutOfMemory && g_batch <= 0 && batch > 1) {
+    (void)hipGetLastError();
+    a_.acc = nullptr;
+    batch = (batch + 1) / 2;
+    e = hipMalloc(&a_.acc, sizeof(float4) * ncell * batch);
+  }
+  if (e != hipSuccess) a_.acc = nullptr;
+  A_OK(e);
   a_.ncell = ncell;
   a_.batch = batch;
   a_.nside = g_nside;
