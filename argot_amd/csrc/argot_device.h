@@ -526,13 +526,13 @@ struct PackedFields {
 // with Kahan sums 31.5 instead of 35.2, on 72 x 58 x 87 and 250 4.9 instead of 5.7.
 // A walk normally ends in its end cell; one that misses
 // it (rounding has carried it past, or a face difference below 2^-126 was no
-// clean 0 or 1) runs on over range-checked loads to the cap of nx + ny + nz
-// crossings, more than any walk inside the mesh has, or meets the end cell's
-// index outside the mesh; both are seen afterwards, false is returned and
-// the caller walks the segment again in the other form.
+// clean 0 or 1) runs on over range-checked loads to the caller's cap, passes of
+// two crossings each, or meets the end cell's index outside the mesh; both are
+// seen afterwards, false is returned and the caller walks the segment again in the
+// other form.  passes: the same for the wavefront.
 template <bool KAHAN, bool HASH, bool POW2, typename Fields>
 __device__ inline bool walk_float(const GridDev& g, const Fields& fields, const RayDir& dir,
-                                  Vec3f s, Vec3f e, WalkOut* out) {
+                                  Vec3f s, Vec3f e, int passes, WalkOut* out) {
   DdaF d = dda_float<POW2>(g, dir, s, e);
   float t0 = 0.0f, t1 = 0.0f, t2 = 0.0f;
   float c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
@@ -565,7 +565,6 @@ __device__ inline bool walk_float(const GridDev& g, const Fields& fields, const 
     actB = active();
   }
   float4 nB = load();
-  int passes = (g.nx + g.ny + g.nz) / 2 + 1;   // wave-uniform
   while (actA && passes > 0) {
     passes--;
     nc++;
@@ -698,15 +697,23 @@ __device__ inline void walk_segment_with(const GridDev& g, const Fields& fields,
   out->hash = h;
 }
 
+// Passes of walk_float that no walk inside the mesh exceeds.
+__device__ __forceinline__ int box_passes(const GridDev& g) {
+  const int n = (g.nx + g.ny + g.nz) / 2 + 1;
+  __builtin_assume(n > 0);
+  return n;
+}
+
 // The walk over the packed per-cell densities nf (float4 per cell) from s to
-// e, along dir (ray_dir of e - s).
+// e, along dir (ray_dir of e - s).  passes: cap of the float form (0: not by it).
 template <bool KAHAN, bool HASH, bool NARROW, bool POW2, bool FLOAT>
 __device__ __forceinline__ void walk_segment(const GridDev& g, const float4* __restrict__ nf,
-                                             const RayDir& dir, Vec3f s, Vec3f e, WalkOut* out) {
+                                             const RayDir& dir, Vec3f s, Vec3f e, int passes,
+                                             WalkOut* out) {
   const uint32_t nbytes = NARROW ? (uint32_t)((int64_t)g.nx * g.nyz * 16) : 0u;
   const PackedFields<NARROW> fields{nf, nbytes};
   if constexpr (FLOAT) {
-    if (walk_float<KAHAN, HASH, POW2>(g, fields, dir, s, e, out)) return;
+    if (passes > 0 && walk_float<KAHAN, HASH, POW2>(g, fields, dir, s, e, passes, out)) return;
   }
   walk_segment_with<KAHAN, HASH, POW2>(g, fields, s, e, out);
 }
