@@ -513,6 +513,14 @@ struct PackedFields {
   }
 };
 
+// The float form's byte offset as an integer: 0 below 0, 2^32 - 1 beyond it (a
+// walk that has left the box), as the instruction has it and C++ does not.
+__device__ __forceinline__ uint32_t byte_offset(float idx) {
+  uint32_t u;
+  asm("v_cvt_u32_f32 %0, %1" : "=v"(u) : "v"(idx));
+  return u;
+}
+
 // The walk in its float form: the same operations on the same values as the
 // walk below (every optical depth and position has its bits), arranged for
 // gfx950's issue rates, where FP32 products and sums take 2 cycles per
@@ -539,9 +547,9 @@ __device__ inline bool walk_float(const GridDev& g, const Fields& fields, const 
   int nc = 0;
   uint64_t h = 0xcbf29ce484222325ull;
   auto active = [&]() { return d.idx != d.idxe; };
-  auto load = [&]() { return fields((uint32_t)d.idx); };
+  auto load = [&]() { return fields(byte_offset(d.idx)); };
   auto mark = [&]() {
-    if (HASH) h = (h ^ (uint64_t)((uint32_t)d.idx >> 4)) * 0x100000001b3ull;
+    if (HASH) h = (h ^ (uint64_t)(byte_offset(d.idx) >> 4)) * 0x100000001b3ull;
   };
   auto add = [&](float r, const float4& n) {
     if (KAHAN) {
