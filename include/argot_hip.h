@@ -666,8 +666,8 @@ void argot_hip_surrogate_set_baseline(const float *coef, int npoly);
 void argot_hip_set_theta(float theta);
 
 /* Persistent grid of the fused kernel, in wavefronts per compute unit
- * (default 24: six per SIMD, the exact-rate kernels' register budget;
- * n <= 0 restores the default). */
+ * (default 16: four per SIMD, the rate kernels' register budget; n <= 0
+ * restores the default). */
 void argot_hip_set_blocks_per_cu(int n);
 
 /* Target tile of one wavefront in the fused kernel: tx*ty*tz = 64 cells,
@@ -697,6 +697,20 @@ struct argot_tune_report {
 void argot_hip_autotune_step(struct fluid_mesh *mesh, struct radiation_src *src,
                              struct run_param *this_run, struct cuda_mem_space *cuda_mem,
                              struct cuda_param *this_cuda, struct argot_tune_report *rep);
+
+/* The kernels' arithmetic on the host, for tests.  quotients: the walk's
+ * q[i] = a[i]/b[i].  rate_rule: the frequency quadrature of run_param's tables,
+ * cross-sections sigma_s and sigma_s - sigma_s(last bin) at its 44 nodes (3 x 44
+ * each), and for nspec spectra of 256 floats their weights (192 each) and limits
+ * (the smallest of the three bin ranges'); returns the number of nodes, 0 where
+ * the tables have no rule.  rate_limits: weights and limits (4 each: by range,
+ * and the first range's for rays it holds next to nothing of) formed on the host
+ * where cuda_mem is null, else by the kernel on the context's tables. */
+void argot_hip_quotients(const float *a, const float *b, float *q, int64_t n);
+int argot_hip_rate_rule(const struct run_param *this_run, const float *spec, int nspec, float *sig,
+                        float *dsig, float *weight, float *limit);
+void argot_hip_rate_limits(struct cuda_mem_space *cuda_mem, const struct run_param *this_run,
+                           const float *spec, int nspec, float *weight, float *limits);
 
 /* Measured device copy bandwidth: best of reps copies of nbytes with a
  * plain streaming kernel, in GB/s of bytes read plus written. */
