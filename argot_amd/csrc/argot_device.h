@@ -527,7 +527,7 @@ __device__ __forceinline__ uint32_t byte_offset(float idx) {
 // wavefront and comparisons, selects, conversions and FP64 take 4: exact
 // quotients by FP32 multiply-adds, the face choice as 0/1 factors, the cell
 // index in FP32, and no test at each crossing whether the cell is inside the
-// mesh.  About 86 cycles per crossing instead of 136: with the gathers (26
+// mesh.  About 90 cycles per crossing instead of 136: with the gathers (26
 // cycles of the vector memory path each) this is what bounds the fused
 // kernel.  With the set-up around it in the same arithmetic (ray_dir) the step
 // on 256^3 cells and 4096 sources took 88 ms instead of 99, on 128^3 and 1024

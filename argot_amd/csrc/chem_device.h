@@ -7,10 +7,11 @@
 //
 // Every float/double promotion of the reference's expressions is written
 // out, and the file is compiled without contraction or fast-math, so each
-// rounding sits where the C source puts it.  The transcendental functions
-// (exp, log, log10, pow) are the device library's double routines; they may
-// differ from a host libm in the last bit, which is the only source of
-// difference from a host restatement of the same code.
+// rounding sits where the C source puts it.  Two things differ from a host
+// restatement of the same code, both far below the floats that the results are
+// rounded to: the transcendental functions are the device library's double
+// routines, which may differ from a host libm in the last bit, and the powers
+// of the fits are formed from one logarithm (below), to a few 1e-15.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <float.h>

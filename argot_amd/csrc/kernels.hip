@@ -670,9 +670,11 @@ __global__ __launch_bounds__(kProjectThreads) void project_spectra_kernel(
   __syncthreads();
   if (t < kRuleLimits * NB && u0 + t / kRuleLimits < nspec) {
     const unsigned f = rule.usable ? fail[t] : 1u;
-    const int g = t % kRuleLimits;
-    const float lim[3] = {rule_limit(0, f), rule_limit(1, f), rule_limit(2, f)};
-    limit[(int64_t)kRuleLimits * u0 + t] = g == 1 ? lim[1] : g == 2 ? lim[2] : lim[0];
+    const int i = t % kRuleLimits;
+    const float lim[kRuleLimits] = {rule_limit(0, f), rule_limit(1, f), rule_limit(2, f),
+                                    rule_limit(3, f)};
+    limit[(int64_t)kRuleLimits * u0 + t] =
+        i == 0 ? lim[0] : i == 1 ? lim[1] : i == 2 ? lim[2] : lim[3];
   }
 }
 
@@ -1009,11 +1011,10 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY void fused_step_kernel(FusedArg
       // along the axis the rays run along mostly (from the node to the tile)
       // go to neighbouring lanes.  Their rays share most of their cells, and
       // the vector memory path serves a 12-B gather four neighbouring lanes at
-      // a time, a cycle for each cache line the four touch: 26 lines for the
-      // 16 groups instead of 31 with lanes in mesh order (rays from random
-      // sources on 256^3; 13% fewer cache accesses counted on 4096 clumped
-      // ones, 1.5% of the time: issue bounds the kernel as much).  Bricks of
-      // 2 x 2 x 2 cells would touch 24, but their alternating strides cost
+      // a time, a cycle for each cache line the four touch: 24.6 lines a gather
+      // instead of 28.2 with lanes in mesh order (counted on 256^3 and 4096
+      // clumped sources; 1.5% of the time: issue bounds the kernel as much).  Bricks of
+      // 2 x 2 x 2 cells would touch a few less, but their alternating strides cost
       // registers, and what they spilled cost 30%.
       const float ax = fabsf(far.x - cx), ay = fabsf(far.y - cy), az = fabsf(far.z - cz);
       int t = lane;

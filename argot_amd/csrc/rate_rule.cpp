@@ -28,11 +28,11 @@
 // Between the test columns the error was at most 2e-7, on 36000 spectra drawn
 // with lines, steps, noise, waves, cut-offs and second temperatures.
 // A 1e5 K blackbody passes to optical depth 104 at the HI edge, 75 at the HeI
-// edge and 18 at the HeII edge, a 3e4 K one to 104, 32 and 8.
+// edge and 21 at the HeII edge, a 3e4 K one to 104, 32 and 8.
 // Measured with the bin loops as the other side: the step on 256^3 cells and 4096
-// sources 147 -> 111 ms, on 72 x 58 x 87 cells and 250 sources 13.0 -> 6.5 ms,
-// with the same error against 64-bit rates (2.6e-7 and 8.4e-6 of the mesh's
-// rates); 10, 12 and 16 nodes serve only half as thick rays at that error, and
+// sources 147 -> 111 ms, on 72 x 58 x 87 cells and 250 sources 13.0 -> 6.5 ms;
+// errors against 64-bit rates 0.7e-7 to 1e-7 by nodes and 2.3e-7 by bins (64^3,
+// uniform); 10, 12 and 16 nodes serve only half as thick rays at that error, and
 // nodes of the continuous Legendre polynomials a fifth.
 #include "rate_rule.h"
 
@@ -260,7 +260,7 @@ void project_spectra_host(const RateRule& r, const float* spec, int nspec, int n
         if (!(fabsf(err) <= kRuleLoose * sum)) loose |= level;
       }
       limit[(size_t)u * kRuleLimits + g] = rule_limit(g, fail);
-      if (g == 0) limit[(size_t)u * kRuleLimits + 3] = rule_limit(0, loose);
+      if (g == 0) limit[(size_t)u * kRuleLimits + 3] = rule_limit(3, loose);
       m += (size_t)n * ncol * 2;
     }
   }

@@ -36,8 +36,11 @@ constexpr float kRuleTol = 1.0e-7f;     // relative error allowed on every test 
 // holds at most kRuleShare.
 constexpr float kRuleLoose = 1.0e-2f;
 constexpr double kRuleShare = 2.0e-6;
-// Limits of a spectrum: by range at kRuleTol, and the first range's at kRuleLoose.
+// Limits of a spectrum: by range at kRuleTol, and the first range's at kRuleLoose,
+// for which its last three scales are (too far apart for the other).
 constexpr int kRuleLimits = 4;
+constexpr int kRuleTopLevel[kRuleLimits] = {kRuleLevels[0] - 3, kRuleLevels[1], kRuleLevels[2],
+                                            kRuleLevels[0]};
 // Optical depths at the lower edges of the three ranges that scale 1 means.
 constexpr double kRuleEdge[3] = {80.0, 25.0, 8.0};
 // The weights carry the cross-sections times this power of two.
@@ -63,15 +66,15 @@ struct RateRule {
 // third range.
 void build_rate_rule(const float* sig, const float* hsig, int ngrid, int k1, int k2, RateRule* r);
 
-// Limit of a range: the largest scale up to which no test of it has failed
+// The i-th limit of a spectrum: the largest scale up to which no test has failed
 // (bit 0 of fail: the reversed columns, bit l: level l - 1), 0 for none.
 #ifdef __HIPCC__
 __host__ __device__
 #endif
-inline float rule_limit(int g, unsigned fail) {
+inline float rule_limit(int i, unsigned fail) {
   float lim = 0.0f;
-  for (int l = 0; l < kRuleLevels[g] && (fail & ((4u << l) - 1u)) == 0u; l++)
-    lim = kRuleLevel[g][l];
+  for (int l = 0; l < kRuleTopLevel[i] && (fail & ((4u << l) - 1u)) == 0u; l++)
+    lim = kRuleLevel[i % 3][l];
   return lim;
 }
 

@@ -126,6 +126,9 @@ def test_each_range_holds_to_its_own_limit():
     w2, lims = limits(None, run, rows)
     assert np.array_equal(w, w2) and np.array_equal(lim, lims[:, :3].min(1))
     assert (lims[:, 3] >= lims[:, 0]).all()
+    # (scales beyond 1.3 are too far apart for the first range's own limit: 3e-7
+    # between 1.3 and 1.7 on a spectrum with 1e-7 at both)
+    assert (lims[:, 0] <= np.float32(1.3)).all() and (lims[:, 0] == np.float32(1.3)).any()
     # a line below the HeI edge leaves the other ranges their limits
     _, smooth = limits(None, run, (blackbody(nu, 1e5) / blackbody(nu, 1e5)[44:].max())[None])
     assert np.array_equal(lims[list(sp).index("1e5 K, one bin up"), 1:3], smooth[0, 1:3])
