@@ -795,8 +795,7 @@ __device__ inline void ray_rate_setup(const GridDev& g, const Chord& c, const fl
   rr->t[2] -= 0.5 * rr->d[2];
   const double a = (double)dist + 0.5 * (double)delta;
   const double b = (double)dist - 0.5 * (double)delta;
-  const double lu = g.lunit;
-  const double vsh = 4.0 * kPi / 3.0 * (a * a * a - b * b * b) * (lu * lu * lu);
+  const double vsh = 4.0 * kPi / 3.0 * (a * a * a - b * b * b) * g.lunit3;
   rr->v[0] = nHI * vsh + kRateTiny;
   rr->v[1] = nHeI * vsh + kRateTiny;
   rr->v[2] = nHeII * vsh + kRateTiny;

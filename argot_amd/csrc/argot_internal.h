@@ -31,6 +31,7 @@ struct GridDev {
   double lunit, denstonh, helium_fact;
   float theta_sq;   // SQR(theta_crit) in FP32 (setup_light_ray_tree.c:577)
   float rdx, rdy, rdz;   // RN(1/dx) etc.
+  double lunit3;   // lunit^3
 };
 
 // Frequency tables (device pointers).  sig/hsig are [3][ngrid] SoA:
@@ -47,6 +48,7 @@ struct RateTables {
   const float* dsig;   // [3*ngrid] sigma_s(k) - sigma_s(last bin), species-major
   double cs_max[3];    // max over bins of sigma_s
   double cs_last[3];   // sigma_s at the last bin
+  double cs_span[3];   // cs_max - cs_last
   // quadrature form (rate_rule.h): cross-sections at its nodes, and the
   // first-bin cross-sections that scale a ray against a spectrum's limit
   const float* qsig;   // [3*kRuleNodes] sigma_s, species-major

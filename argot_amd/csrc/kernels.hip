@@ -684,7 +684,7 @@ __device__ __forceinline__ bool fast_rate_ok(const RateTables& rt, const RayRate
   double lo = 0.0, dmax = 0.0;
   bool finite = true;
   for (int s = 0; s < 3; s++) {
-    lo += rr.t[s] >= 0.0 ? -rr.t[s] * rt.cs_last[s] : rr.t[s] * (rt.cs_max[s] - rt.cs_last[s]);
+    lo += rr.t[s] >= 0.0 ? -rr.t[s] * rt.cs_last[s] : rr.t[s] * rt.cs_span[s];
     dmax += rr.d[s] * rt.cs_max[s];
     finite = finite && fabs(rr.t[s]) < 1.0e36 && rr.d[s] < 1.0e36;
   }
@@ -914,10 +914,21 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY void fused_step_kernel(FusedArg
   const bool morton = mbits <= 10 && ncube <= 8 * ntile;
   const int64_t nqueue_tiles = morton ? ncube : ntile;
   int q = blockIdx.x % kNumQueues, tried = 0;
-  // per-lane counts (a lane's rays and crossings over the launch fit in 32
-  // bits); wave-uniform visit counts
-  unsigned int my_ray = 0, my_cross = 0, my_fb = 0, my_surr = 0;
-  unsigned long long my_visit = 0, my_emit_iter = 0;
+  // Each lane's counts: rays, crossings, FP64 fallbacks and, the same in every
+  // lane, visits and visits with a ray (over a launch they fit in 32 bits).  They
+  // are in LDS, where adding to them takes no register: as variables they were
+  // spilled, and read and written back at every visit through the texture path,
+  // which bounds the kernel (16 cycles of it an 8-B access; with 64-bit visits 3%
+  // of the launch).  (The surrogate variant has no room for the visits' in LDS.)
+  constexpr int kCounts = SURR ? 3 : 5;
+  __shared__ unsigned int count_lds[kCounts][64];
+  unsigned int my_surr = 0, my_visit = 0, my_emit_iter = 0;
+  const auto count = [&](int i, unsigned int by) {
+    (void)__hip_atomic_fetch_add(&count_lds[i][lane], by, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_WAVEFRONT);
+  };
+#pragma unroll
+  for (int i = 0; i < kCounts; i++) count_lds[i][lane] = 0u;
   // The targets' per-cell FP64 sums, centres, and densities and fractions live
   // in LDS between rays, by the target's place in the tile: the walk and the
   // frequency loop have the registers to themselves, and a ray can be worked
@@ -1003,10 +1014,16 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY void fused_step_kernel(FusedArg
       const bool leaf = ln.n <= 1;
       const bool emit = here && (accept || ln.n == 1);
       if (here) p = (accept || leaf || ln.first < 0) ? ln.skip : ln.first;
-      my_visit++;
+      if constexpr (SURR)
+        my_visit++;
+      else
+        count(3, 1u);
       const unsigned long long emitting = __ballot(emit);
       if (emitting == 0) continue;
-      my_emit_iter++;
+      if constexpr (SURR)
+        my_emit_iter++;
+      else
+        count(4, 1u);
       // Which target's ray each lane works: targets that follow one another
       // along the axis the rays run along mostly (from the node to the tile)
       // go to neighbouring lanes.  Their rays share most of their cells, and
@@ -1087,7 +1104,7 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY void fused_step_kernel(FusedArg
       // sums; this loop serves the rays FP32 cannot).  It comes first, so that
       // the ray's FP64 quantities need not outlive the FP32 loop.
       rate_f64_wave(rt, rr, wide, [&](int, int k) { return (double)sp[k] * sc; }, res);
-      if (wide) my_fb++;
+      if (wide) count(2, 1u);
       if (exact && !wide) {
         const F4* wt = reinterpret_cast<const F4*>(tr.weight + (int64_t)u * kRuleWeights);
         rate_loop_f32(rt, rr, sc, [&](int k) { return ldc(tr.limit + kRuleLimits * u + k); },
@@ -1098,8 +1115,8 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY void fused_step_kernel(FusedArg
       if (work) {
 #pragma unroll
         for (int k = 0; k < 6; k++) acc_lds[k][t] += res[k];
-        my_ray++;
-        my_cross += (unsigned int)w.ncross;
+        count(0, 1u);
+        count(1, (unsigned int)w.ncross);
         if (CAPTURE) {
           const unsigned long long slot = atomicAdd(&a.ctr->nrecord, 1ull);
           if (slot < (unsigned long long)a.rec_cap) {
@@ -1127,9 +1144,13 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY void fused_step_kernel(FusedArg
       for (int k = 0; k < 6; k++) r[k] = (float)((double)r[k] + acc_lds[k][lane]);
     }
   }
-  const unsigned long long sr = wave_sum((unsigned long long)my_ray),
-                           sc = wave_sum((unsigned long long)my_cross),
-                           sf = wave_sum((unsigned long long)my_fb),
+  if constexpr (!SURR) {
+    my_visit = count_lds[3][lane];
+    my_emit_iter = count_lds[4][lane];
+  }
+  const unsigned long long sr = wave_sum((unsigned long long)count_lds[0][lane]),
+                           sc = wave_sum((unsigned long long)count_lds[1][lane]),
+                           sf = wave_sum((unsigned long long)count_lds[2][lane]),
                            ss = wave_sum((unsigned long long)my_surr);
   if (lane == 0 && my_visit) {
     StepCounters::Queue& c = a.ctr->queue[blockIdx.x % kNumQueues];
@@ -1137,8 +1158,8 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY void fused_step_kernel(FusedArg
     atomicAdd(&c.ncross, sc);
     if (sf) atomicAdd(&c.nfallback, sf);
     if (SURR && ss) atomicAdd(&c.nsurrogate, ss);
-    atomicAdd(&c.nvisit, my_visit);
-    atomicAdd(&c.nemit_iter, my_emit_iter);
+    atomicAdd(&c.nvisit, (unsigned long long)my_visit);
+    atomicAdd(&c.nemit_iter, (unsigned long long)my_emit_iter);
   }
 }
 

@@ -310,6 +310,7 @@ GridDev make_grid(const run_param* r) {
   d.rdz = 1.0f / d.dz;
   d.lunit = r->lunit;
   d.denstonh = r->denstonh;
+  d.lunit3 = d.lunit * d.lunit * d.lunit;
   d.helium_fact = g_helium_fact;
   const float th = r->theta_crit;
   d.theta_sq = th * th;
@@ -329,6 +330,7 @@ RateTables rate_tables(const Ctx& g) {
   for (int s = 0; s < 3; s++) {
     t.cs_max[s] = g.cs_max[s];
     t.cs_last[s] = g.cs_last[s];
+    t.cs_span[s] = g.cs_max[s] - g.cs_last[s];
   }
   t.qsig = g.qsig;
   t.qdsig = g.qdsig;
