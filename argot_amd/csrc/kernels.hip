@@ -157,6 +157,10 @@ __device__ inline int segment_passes(const GridDev& g, Vec3f s, Vec3f e) {
 // The walk over packed densities (see walk_segment).
 template <bool NARROW, bool POW2, bool FLOAT>
 struct WalkPacked {
+  // Wavefronts per SIMD.  The float form is bound by the gathers' cache lines:
+  // more wavefronts push one another's out (8 Mi segments on 256^3: 4, 5 and 8
+  // take 2.68, 2.85 and 3.0 ms).
+  static constexpr int kWaves = FLOAT ? 4 : 8;
   const float4* nf;
   __device__ __forceinline__ void operator()(const GridDev& g, Vec3f s, Vec3f e, bool kahan,
                                              WalkOut* w) const {
@@ -172,6 +176,7 @@ struct WalkPacked {
 // The walk over the mesh records.
 template <bool POW2>
 struct WalkMesh {
+  static constexpr int kWaves = 8;
   MeshFields f;
   __device__ __forceinline__ void operator()(const GridDev& g, Vec3f s, Vec3f e, bool kahan,
                                              WalkOut* w) const {
@@ -183,7 +188,8 @@ struct WalkMesh {
 };
 
 template <typename Walk>
-__global__ __launch_bounds__(kWalkBlock) void walk_segments_kernel(
+__global__ __launch_bounds__(kWalkBlock)
+    __attribute__((amdgpu_waves_per_eu(Walk::kWaves, Walk::kWaves))) void walk_segments_kernel(
     GridDev g, Walk walk, unsigned char* __restrict__ seg, int64_t nseg, int kahan) {
   __shared__ unsigned bucket_lds[64];
   __shared__ unsigned perm_lds[kWalkBlock];
