@@ -502,11 +502,11 @@ __device__ __forceinline__ void rate_range(const RateTables& rt, bool nodes, boo
 // the HeI and HeII edges skip the absent species.
 // In a range within whose limit of its spectrum it lies a ray takes the sums as
 // quadratures over the range's nodes (rate_rule.cpp), in any other bin by bin;
-// which one depends on the ray alone, not on its wavefront.  limit(i): the
-// spectrum's limits (kRuleLimits).
-template <typename LimitF, typename SpecF, typename WeightF>
+// which one depends on the ray alone, not on its wavefront.  limit: the
+// spectrum's (kRuleLimits).
+template <typename SpecF, typename WeightF>
 __device__ inline void rate_loop_f32(const RateTables& rt, const RayRate& rr, double scale,
-                                     LimitF limit, SpecF spec, WeightF weight, double out[6]) {
+                                     F4 limit, SpecF spec, WeightF weight, double out[6]) {
   const double sh2 = rr.t[2] * rt.cs_last[2];
   const double sh1 = __builtin_fma(rr.t[1], rt.cs_last[1], sh2);
   const double tsh = __builtin_fma(rr.t[0], rt.cs_last[0], sh1);
@@ -532,9 +532,9 @@ __device__ inline void rate_loop_f32(const RateTables& rt, const RayRate& rr, do
         e = __builtin_fmaf(fabsf(tf[s]), rt.edge[3 * g + s], e);
         m = __builtin_fmaf(tn[s], rt.edge[3 * g + s], m);
       }
-      const float top = limit(g);
+      const float top = limit[g];
       nodes[g] = e <= top && m <= kRuleNegative && top > 0.0f;
-      if (g == 0) loose = !nodes[0] && e <= limit(3) && m <= kRuleNegative && limit(3) > 0.0f;
+      if (g == 0) loose = !nodes[0] && e <= limit[3] && m <= kRuleNegative && limit[3] > 0.0f;
     }
   }
   // per-ray prefactors first (same operations as after the loop), so that
@@ -785,8 +785,8 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY void target_rates_kernel(
     if (more && !wide) {
       const float* s32 = sp.spec32 + (int64_t)u * ng;
       const F4* w = reinterpret_cast<const F4*>(sp.weight + (int64_t)u * kRuleWeights);
-      rate_loop_f32(rt, rr, sp.scale[u], [&](int k) { return sp.limit[kRuleLimits * (int64_t)u + k]; },
-                    [&](int k) { return s32[k]; },
+      const F4 limit = reinterpret_cast<const F4*>(sp.limit)[u];
+      rate_loop_f32(rt, rr, sp.scale[u], limit, [&](int k) { return s32[k]; },
                     [&](int i) { return w[i]; }, res);
     }
     if (more) {
@@ -1113,7 +1113,7 @@ __global__ __launch_bounds__(64) ARGOT_OCCUPANCY void fused_step_kernel(FusedArg
       if (wide) count(2, 1u);
       if (exact && !wide) {
         const F4* wt = reinterpret_cast<const F4*>(tr.weight + (int64_t)u * kRuleWeights);
-        rate_loop_f32(rt, rr, sc, [&](int k) { return ldc(tr.limit + kRuleLimits * u + k); },
+        rate_loop_f32(rt, rr, sc, ldc(reinterpret_cast<const F4*>(tr.limit) + u),
                       [&](int k) { return ldc(sp + k); },
                       [&](int i) { return ldc(wt + i); }, res);
       }

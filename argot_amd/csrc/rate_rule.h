@@ -38,7 +38,7 @@ constexpr float kRuleLoose = 1.0e-2f;
 constexpr double kRuleShare = 2.0e-6;
 // Limits of a spectrum: by range at kRuleTol, and the first range's at kRuleLoose,
 // for which its last three scales are (too far apart for the other).
-constexpr int kRuleLimits = 4;
+constexpr int kRuleLimits = 4;   // (16 B: read at once)
 constexpr int kRuleTopLevel[kRuleLimits] = {kRuleLevels[0] - 3, kRuleLevels[1], kRuleLevels[2],
                                             kRuleLevels[0]};
 // Optical depths at the lower edges of the three ranges that scale 1 means.
